@@ -24,12 +24,12 @@ void flowhip_step_fused(FlowHipCtx* h, const FlowHipStep* st) {
   /* under the serial CFL rule the Lagrangian kernel stores its candidates
    * and fk_timestep_serial folds them in omp3's order */
   const FkReduce lr = flowhip_lagrangian_red(h, m.nx, m.ny);
+  int lag_parts = 0, parts = 0;
   if (h->schedule == FLOWHIP_MARCH)
     FK_LAUNCH(h, "lagrangian",
               fk_march_lagrangian(m, st->rho, st->e, st->mom_x, st->mom_y, mx1,
-                                  my1, u0, v0, e1, rho0, lr, st->max_dt,
-                                  st->tt == 0, flowhip_rows(h, FLOWHIP_K_LAGRANGIAN, 0),
-                                  s));
+                                  my1, u0, v0, e1, rho0, lr, st->max_dt, &lag_parts,
+                                  flowhip_rows(h, FLOWHIP_K_LAGRANGIAN, 0), s));
   else
     FK_LAUNCH(h, "lagrangian",
               fk_lagrangian(m, st->rho, st->e, st->mom_x, st->mom_y, mx1, my1,
@@ -41,7 +41,8 @@ void flowhip_step_fused(FlowHipCtx* h, const FlowHipStep* st) {
   if (h->schedule == FLOWHIP_MARCH)
     FK_LAUNCH(h, "advect_mass_energy",
               fk_march_mass_energy(m, st->tt, u0, v0, rho0, e1, st->rho, st->e,
-                                   st->F_x, st->F_y, h->red,
+                                   st->F_x, st->F_y, h->red, st->max_dt, st->tt == 0,
+                                   lr.cfl ? 0 : lag_parts, &parts,
                                    flowhip_rows(h, FLOWHIP_K_MASS, 0), s));
   else
     FK_LAUNCH(h, "advect_mass_energy",
@@ -51,7 +52,7 @@ void flowhip_step_fused(FlowHipCtx* h, const FlowHipStep* st) {
     FK_LAUNCH(h, "advect_momentum",
               fk_march_momentum(m, st->tt, u0, v0, st->F_x, st->F_y, st->rho, mx1,
                                 my1, st->mom_x, st->mom_y, st->u, st->v,
-                                h->red, flowhip_rows(h, FLOWHIP_K_MOMENTUM, 0), s));
+                                h->red, parts, flowhip_rows(h, FLOWHIP_K_MOMENTUM, 0), s));
   } else {
     FK_LAUNCH(h, "advect_momentum_x",
               fk_advect_momentum_x(m, st->tt, u0, v0, st->F_x, st->F_y, st->rho,

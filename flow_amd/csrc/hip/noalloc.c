@@ -98,14 +98,14 @@ int flowhip_solve_hydro_2d_static(Mesh* mesh, int tt, double* P, double* rho,
   HIPCHECK(fk_reciprocal(ny + 1, inv_y, mesh->edgedy, stream));
   flowhip_step_fused(&h, &st);
 
-  /* dt pair and totals are adjacent in the scratch: one copy */
-  double out[4];
+  /* the dt pairs and the totals are adjacent in the scratch: one copy */
+  double out[6];
   HIPCHECK(hipMemcpyAsync(out, h.red.dtp, sizeof(out), hipMemcpyDeviceToHost, stream));
   HIPCHECK(hipStreamSynchronize(stream));
   mesh->dt = out[0];
   mesh->dt_h = out[1];
-  if (mass) *mass = out[2];
-  if (energy) *energy = out[3];
+  if (mass) *mass = out[4];
+  if (energy) *energy = out[5];
   if (!isfinite(mesh->dt) || !(mesh->dt > 0.0) || !isfinite(mesh->dt_h)) {
     fprintf(stderr, "flowhip_solve_hydro_2d_static: non-finite or non-positive "
                     "timestep (dt=%.12e dt_h=%.12e): the state has diverged\n",

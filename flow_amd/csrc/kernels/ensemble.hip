@@ -82,8 +82,8 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_lagrangian(
     unsigned int* __restrict__ queue,
     int H, FkEnsPartials part) {
   const int lane = threadIdx.x % kWave;
-  MarchQueue<true> mq(queue, nwork);
-  for (int w = mq.next(); w < mq.end; w = mq.next()) {
+  MarchQueue<true> mq(queue, kStageLag, nwork, blockIdx.x, gridDim.x);
+  for (int w = mq.first(); w < mq.end; w = mq.next()) {
     const int2 wi = work[w];
     const FkEnsInst& in = insts[wi.x];
     const MLagIO<T> io{arr<T>(in, kRho),   arr<T>(in, kE),   arr<T>(in, kMomX),
@@ -113,7 +113,6 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_lagrangian(
       part.nan[in.item0 + wi.y] = nan_count;
     }
   }
-  mq.finish();
 }
 
 template <typename T, bool P2, bool UNI>
@@ -122,8 +121,8 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_mass(
     unsigned int* __restrict__ queue,
     int H, int tt, FkEnsPartials part) {
   const int lane = threadIdx.x % kWave;
-  MarchQueue<true> mq(queue, nwork);
-  for (int w = mq.next(); w < mq.end; w = mq.next()) {
+  MarchQueue<true> mq(queue, kStageMass, nwork, blockIdx.x, gridDim.x);
+  for (int w = mq.first(); w < mq.end; w = mq.next()) {
     const int2 wi = work[w];
     const FkEnsInst& in = insts[wi.x];
     const MMassIO<T> io{arr<T>(in, kUFx), arr<T>(in, kUFy), arr<T>(in, kRhoOld),
@@ -155,7 +154,6 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_mass(
       p[3] = es.c;
     }
   }
-  mq.finish();
 }
 
 /* ydir 0: x momentum (u0 = uF_x), 1: y momentum (io.u = the u just written) */
@@ -165,8 +163,9 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_momentum(
     unsigned int* __restrict__ queue,
     int H, int tt, int ydir) {
   const int lane = threadIdx.x % kWave;
-  MarchQueue<true> mq(queue, nwork);
-  for (int w = mq.next(); w < mq.end; w = mq.next()) {
+  /* no epilogue kernel between the two directions: a set each */
+  MarchQueue<true> mq(queue, ydir ? kStageLag : kStageMom, nwork, blockIdx.x, gridDim.x);
+  for (int w = mq.first(); w < mq.end; w = mq.next()) {
     const int2 wi = work[w];
     const FkEnsInst& in = insts[wi.x];
     const T dt = T(in.dtp[0]), dt_h = T(in.dtp[1]);
@@ -190,7 +189,6 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_momentum(
         momy_yx_item<T, P2>(g, io, dt, dt_h, ml, wi.y, lane);
     }
   }
-  mq.finish();
 }
 
 /* Both momentum directions in one march (momxy_*_item). */
@@ -202,8 +200,8 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_momentum_xy(
   const int lane = threadIdx.x % kWave;
   /* claimed per block, as the single-mesh fused momentum march */
   const int wave = threadIdx.x / kWave;
-  MarchBlockQueue mq(queue, nwork);
-  for (int base = mq.next(); base < mq.end; base = mq.next()) {
+  MarchBlockQueue mq(queue, kStageMom, nwork, blockIdx.x, gridDim.x);
+  for (int base = mq.first(); base < mq.end; base = mq.next()) {
     const int w = __builtin_amdgcn_readfirstlane(base + wave);
     if (w >= mq.end) continue;
     const int2 wi = work[w];
@@ -228,7 +226,6 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_momentum_xy(
         momxy_yx_item<T, P2, 0, false, UNI>(g, io, dt, dt_h, ml, wi.y, lane);
     }
   }
-  mq.finish();
 }
 
 /* CFL candidates of one item's cells (the pre-loop set_timestep). */
@@ -238,8 +235,8 @@ __global__ __launch_bounds__(kMNT) void k_ens_timestep(
     unsigned int* __restrict__ queue,
     int H, FkEnsPartials part) {
   const int lane = threadIdx.x % kWave;
-  MarchQueue<true> mq(queue, nwork);
-  for (int w = mq.next(); w < mq.end; w = mq.next()) {
+  MarchQueue<true> mq(queue, kStageLag, nwork, blockIdx.x, gridDim.x);
+  for (int w = mq.first(); w < mq.end; w = mq.next()) {
     const int2 wi = work[w];
     const FkEnsInst& in = insts[wi.x];
     const MGeo<T> g = ens_geo<T>(in);
@@ -271,18 +268,21 @@ __global__ __launch_bounds__(kMNT) void k_ens_timestep(
       part.nan[in.item0 + wi.y] = nan_count;
     }
   }
-  mq.finish();
 }
 
-/* ---- per-instance epilogues: one wave per instance ---- */
+/* ---- per-instance epilogues: one wave per instance ----
+ * One of them follows each march stage of a step; its first block also
+ * zeroes the work-queue counters, which no other kernel uses meanwhile. */
 
 /* dt pair of omp3/flow.c:103-105 from the instance's item minima; history
  * row *counter when hist != null. */
 __global__ __launch_bounds__(kWave) void k_ens_dt(const FkEnsInst* __restrict__ insts,
                                                   int ninst, FkEnsPartials part,
                                                   int first_step, int squared,
-                                                  FkEnsHistory hist) {
+                                                  FkEnsHistory hist,
+                                                  unsigned int* __restrict__ queue) {
   const int inst = blockIdx.x;
+  if (inst == 0) march_queue_reset(queue, -1);
   if (inst >= ninst) return;
   const FkEnsInst& in = insts[inst];
   const int lane = threadIdx.x;
@@ -314,8 +314,10 @@ __global__ __launch_bounds__(kWave) void k_ens_dt(const FkEnsInst* __restrict__ 
  * order; history row *counter. */
 __global__ __launch_bounds__(kWave) void k_ens_sums(const FkEnsInst* __restrict__ insts,
                                                     int ninst, FkEnsPartials part,
-                                                    FkEnsHistory hist) {
+                                                    FkEnsHistory hist,
+                                                    unsigned int* __restrict__ queue) {
   const int inst = blockIdx.x;
+  if (inst == 0) march_queue_reset(queue, -1);
   if (inst >= ninst) return;
   const FkEnsInst& in = insts[inst];
   const int lane = threadIdx.x;
@@ -334,8 +336,10 @@ __global__ __launch_bounds__(kWave) void k_ens_sums(const FkEnsInst* __restrict_
   }
 }
 
-__global__ void k_ens_advance(int* counter) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *counter += 1;
+__global__ __launch_bounds__(kWave) void k_ens_advance(int* counter,
+                                                       unsigned int* __restrict__ queue) {
+  march_queue_reset(queue, -1);
+  if (threadIdx.x == 0) *counter += 1;
 }
 
 __global__ void k_ens_set_counter(int* counter, int v) {
@@ -355,12 +359,12 @@ hipError_t ens_step_p(const FkEnsLaunch& L, int tt, hipStream_t s) {
                      dim3(kMNT), 0, s, L.insts, work, nw, L.queue, L.chunk_rows, L.part);
   hipLaunchKernelGGL(k_ens_dt, dim3(L.ninst), dim3(kWave), 0, s, L.insts, L.ninst,
                      L.part, tt == 0 ? 1 : 0, std::is_same<T, float>::value ? 1 : 0,
-                     L.hist);
+                     L.hist, L.queue);
   hipLaunchKernelGGL((k_ens_mass<T, P2, UNI>),
                      dim3(march_grid(k_ens_mass<T, P2, UNI>, pc_mass, nw, kMarchMaxWaves<T>)),
                      dim3(kMNT), 0, s, L.insts, work, nw, L.queue, L.chunk_rows, tt, L.part);
   hipLaunchKernelGGL(k_ens_sums, dim3(L.ninst), dim3(kWave), 0, s, L.insts, L.ninst,
-                     L.part, L.hist);
+                     L.part, L.hist, L.queue);
   if (L.fused_momentum) {
     static int pc_momxy = 0;
     hipLaunchKernelGGL((k_ens_momentum_xy<T, P2, UNI>),
@@ -374,7 +378,7 @@ hipError_t ens_step_p(const FkEnsLaunch& L, int tt, hipStream_t s) {
     hipLaunchKernelGGL((k_ens_momentum<T, P2>), dim3(gm), dim3(kMNT), 0, s, L.insts,
                        work, nw, L.queue, L.chunk_rows, tt, 1);
   }
-  hipLaunchKernelGGL(k_ens_advance, dim3(1), dim3(1), 0, s, L.hist.counter);
+  hipLaunchKernelGGL(k_ens_advance, dim3(1), dim3(kWave), 0, s, L.hist.counter, L.queue);
   return hipGetLastError();
 }
 
@@ -399,7 +403,7 @@ hipError_t ens_timestep(const FkEnsLaunch& L, hipStream_t s) {
                      dim3(kMNT), 0, s, L.insts, (const int2*)L.work, nw, L.queue,
                      L.chunk_rows, L.part);
   hipLaunchKernelGGL(k_ens_dt, dim3(L.ninst), dim3(kWave), 0, s, L.insts, L.ninst,
-                     L.part, 0, 0, none);
+                     L.part, 0, 0, none, L.queue);
   return hipGetLastError();
 }
 

@@ -127,7 +127,6 @@ template <typename T>
 __global__ __launch_bounds__(kNT, FLOWHIP_MIN_WAVES) void k_lagrangian(Geo<T> g, LagIO<T> io,
                                                     const double* dtp,
                                                     FkReduce red, double max_dt,
-                                                    int first_step,
                                                     TileList tl) {
   constexpr int TX = kTX, TY = kTY, NT = kNT;
   const int nx = g.nx, ny = g.ny, sx = nx + 1;
@@ -274,7 +273,7 @@ __global__ __launch_bounds__(kNT, FLOWHIP_MIN_WAVES) void k_lagrangian(Geo<T> g,
     else
       body(std::false_type{});
   }
-  finish_timestep<NT>(local_min, nan_count, red, max_dt, first_step);
+  publish_min<NT>(local_min, nan_count, red);
 }
 
 /* ======================================================================= */
@@ -381,7 +380,7 @@ __global__ __launch_bounds__(kNT, FLOWHIP_MIN_WAVES) void k_mass_energy_xy(Geo<T
     else
       body(std::false_type{});
   }
-  finish_sums<NT>(ms, es, red);
+  publish_sums<NT>(ms, es, red);
 }
 
 /* y-sweep first (odd tt, omp3/flow.c:315-322). */
@@ -473,7 +472,7 @@ __global__ __launch_bounds__(kNT, FLOWHIP_MIN_WAVES) void k_mass_energy_yx(Geo<T
     else
       body(std::false_type{});
   }
-  finish_sums<NT>(ms, es, red);
+  publish_sums<NT>(ms, es, red);
 }
 
 /* ======================================================================= */
@@ -869,8 +868,9 @@ hipError_t launch_lagrangian(Geo<T> g, LagIO<T> io, FkReduce r, double max_dt,
   static int per_cu = 0;
   const int grid = grid_for(k_lagrangian<T>, per_cu, tl.ntiles);
   hipLaunchKernelGGL(k_lagrangian<T>, dim3(grid), dim3(kNT), 0, s, g, io,
-                     (const double*)r.dtp, r, max_dt, first_step, tl);
-  return hipGetLastError();
+                     (const double*)r.dtp, r, max_dt, tl);
+  /* with r.cfl set, fk_timestep_serial makes the update from the candidates */
+  return r.cfl ? hipGetLastError() : fk_finish_timestep(r, grid, max_dt, first_step, s);
 }
 
 template <typename T>
@@ -878,18 +878,19 @@ hipError_t launch_mass_energy(Geo<T> g, MassIO<T> io, int tt, FkReduce r,
                               hipStream_t s) {
   const TileList tl = make_tiles(g.nx, g.ny, kTX, kTY);
   if (tl.ntiles < 1) return hipErrorInvalidValue;
+  int grid;
   if (tt % 2 == 0) {
     static int per_cu = 0;
-    const int grid = grid_for(k_mass_energy_xy<T>, per_cu, tl.ntiles);
+    grid = grid_for(k_mass_energy_xy<T>, per_cu, tl.ntiles);
     hipLaunchKernelGGL(k_mass_energy_xy<T>, dim3(grid), dim3(kNT), 0, s, g, io,
                        (const double*)r.dtp, r, tl);
   } else {
     static int per_cu = 0;
-    const int grid = grid_for(k_mass_energy_yx<T>, per_cu, tl.ntiles);
+    grid = grid_for(k_mass_energy_yx<T>, per_cu, tl.ntiles);
     hipLaunchKernelGGL(k_mass_energy_yx<T>, dim3(grid), dim3(kNT), 0, s, g, io,
                        (const double*)r.dtp, r, tl);
   }
-  return hipGetLastError();
+  return fk_finish_sums(r, grid, s);
 }
 
 template <typename T>

@@ -162,48 +162,68 @@ __device__ __forceinline__ MarchWalk march_walk(int nitems) {
   return w;
 }
 
-/* Dynamic form of the banded walk: the waves of band b claim its items one
- * at a time from band b's counter (atomicAdd by lane 0) as they finish the
- * previous one, so a wave that draws short or fast items takes more of them
- * and the band's waves finish together. Claiming the next item when
+/* Dynamic form of the banded walk. Wave k of band b starts on the band's
+ * item k; as the waves finish an item they claim the band's further items
+ * one at a time from band b's counter (atomicAdd by lane 0), so a wave that
+ * draws short or fast items takes more of them and the band's waves finish
+ * together. A band with no more items than waves (a mesh that does not fill
+ * the GPU, march_grid) takes no atomic at all. Claiming the next item when
  * starting the current one, to hide the claim's round trip, was slower on
  * MI355X: a wave then holds an item it cannot start, and the band's tail
- * grows by up to an item. The last wave of the grid to run out (counter
- * kMarchBands) resets every counter, so they are zero between launches
- * without a memset (the launches stay capturable in a graph). Every wave
- * reaches finish(); no wave waits on another. UNIFORM as for march_walk.
+ * grows by up to an item. No wave waits on another. UNIFORM as for
+ * march_walk.
  *
- * Counter k lives at queue[k * kQueueStride], one per 128-byte line: with
- * all of them in one line the claims of the eight bands serialise on it,
- * and the kernels ran 2-3% slower on MI355X. */
+ * The counters come in sets, one per stage of a step. A launch uses its
+ * stage's set, which is zero when it starts, and zeroes the other sets
+ * (march_queue_reset; the ensemble's epilogue kernels do it there), so no
+ * wave counts itself out at the end of a kernel and no memset is needed
+ * (the launches stay capturable in a graph). Counting the waves out, with
+ * the last one resetting the counters, was an atomic per wave on one
+ * address, up to 30 us at the end of a launch whose 2800 waves end together.
+ *
+ * Counter b of a set lives at set + b * kQueueStride, one per 128-byte line:
+ * with all of them in one line the claims of the eight bands serialise on
+ * it, and the kernels ran 2-3% slower on MI355X. */
 constexpr int kQueueStride = 32;
-static_assert((kMarchBands + 1) * kQueueStride <= FK_MARCH_QUEUE_WORDS, "queue counters");
+constexpr int kQueueSet = kMarchBands * kQueueStride;
+constexpr int kQueueSets = 3;
+static_assert(kQueueSets * kQueueSet <= FK_MARCH_QUEUE_WORDS, "queue counters");
+/* sets of the three stages of a step */
+enum { kStageLag = 0, kStageMass = 1, kStageMom = 2 };
 
-template <bool UNIFORM, int BANDS = kMarchBands>
+/* Zeroes every set but `stage` (-1: every set), by the first threads of one
+ * block; the sets' users run in other launches. */
+__device__ __forceinline__ void march_queue_reset(unsigned int* queue, int stage) {
+  const int k = threadIdx.x;
+  if (k < kQueueSets * kMarchBands && k / kMarchBands != stage) queue[k * kQueueStride] = 0u;
+}
+
+template <bool UNIFORM>
 struct MarchQueue {
-  static_assert(BANDS >= 1 && BANDS <= kMarchBands, "bands");
   unsigned int* ctr;
-  int lo, end, band;
-  __device__ MarchQueue(unsigned int* queue, int nitems) : ctr(queue) {
-    const int nb = gridDim.x;
-    const int bands = nb < BANDS ? nb : BANDS;
-    band = blockIdx.x % bands;
+  int lo, end, waves, head;
+  /* the queue of block blk of nblk marching blocks, on set `stage` */
+  __device__ MarchQueue(unsigned int* queue, int stage, int nitems, int blk, int nblk) {
+    const int bands = nblk < kMarchBands ? nblk : kMarchBands;
+    const int band = blk % bands, local = blk / bands;
+    ctr = queue + stage * kQueueSet + band * kQueueStride;
     lo = (int)((long)band * nitems / bands);
     end = (int)((long)(band + 1) * nitems / bands);
+    waves = (nblk - band + bands - 1) / bands * kMWaves;
+    head = lo + local * kMWaves;
   }
-  /* the next item of the band; end or beyond once the band is drained */
+  /* the wave's first item (end or beyond: none) */
+  __device__ int first() const {
+    const int k = head + (int)threadIdx.x / kWave;
+    return UNIFORM ? __builtin_amdgcn_readfirstlane(k) : k;
+  }
+  /* the wave's next item; end or beyond once the band is drained */
   __device__ int next() {
+    if (end - lo <= waves) return end;
     unsigned int v = 0;
-    if (threadIdx.x % kWave == 0) v = atomicAdd(&ctr[band * kQueueStride], 1u);
-    if (UNIFORM) return lo + (int)__builtin_amdgcn_readfirstlane(v);
-    return lo + (int)__shfl(v, 0, kWave);
-  }
-  __device__ void finish() {
-    if (threadIdx.x % kWave == 0) {
-      const unsigned int waves = gridDim.x * kMWaves;
-      if (atomicAdd(&ctr[kMarchBands * kQueueStride], 1u) == waves - 1)
-        for (int k = 0; k <= kMarchBands; ++k) atomicExch(&ctr[k * kQueueStride], 0u);
-    }
+    if (threadIdx.x % kWave == 0) v = atomicAdd(ctr, 1u);
+    if (UNIFORM) return lo + waves + (int)__builtin_amdgcn_readfirstlane(v);
+    return lo + waves + (int)__shfl(v, 0, kWave);
   }
 };
 
@@ -217,22 +237,22 @@ struct MarchQueue {
  * they keep the per-wave queue). Every wave of the block takes part in
  * every claim, and the loop ends for the whole block at once:
  *
- *   MarchBlockQueue mq(queue, nitems);
- *   for (int base = mq.next(); base < mq.end; base = mq.next()) {
+ *   MarchBlockQueue mq(queue, stage, nitems, blk, nblk);
+ *   for (int base = mq.first(); base < mq.end; base = mq.next()) {
  *     const int item = base + wave;
  *     if (item < mq.end) ... march item ...
  *   }
- *   mq.finish();
  */
 struct MarchBlockQueue : MarchQueue<true> {
-  __device__ MarchBlockQueue(unsigned int* queue, int nitems)
-      : MarchQueue<true>(queue, nitems) {}
-  /* the block's next base item; the same in every wave */
+  __device__ MarchBlockQueue(unsigned int* queue, int stage, int nitems, int blk, int nblk)
+      : MarchQueue<true>(queue, stage, nitems, blk, nblk) {}
+  /* the block's first and next base item; the same in every wave */
+  __device__ int first() const { return head; }
   __device__ int next() {
     __shared__ int s_base;
+    if (end - lo <= waves) return end;
     __syncthreads(); /* every wave has read the previous base */
-    if (threadIdx.x == 0)
-      s_base = lo + (int)atomicAdd(&ctr[band * kQueueStride], (unsigned int)kMWaves);
+    if (threadIdx.x == 0) s_base = lo + waves + (int)atomicAdd(ctr, (unsigned int)kMWaves);
     __syncthreads();
     return __builtin_amdgcn_readfirstlane(s_base);
   }
@@ -553,6 +573,49 @@ struct PlainSum {
 template <typename T>
 using ItemSum = typename std::conditional<sizeof(T) == 4, PlainSum, CSum>::type;
 
+/* ---- the scalars of a step ----
+ * The dt pair of a step goes from kernel to kernel without a kernel of its
+ * own. FkReduce.dtp[0..1] is the pair the Lagrangian march uses; it leaves
+ * its blocks' CFL minima. Every block of the mass/energy march folds them
+ * (a few loads a thread, all from L2) and computes the new pair for itself;
+ * block 0 publishes it in dtp[2..3], where the momentum march reads it. The
+ * momentum march's block 0 marches nothing: it moves the new pair to
+ * dtp[0..1], which no block of that kernel reads, and folds the totals the
+ * mass/energy march's blocks left. */
+struct MarchStep {
+  double max_dt;
+  int first_step;
+  int lag_parts; /* blocks of the Lagrangian march; 0: dtp[0..1] holds the new
+                    pair already (FkReduce.cfl, fk_timestep_serial) */
+};
+
+template <typename T>
+__device__ __forceinline__ DtPair mass_pair(const FkReduce& red, const MarchStep& st) {
+  DtPair p{red.dtp[0], red.dtp[1]};
+  if (blockIdx.x == 0) march_queue_reset(red.queue, kStageMass);
+  double g = 0.0, bad = 0.0;
+  if (st.lag_parts) {
+    fold_min<kMNT, std::is_same<T, float>::value>(red, st.lag_parts, st.max_dt, g, bad);
+    p = next_pair(g, p.dt_h, st.first_step);
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    red.dtp[2] = p.dt;
+    red.dtp[3] = p.dt_h;
+    if (st.lag_parts) {
+      red.sums[2] = g;
+      red.status[1] = (int)bad;
+    }
+  }
+  return p;
+}
+
+/* Block 0 of the momentum march; parts: blocks of the mass/energy march. */
+__device__ __forceinline__ void step_epilogue(const FkReduce& red, int parts) {
+  march_queue_reset(red.queue, kStageMom);
+  if (threadIdx.x < 2) red.dtp[threadIdx.x] = red.dtp[2 + threadIdx.x];
+  fold_limbs<kMNT>(red, parts);
+}
+
 /* ======================================================================= */
 /* mass and energy, x sweep first (even tt)                                 */
 /* ======================================================================= */
@@ -853,14 +916,15 @@ __device__ __forceinline__ void mass_xy_pair(const MGeo<T>& g, const MMassIO<T>&
  * kMassW). */
 template <typename T, bool P2, bool UNI = false, bool PAIR = false>
 __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_mass_xy(
-    MGeo<T> g, MMassIO<T> io, const double* dtp, FkReduce red, MarchList ml) {
-  const T dt = T(dtp[0]), dt_h = T(dtp[1]);
+    MGeo<T> g, MMassIO<T> io, FkReduce red, MarchStep st, MarchList ml) {
+  const DtPair pair = mass_pair<T>(red, st);
+  const T dt = T(pair.dt), dt_h = T(pair.dt_h);
   const int lane = threadIdx.x % kWave;
   /* each item's per-lane compensated sums, rounded once, go into exact
    * accumulators: the totals do not depend on which wave takes which item */
   FixSum fm{0, 0, 0, 0}, fe{0, 0, 0, 0};
-  MarchQueue<true> mq(red.queue, ml.nitems);
-  for (int item = mq.next(); item < mq.end; item = mq.next()) {
+  MarchQueue<true> mq(red.queue, kStageMass, ml.nitems, blockIdx.x, gridDim.x);
+  for (int item = mq.first(); item < mq.end; item = mq.next()) {
     ItemSum<T> ms{0.0, 0.0}, es{0.0, 0.0};
     if constexpr (PAIR) {
       const ItemBox b = item_box(ml, g.nx, item);
@@ -880,8 +944,7 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_mass_xy(
     fm.add(ms.s + ms.c);
     fe.add(es.s + es.c);
   }
-  mq.finish();
-  finish_fixed_sums<kMNT>(fm, fe, red);
+  publish_limbs<kMNT>(fm, fe, red);
 }
 
 /* ======================================================================= */
@@ -1167,14 +1230,15 @@ __device__ __forceinline__ void mass_yx_pair(const MGeo<T>& g, const MMassIO<T>&
 
 template <typename T, bool P2, bool UNI = false, bool PAIR = false>
 __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_mass_yx(
-    MGeo<T> g, MMassIO<T> io, const double* dtp, FkReduce red, MarchList ml) {
-  const T dt = T(dtp[0]), dt_h = T(dtp[1]);
+    MGeo<T> g, MMassIO<T> io, FkReduce red, MarchStep st, MarchList ml) {
+  const DtPair pair = mass_pair<T>(red, st);
+  const T dt = T(pair.dt), dt_h = T(pair.dt_h);
   const int lane = threadIdx.x % kWave;
   /* each item's per-lane compensated sums, rounded once, go into exact
    * accumulators: the totals do not depend on which wave takes which item */
   FixSum fm{0, 0, 0, 0}, fe{0, 0, 0, 0};
-  MarchQueue<true> mq(red.queue, ml.nitems);
-  for (int item = mq.next(); item < mq.end; item = mq.next()) {
+  MarchQueue<true> mq(red.queue, kStageMass, ml.nitems, blockIdx.x, gridDim.x);
+  for (int item = mq.first(); item < mq.end; item = mq.next()) {
     ItemSum<T> ms{0.0, 0.0}, es{0.0, 0.0};
     if constexpr (PAIR) {
       const ItemBox b = item_box(ml, g.nx, item);
@@ -1194,8 +1258,7 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_mass_yx(
     fm.add(ms.s + ms.c);
     fe.add(es.s + es.c);
   }
-  mq.finish();
-  finish_fixed_sums<kMNT>(fm, fe, red);
+  publish_limbs<kMNT>(fm, fe, red);
 }
 
 
@@ -2195,16 +2258,16 @@ constexpr int kLagMinWaves = (PAIR && sizeof(T) == 4) ? kLagPairWaves<T> : 1;
 
 template <typename T, bool P2, bool UNI = false, bool PAIR = false>
 __global__ __launch_bounds__(kMNT) __attribute__((amdgpu_waves_per_eu(kLagMinWaves<T, PAIR>)))
-void k_march_lagrangian(MGeo<T> g, MLagIO<T> io, const double* dtp, FkReduce red,
-                        double max_dt, int first_step, MarchList ml) {
-  const T dt = T(dtp[0]), dt_h = T(dtp[1]);
+void k_march_lagrangian(MGeo<T> g, MLagIO<T> io, FkReduce red, double max_dt, MarchList ml) {
+  const T dt = T(red.dtp[0]), dt_h = T(red.dtp[1]);
+  if (blockIdx.x == 0) march_queue_reset(red.queue, kStageLag);
   const int lane = threadIdx.x % kWave;
   constexpr bool kSq = std::is_same<T, float>::value;
   double local_min = kSq ? max_dt * max_dt : max_dt;
   int nan_count = 0;
-  MarchBlockQueue mq(red.queue, ml.nitems);
+  MarchBlockQueue mq(red.queue, kStageLag, ml.nitems, blockIdx.x, gridDim.x);
   const int wave = threadIdx.x / kWave;
-  for (int base = mq.next(); base < mq.end; base = mq.next()) {
+  for (int base = mq.first(); base < mq.end; base = mq.next()) {
     const int item = __builtin_amdgcn_readfirstlane(base + wave);
     if (item >= mq.end) continue;
     if constexpr (PAIR) {
@@ -2231,8 +2294,7 @@ void k_march_lagrangian(MGeo<T> g, MLagIO<T> io, const double* dtp, FkReduce red
                                            nan_count);
     }
   }
-  mq.finish();
-  finish_timestep<kMNT, kSq>(local_min, nan_count, red, max_dt, first_step);
+  publish_min<kMNT>(local_min, nan_count, red);
 }
 
 /* ======================================================================= */
@@ -2618,12 +2680,16 @@ __device__ __forceinline__ void momxy_yx_item(const MGeo<T>& g, const MMom2IO<T>
 
 template <typename T, bool P2, bool UNI = false>
 __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_momxy_xy(
-    MGeo<T> g, MMom2IO<T> io, const double* dtp, unsigned int* queue, MarchList ml) {
-  const T dt = T(dtp[0]), dt_h = T(dtp[1]);
+    MGeo<T> g, MMom2IO<T> io, FkReduce red, int parts, MarchList ml) {
+  if (blockIdx.x == 0) {
+    step_epilogue(red, parts);
+    return;
+  }
+  const T dt = T(red.dtp[2]), dt_h = T(red.dtp[3]);
   const int lane = threadIdx.x % kWave;
   const int wave = threadIdx.x / kWave;
-  MarchBlockQueue mq(queue, ml.nitems);
-  for (int base = mq.next(); base < mq.end; base = mq.next()) {
+  MarchBlockQueue mq(red.queue, kStageMom, ml.nitems, blockIdx.x - 1, gridDim.x - 1);
+  for (int base = mq.first(); base < mq.end; base = mq.next()) {
     const int item = __builtin_amdgcn_readfirstlane(base + wave);
     if (item >= mq.end) continue;
     if (!item_edge(ml, g.nx, g.ny, item))
@@ -2633,17 +2699,20 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_momxy_xy(
     else
       momxy_xy_item<T, P2, 0, true, UNI>(g, io, dt, dt_h, ml, item, lane);
   }
-  mq.finish();
 }
 
 template <typename T, bool P2, bool UNI = false>
 __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_momxy_yx(
-    MGeo<T> g, MMom2IO<T> io, const double* dtp, unsigned int* queue, MarchList ml) {
-  const T dt = T(dtp[0]), dt_h = T(dtp[1]);
+    MGeo<T> g, MMom2IO<T> io, FkReduce red, int parts, MarchList ml) {
+  if (blockIdx.x == 0) {
+    step_epilogue(red, parts);
+    return;
+  }
+  const T dt = T(red.dtp[2]), dt_h = T(red.dtp[3]);
   const int lane = threadIdx.x % kWave;
   const int wave = threadIdx.x / kWave;
-  MarchBlockQueue mq(queue, ml.nitems);
-  for (int base = mq.next(); base < mq.end; base = mq.next()) {
+  MarchBlockQueue mq(red.queue, kStageMom, ml.nitems, blockIdx.x - 1, gridDim.x - 1);
+  for (int base = mq.first(); base < mq.end; base = mq.next()) {
     const int item = __builtin_amdgcn_readfirstlane(base + wave);
     if (item >= mq.end) continue;
     if (!item_edge(ml, g.nx, g.ny, item))
@@ -2653,12 +2722,13 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_momxy_yx(
     else
       momxy_yx_item<T, P2, 0, true, UNI>(g, io, dt, dt_h, ml, item, lane);
   }
-  mq.finish();
 }
 
 /* Persistent grid of a march kernel: as many blocks as stay resident on the
  * device (per_cu per CU, from the occupancy query on first use, at most
- * max_per_cu when that is positive), and no more than the items need. */
+ * max_per_cu when that is positive), and no more than give every band a wave
+ * for each of its items (a grid of nitems / kMWaves blocks left some bands an
+ * item short of waves, and the launch took two rounds of items for one). */
 template <typename K>
 int march_grid(K kernel, int& per_cu, int nitems, int max_per_cu = 0) {
   static int cus = 0;
@@ -2678,7 +2748,8 @@ int march_grid(K kernel, int& per_cu, int nitems, int max_per_cu = 0) {
     per_cu = 1;
   if (max_per_cu > 0 && per_cu > max_per_cu) per_cu = max_per_cu;
   long gsz = (long)cus * per_cu;
-  const long need = (nitems + kMWaves - 1) / kMWaves;
+  const long band = (nitems + kMarchBands - 1) / kMarchBands;
+  const long need = kMarchBands * ((band + kMWaves - 1) / kMWaves);
   if (gsz > need) gsz = need;
   if (gsz > kMaxReduceBlocks) gsz = kMaxReduceBlocks;
   return gsz < 1 ? 1 : (int)gsz;

@@ -77,25 +77,27 @@ inline MarchList march_items(int nx, int ny, int W, int chunk_rows, Taper t) {
 }
 
 template <typename T, bool P2, bool UNI, bool PAIR = false>
-hipError_t launch_march_mass_p(MGeo<T> g, MMassIO<T> io, int tt, FkReduce r,
-                               int chunk_rows, hipStream_t s) {
+hipError_t launch_march_mass_p(MGeo<T> g, MMassIO<T> io, int tt, FkReduce r, MarchStep st,
+                               int* parts, int chunk_rows, hipStream_t s) {
   const MarchList ml = march_items(
       g.nx, g.ny, PAIR ? kMassW2 : kMassW, chunk_rows,
       PAIR ? (sizeof(T) == 8 ? Taper{FLOWHIP_TAPER_MASS64P} : Taper{FLOWHIP_TAPER_MASS32P})
            : taper_of<T>(kKMass));
-  if (ml.nitems < 1 || !r.queue || !r.totals) return hipErrorInvalidValue;
+  if (ml.nitems < 1 || !r.queue) return hipErrorInvalidValue;
   if (tt % 2 == 0) {
     static int per_cu = 0;
     const int grid = march_grid(k_march_mass_xy<T, P2, UNI, PAIR>, per_cu, ml.nitems,
                                 PAIR ? kMassPairWaves<T> : kMarchMaxWaves<T>);
     hipLaunchKernelGGL((k_march_mass_xy<T, P2, UNI, PAIR>), dim3(grid), dim3(kMNT), 0, s,
-                       g, io, (const double*)r.dtp, r, ml);
+                       g, io, r, st, ml);
+    *parts = grid;
   } else {
     static int per_cu = 0;
     const int grid = march_grid(k_march_mass_yx<T, P2, UNI, PAIR>, per_cu, ml.nitems,
                                 PAIR ? kMassPairWaves<T> : kMarchMaxWaves<T>);
     hipLaunchKernelGGL((k_march_mass_yx<T, P2, UNI, PAIR>), dim3(grid), dim3(kMNT), 0, s,
-                       g, io, (const double*)r.dtp, r, ml);
+                       g, io, r, st, ml);
+    *parts = grid;
   }
   return hipGetLastError();
 }
@@ -121,7 +123,7 @@ inline bool pairs_fit(const MGeo<T>& g, const MMassIO<T>& io) {
 
 template <typename T, bool P2, bool UNI, bool PAIR = false>
 hipError_t launch_march_lagrangian_p(MGeo<T> g, MLagIO<T> io, FkReduce r, double max_dt,
-                                     int first_step, int chunk_rows, hipStream_t s) {
+                                     int* parts, int chunk_rows, hipStream_t s) {
   const MarchList ml = march_items(
       g.nx, g.ny, PAIR ? kLagW2 : kLagW, chunk_rows,
       PAIR ? (sizeof(T) == 8 ? Taper{FLOWHIP_TAPER_LAG64P} : Taper{FLOWHIP_TAPER_LAG32P})
@@ -131,7 +133,8 @@ hipError_t launch_march_lagrangian_p(MGeo<T> g, MLagIO<T> io, FkReduce r, double
   const int grid = march_grid(k_march_lagrangian<T, P2, UNI, PAIR>, per_cu, ml.nitems,
                               PAIR ? kLagPairWaves<T> : kLagMaxWaves<T>);
   hipLaunchKernelGGL((k_march_lagrangian<T, P2, UNI, PAIR>), dim3(grid), dim3(kMNT), 0, s,
-                     g, io, (const double*)r.dtp, r, max_dt, first_step, ml);
+                     g, io, r, max_dt, ml);
+  *parts = grid;
   return hipGetLastError();
 }
 
@@ -184,22 +187,23 @@ hipError_t launch_march_momentum_p(MGeo<T> g, MMomIO<T> io, int tt, int ydir,
 constexpr int kMomXYW = kWave - 5;
 
 template <typename T, bool P2, bool UNI>
-hipError_t launch_march_momxy_p(MGeo<T> g, MMom2IO<T> io, int tt, const double* dtp,
-                                unsigned int* queue, int chunk_rows, hipStream_t s) {
+hipError_t launch_march_momxy_p(MGeo<T> g, MMom2IO<T> io, int tt, FkReduce r, int parts,
+                                int chunk_rows, hipStream_t s) {
   const MarchList ml = march_items(g.nx, g.ny, kMomXYW, chunk_rows, taper_of<T>(kKMom));
-  if (ml.nitems < 1 || !queue) return hipErrorInvalidValue;
+  if (ml.nitems < 1 || !r.queue) return hipErrorInvalidValue;
+  /* one block more, for the step's epilogue */
   if (tt % 2) {
     static int per_cu = 0;
     const int grid =
         march_grid(k_march_momxy_xy<T, P2, UNI>, per_cu, ml.nitems, kMarchMaxWaves<T>);
-    hipLaunchKernelGGL((k_march_momxy_xy<T, P2, UNI>), dim3(grid), dim3(kMNT), 0, s, g,
-                       io, dtp, queue, ml);
+    hipLaunchKernelGGL((k_march_momxy_xy<T, P2, UNI>), dim3(grid + 1), dim3(kMNT), 0, s, g,
+                       io, r, parts, ml);
   } else {
     static int per_cu = 0;
     const int grid =
         march_grid(k_march_momxy_yx<T, P2, UNI>, per_cu, ml.nitems, kMarchMaxWaves<T>);
-    hipLaunchKernelGGL((k_march_momxy_yx<T, P2, UNI>), dim3(grid), dim3(kMNT), 0, s, g,
-                       io, dtp, queue, ml);
+    hipLaunchKernelGGL((k_march_momxy_yx<T, P2, UNI>), dim3(grid + 1), dim3(kMNT), 0, s, g,
+                       io, r, parts, ml);
   }
   return hipGetLastError();
 }
@@ -209,33 +213,30 @@ hipError_t launch_march_momxy_p(MGeo<T> g, MMom2IO<T> io, int tt, const double* 
  * and fused momentum marches, whether such a mesh is also uniform (row
  * geometry read once per item). */
 template <typename T>
-hipError_t launch_march_mass(MGeo<T> g, MMassIO<T> io, int tt, FkReduce r,
-                             int chunk_rows, int pow2, int uniform, int pairs, hipStream_t s) {
+hipError_t launch_march_mass(MGeo<T> g, MMassIO<T> io, int tt, FkReduce r, MarchStep st,
+                             int* parts, int chunk_rows, int pow2, int uniform, int pairs,
+                             hipStream_t s) {
   if (pairs_wanted(pairs, g.nx, g.ny) && pow2 && uniform && pairs_fit(g, io))
-    return launch_march_mass_p<T, true, true, true>(g, io, tt, r, chunk_rows, s);
-  if (pow2 && uniform) return launch_march_mass_p<T, true, true>(g, io, tt, r, chunk_rows, s);
-  return pow2 ? launch_march_mass_p<T, true, false>(g, io, tt, r, chunk_rows, s)
-              : launch_march_mass_p<T, false, false>(g, io, tt, r, chunk_rows, s);
+    return launch_march_mass_p<T, true, true, true>(g, io, tt, r, st, parts, chunk_rows, s);
+  if (pow2 && uniform) return launch_march_mass_p<T, true, true>(g, io, tt, r, st, parts, chunk_rows, s);
+  return pow2 ? launch_march_mass_p<T, true, false>(g, io, tt, r, st, parts, chunk_rows, s)
+              : launch_march_mass_p<T, false, false>(g, io, tt, r, st, parts, chunk_rows, s);
 }
 
 /* The Lagrangian march takes the uniform-mesh form in FP32 only (in FP64 it
  * measured 1% slower than the per-row loads). */
 template <typename T>
 hipError_t launch_march_lagrangian(MGeo<T> g, MLagIO<T> io, FkReduce r, double max_dt,
-                                   int first_step, int chunk_rows, int pow2, int uniform,
+                                   int* parts, int chunk_rows, int pow2, int uniform,
                                    int pairs, hipStream_t s) {
   if (pairs_wanted(pairs, g.nx, g.ny) && pow2 && uniform && lag_pairs_fit(g, io))
-    return launch_march_lagrangian_p<T, true, true, true>(g, io, r, max_dt, first_step,
-                                                          chunk_rows, s);
+    return launch_march_lagrangian_p<T, true, true, true>(g, io, r, max_dt, parts, chunk_rows, s);
   if constexpr (sizeof(T) == 4) {
     if (pow2 && uniform)
-      return launch_march_lagrangian_p<T, true, true>(g, io, r, max_dt, first_step,
-                                                      chunk_rows, s);
+      return launch_march_lagrangian_p<T, true, true>(g, io, r, max_dt, parts, chunk_rows, s);
   }
-  return pow2 ? launch_march_lagrangian_p<T, true, false>(g, io, r, max_dt, first_step,
-                                                          chunk_rows, s)
-              : launch_march_lagrangian_p<T, false, false>(g, io, r, max_dt, first_step,
-                                                           chunk_rows, s);
+  return pow2 ? launch_march_lagrangian_p<T, true, false>(g, io, r, max_dt, parts, chunk_rows, s)
+              : launch_march_lagrangian_p<T, false, false>(g, io, r, max_dt, parts, chunk_rows, s);
 }
 
 template <typename T>
@@ -247,13 +248,12 @@ hipError_t launch_march_momentum(MGeo<T> g, MMomIO<T> io, int tt, int ydir,
 }
 
 template <typename T>
-hipError_t launch_march_momxy(MGeo<T> g, MMom2IO<T> io, int tt, const double* dtp,
-                              unsigned int* queue, int chunk_rows, int pow2, int uniform,
-                              hipStream_t s) {
+hipError_t launch_march_momxy(MGeo<T> g, MMom2IO<T> io, int tt, FkReduce r, int parts,
+                              int chunk_rows, int pow2, int uniform, hipStream_t s) {
   if (pow2 && uniform)
-    return launch_march_momxy_p<T, true, true>(g, io, tt, dtp, queue, chunk_rows, s);
-  return pow2 ? launch_march_momxy_p<T, true, false>(g, io, tt, dtp, queue, chunk_rows, s)
-              : launch_march_momxy_p<T, false, false>(g, io, tt, dtp, queue, chunk_rows, s);
+    return launch_march_momxy_p<T, true, true>(g, io, tt, r, parts, chunk_rows, s);
+  return pow2 ? launch_march_momxy_p<T, true, false>(g, io, tt, r, parts, chunk_rows, s)
+              : launch_march_momxy_p<T, false, false>(g, io, tt, r, parts, chunk_rows, s);
 }
 
 }  // namespace flowhip
@@ -271,20 +271,20 @@ extern "C" {
 hipError_t fk_march_lagrangian(FkMesh m, const double* rho, const double* e,
                                const double* mom_x, const double* mom_y, double* mx1,
                                double* my1, double* u0, double* v0, double* e1,
-                               double* rho_old, FkReduce r, double max_dt,
-                               int first_step, int chunk_rows, hipStream_t s) {
+                               double* rho_old, FkReduce r, double max_dt, int* parts,
+                               int chunk_rows, hipStream_t s) {
   MLagIO<double> io{rho, e, mom_x, mom_y, mx1, my1, u0, v0, e1, rho_old, r.cfl};
-  return launch_march_lagrangian<double>(mgeo64(m), io, r, max_dt, first_step,
-                                         chunk_rows, m.pow2, m.uniform, m.pairs, s);
+  return launch_march_lagrangian<double>(mgeo64(m), io, r, max_dt, parts, chunk_rows, m.pow2,
+                                         m.uniform, m.pairs, s);
 }
 
 hipError_t fk_march_momentum(FkMesh m, int tt, const double* u0, const double* v0,
                              const double* F_x, const double* F_y, const double* rho,
                              const double* mx1, const double* my1, double* mom_x,
                              double* mom_y, double* u, double* v, FkReduce r,
-                             int chunk_rows, hipStream_t s) {
+                             int parts, int chunk_rows, hipStream_t s) {
   MMom2IO<double> io{u0, v0, F_x, F_y, rho, mx1, my1, mom_x, mom_y, u, v};
-  return launch_march_momxy<double>(mgeo64(m), io, tt, r.dtp, r.queue, chunk_rows,
+  return launch_march_momxy<double>(mgeo64(m), io, tt, r, parts, chunk_rows,
                                     m.pow2, m.uniform, s);
 }
 
@@ -309,10 +309,12 @@ hipError_t fk_march_momentum_y(FkMesh m, int tt, const double* u1,
 hipError_t fk_march_mass_energy(FkMesh m, int tt, const double* u0,
                                 const double* v0, const double* rho0,
                                 const double* e1, double* rho, double* e,
-                                double* F_x, double* F_y, FkReduce r,
+                                double* F_x, double* F_y, FkReduce r, double max_dt,
+                                int first_step, int lag_parts, int* parts,
                                 int chunk_rows, hipStream_t s) {
   MMassIO<double> io{u0, v0, rho0, e1, rho, e, F_x, F_y};
-  return launch_march_mass<double>(mgeo64(m), io, tt, r, chunk_rows, m.pow2, m.uniform,
+  const MarchStep st{max_dt, first_step, lag_parts};
+  return launch_march_mass<double>(mgeo64(m), io, tt, r, st, parts, chunk_rows, m.pow2, m.uniform,
                                    m.pairs, s);
 }
 
@@ -326,20 +328,22 @@ hipError_t fk_march_lagrangian_f32(FkMesh32 m, const float* rho, const float* e,
                                    const float* mom_x, const float* mom_y,
                                    float* mx1, float* my1, float* u0, float* v0,
                                    float* e1, float* rho_old, FkReduce r,
-                                   double max_dt, int first_step, int chunk_rows,
+                                   double max_dt, int* parts, int chunk_rows,
                                    hipStream_t s) {
   MLagIO<float> io{rho, e, mom_x, mom_y, mx1, my1, u0, v0, e1, rho_old};
-  return launch_march_lagrangian<float>(mgeo32(m), io, r, max_dt, first_step,
-                                        chunk_rows, m.pow2, m.uniform, m.pairs, s);
+  return launch_march_lagrangian<float>(mgeo32(m), io, r, max_dt, parts, chunk_rows, m.pow2,
+                                        m.uniform, m.pairs, s);
 }
 
 hipError_t fk_march_mass_energy_f32(FkMesh32 m, int tt, const float* u0,
                                     const float* v0, const float* rho0,
                                     const float* e1, float* rho, float* e,
-                                    float* F_x, float* F_y, FkReduce r,
+                                    float* F_x, float* F_y, FkReduce r, double max_dt,
+                                    int first_step, int lag_parts, int* parts,
                                     int chunk_rows, hipStream_t s) {
   MMassIO<float> io{u0, v0, rho0, e1, rho, e, F_x, F_y};
-  return launch_march_mass<float>(mgeo32(m), io, tt, r, chunk_rows, m.pow2, m.uniform,
+  const MarchStep st{max_dt, first_step, lag_parts};
+  return launch_march_mass<float>(mgeo32(m), io, tt, r, st, parts, chunk_rows, m.pow2, m.uniform,
                                   m.pairs, s);
 }
 
@@ -347,9 +351,9 @@ hipError_t fk_march_momentum_f32(FkMesh32 m, int tt, const float* u0, const floa
                                  const float* F_x, const float* F_y, const float* rho,
                                  const float* mx1, const float* my1, float* mom_x,
                                  float* mom_y, float* u, float* v, FkReduce r,
-                                 int chunk_rows, hipStream_t s) {
+                                 int parts, int chunk_rows, hipStream_t s) {
   MMom2IO<float> io{u0, v0, F_x, F_y, rho, mx1, my1, mom_x, mom_y, u, v};
-  return launch_march_momxy<float>(mgeo32(m), io, tt, r.dtp, r.queue, chunk_rows,
+  return launch_march_momxy<float>(mgeo32(m), io, tt, r, parts, chunk_rows,
                                    m.pow2, m.uniform, s);
 }
 

@@ -1,10 +1,9 @@
 /*
  * noalloc.hip -- the device scratch of flowhip_solve_hydro_2d_static: one
  * file-scope device array holding every buffer the march step's kernels use
- * beyond the caller's arrays (the reduction partials and ticket, the dt
- * pair and totals, the status counts, the work-queue counters, the
- * fixed-point accumulators and the reciprocal edge spacings), so that the
- * entry point allocates nothing. Each GPU holds its own copy, at its own
+ * beyond the caller's arrays (the reduction partials, the dt pairs and
+ * totals, the status counts, the work-queue counters and the reciprocal
+ * edge spacings), so that the entry point allocates nothing. Each GPU holds its own copy, at its own
  * address, until the process ends.
  */
 #include "reduce_common.h"
@@ -13,24 +12,22 @@ namespace flowhip {
 namespace {
 
 /* Byte layout of the scratch, every part 256-byte aligned. The counter
- * words (ticket, status, queue, totals) are contiguous so one launch clears
- * them; the dt pair and the totals are contiguous so one copy reads both. */
+ * words (status, queue) are contiguous so one launch clears them; the dt
+ * pairs and the totals are contiguous so one copy reads both. */
 constexpr size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 constexpr size_t kOffPartials = 0;
-constexpr size_t kPartialsBytes = align256(sizeof(double) * 4 * kMaxReduceBlocks);
-constexpr size_t kOffTicket = kOffPartials + kPartialsBytes;
-constexpr size_t kOffStatus = kOffTicket + 256;
+constexpr size_t kPartialsBytes = align256(sizeof(double) * kPartialsDoubles);
+constexpr size_t kOffStatus = kOffPartials + kPartialsBytes;
 constexpr size_t kOffQueue = kOffStatus + 256;
-constexpr size_t kOffTotals = kOffQueue + align256(sizeof(unsigned int) * FK_MARCH_QUEUE_WORDS);
-constexpr size_t kOffPair = kOffTotals + align256(sizeof(unsigned long long) * FK_TOTALS_WORDS);
-constexpr size_t kCounterWords = (kOffPair - kOffTicket) / sizeof(unsigned int);
+constexpr size_t kOffPair = kOffQueue + align256(sizeof(unsigned int) * FK_MARCH_QUEUE_WORDS);
+constexpr size_t kCounterWords = (kOffPair - kOffStatus) / sizeof(unsigned int);
 /* the largest mesh the library indexes: FLOWHIP_MAX_CELLS_SIDE interior
  * cells a side, L + 1 = side + 5 edge spacings */
 constexpr int kMaxSide = 46335;
 constexpr size_t kInvBytes = align256(sizeof(double) * (kMaxSide + 5));
 constexpr size_t kOffInvX = kOffPair + 256;
 constexpr size_t kOffInvY = kOffInvX + kInvBytes;
-constexpr size_t kScratchBytes = kOffInvY + kInvBytes;  /* 1008896 B, < 1 MiB */
+constexpr size_t kScratchBytes = kOffInvY + kInvBytes;  /* 1007616 B, < 1 MiB */
 static_assert(kScratchBytes < (1u << 20), "scratch stays below 1 MiB");
 
 constexpr int kMaxDevices = 64;
@@ -77,13 +74,10 @@ hipError_t fk_static_scratch(FkReduce* r, double** inv_edgedx, double** inv_edge
   unsigned char* base = static_cast<unsigned char*>(g_scratch[dev]);
   FkReduce q;
   q.partials = reinterpret_cast<double*>(base + kOffPartials);
-  q.ticket = reinterpret_cast<unsigned int*>(base + kOffTicket);
   q.status = reinterpret_cast<int*>(base + kOffStatus);
   q.queue = reinterpret_cast<unsigned int*>(base + kOffQueue);
-  q.totals = reinterpret_cast<unsigned long long*>(base + kOffTotals);
   q.dtp = reinterpret_cast<double*>(base + kOffPair);
-  q.sums = q.dtp + 2; /* right after the dt pair: one copy reads both */
-  q.max_blocks = kMaxReduceBlocks;
+  q.sums = q.dtp + 4; /* right after the dt pairs: one copy reads both */
   q.cfl = nullptr;
   *r = q;
   *inv_edgedx = reinterpret_cast<double*>(base + kOffInvX);
@@ -93,11 +87,11 @@ hipError_t fk_static_scratch(FkReduce* r, double** inv_edgedx, double** inv_edge
   return hipSuccess;
 }
 
-/* Zero the counter words of r (ticket, status, queue, totals: the kernels
- * count on them starting at zero) and set the dt pair, in one launch. */
+/* Zero the counter words of r (status, queue: the kernels count on the
+ * queue's starting at zero) and set the dt pair, in one launch. */
 hipError_t fk_static_begin(FkReduce r, double dt, double dt_h, hipStream_t s) {
-  hipLaunchKernelGGL(k_static_begin, dim3(4), dim3(256), 0, s, r.ticket,
-                     (int)kCounterWords, r.dtp, dt, dt_h);
+  hipLaunchKernelGGL(k_static_begin, dim3(4), dim3(256), 0, s,
+                     reinterpret_cast<unsigned int*>(r.status), (int)kCounterWords, r.dtp, dt, dt_h);
   return hipGetLastError();
 }
 

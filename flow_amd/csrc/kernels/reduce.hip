@@ -1,12 +1,11 @@
 /*
- * reduce.hip -- single-pass grid reductions of the stagewise schedule: the
- * CFL timestep minimum (omp3/flow.c:77-105) and the conservation totals
+ * reduce.hip -- grid reductions of the stagewise schedule: the CFL timestep
+ * minimum (omp3/flow.c:77-105) and the conservation totals
  * (omp3/flow.c:973-995).
  *
- * Each block reduces its share through wave64 shuffles and LDS, writes one
- * partial, and takes a ticket; the last block to arrive combines the
- * partials, writes the result and resets the ticket to zero, so no memset is
- * needed between launches (or inside a captured graph).
+ * Each block reduces its share through wave64 shuffles and LDS and writes
+ * one partial; a one-block launch folds the partials (reduce_common.h says
+ * why that beats folding in the last block to finish).
  */
 #include "reduce_common.h"
 
@@ -25,24 +24,58 @@ template <typename M, typename T>
 __global__ __launch_bounds__(kRedThreads) void k_timestep(
     M m, const T* __restrict__ Qxx, const T* __restrict__ Qyy,
     const T* __restrict__ rho, const T* __restrict__ e, FkReduce r,
-    double max_dt, int first_step) {
-  const int pad = m.pad, wx = m.nx - 2 * pad, wy = m.ny - 2 * pad;
-  const long n = (long)wx * wy;
+    double max_dt) {
+  /* (the interior of the largest mesh has fewer than 2^31 cells, so a cell
+   * index and the stride past it fit 32 bits: one 32-bit division a cell) */
+  const int pad = m.pad;
+  const unsigned int wx = m.nx - 2 * pad, n = wx * (unsigned int)(m.ny - 2 * pad);
   double local = max_dt;
   int bad = 0;
-  for (long k = (long)blockIdx.x * blockDim.x + threadIdx.x; k < n;
-       k += (long)gridDim.x * blockDim.x) {
+  for (unsigned int k = blockIdx.x * blockDim.x + threadIdx.x; k < n;
+       k += gridDim.x * blockDim.x) {
     const int i = pad + (int)(k / wx), j = pad + (int)(k % wx);
     const int c = i * m.nx + j;
-    const double cand = cell_timestep(double(e[c]), double(Qxx[c]), double(Qyy[c]),
-                                      double(rho[c]), double(m.celldx[j]),
-                                      double(m.celldy[i]));
+    const double ec = double(e[c]), qx = double(Qxx[c]), qy = double(Qyy[c]),
+                 rc = double(rho[c]), dx = double(m.celldx[j]), dy = double(m.celldy[i]);
+    if (cfl_above(ec, qx, qy, rc, dx, dy, local * local)) continue;
+    const double cand = cell_timestep(ec, qx, qy, rc, dx, dy);
     if (cand == cand)
       local = lesser(local, cand);
     else
       ++bad;
   }
-  finish_timestep<kRedThreads>(local, bad, r, max_dt, first_step);
+  publish_min<kRedThreads>(local, bad, r);
+}
+
+/* The (dt, dt_h) update from parts blocks' minima. */
+__global__ __launch_bounds__(kRedThreads) void k_finish_timestep(FkReduce r, int parts,
+                                                                 double max_dt,
+                                                                 int first_step) {
+  double g, bad;
+  fold_min<kRedThreads, false>(r, parts, max_dt, g, bad);
+  if (threadIdx.x == 0) {
+    const DtPair p = next_pair(g, r.dtp[1], first_step);
+    r.dtp[0] = p.dt;
+    r.dtp[1] = p.dt_h;
+    r.sums[2] = g;
+    r.status[1] = (int)bad;
+  }
+}
+
+/* The totals from parts blocks' compensated sums. */
+__global__ __launch_bounds__(kRedThreads) void k_finish_sums(FkReduce r, int parts) {
+  CSum gm{0.0, 0.0}, ge{0.0, 0.0};
+  for (int b = threadIdx.x; b < parts; b += kRedThreads) {
+    const double* p = r.partials + kTotalsOffset + 4 * b;
+    gm.merge(CSum{p[0], p[1]});
+    ge.merge(CSum{p[2], p[3]});
+  }
+  gm = block_csum<kRedThreads>(gm);
+  ge = block_csum<kRedThreads>(ge);
+  if (threadIdx.x == 0) {
+    r.sums[0] = gm.s + gm.c;
+    r.sums[1] = ge.s + ge.c;
+  }
 }
 
 /* State of omp3's serial CFL fold over a run of consecutive candidates
@@ -87,15 +120,16 @@ __device__ __forceinline__ SerialFold wave_fold(double cand, bool valid) {
 
 /* omp3/flow.c:77-105 read as one OpenMP thread executes it (see
  * fk_timestep_serial): block b folds a contiguous range of the interior in
- * row-major order, its waves contiguous sub-ranges, 64 cells at a time; the
- * last block joins the blocks' folds in order. */
+ * row-major order, its waves contiguous sub-ranges, 64 cells at a time;
+ * k_finish_serial joins the blocks' folds in order. */
 template <bool kFromArrays>
 __global__ __launch_bounds__(kRedThreads) void k_timestep_serial(
     FkMesh m, const double* __restrict__ cfl, const double* __restrict__ Qxx,
     const double* __restrict__ Qyy, const double* __restrict__ rho,
-    const double* __restrict__ e, FkReduce r, double max_dt, int first_step) {
+    const double* __restrict__ e, FkReduce r) {
   constexpr int kWaves = kRedThreads / kWave;
   __shared__ SerialFold s_fold[kWaves];
+  __shared__ int s_bad[kWaves];
   const int pad = m.pad, wx = m.nx - 2 * pad, wy = m.ny - 2 * pad;
   const long n = (long)wx * wy;
   const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
@@ -115,53 +149,73 @@ __global__ __launch_bounds__(kRedThreads) void k_timestep_serial(
                          : cfl[c];
     }
     const SerialFold f = wave_fold(cand, valid);
-    if (kFromArrays && f.nan) bad += __popcll(__ballot(valid && cand != cand));
+    if (f.nan) bad += __popcll(__ballot(valid && cand != cand));
     acc = fold_join(acc, f);
   }
-  if (kFromArrays && lane == 0 && bad) atomicAdd(r.status, bad);
-  if (lane == 0) s_fold[w] = acc;
+  if (lane == 0) {
+    s_fold[w] = acc;
+    s_bad[w] = bad;
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
     SerialFold blk = s_fold[0];
-    for (int q = 1; q < kWaves; ++q) blk = fold_join(blk, s_fold[q]);
-    r.partials[2 * blockIdx.x] = blk.p;
-    r.partials[2 * blockIdx.x + 1] = (double)(blk.nan + 2 * blk.any);
+    int blk_bad = s_bad[0];
+    for (int q = 1; q < kWaves; ++q) {
+      blk = fold_join(blk, s_fold[q]);
+      blk_bad += s_bad[q];
+    }
+    double* p = r.partials + 4 * blockIdx.x;
+    p[0] = blk.p;
+    p[1] = (double)(blk.nan + 2 * blk.any);
+    p[2] = (double)blk_bad;
   }
-  if (!last_block_arrives(r.ticket)) return;
+}
+
+/* Joins the folds of parts blocks (at most kRedBlocks) in order, and the
+ * (dt, dt_h) update. */
+__global__ __launch_bounds__(kRedThreads) void k_finish_serial(FkReduce r, int parts,
+                                                               double max_dt,
+                                                               int first_step) {
+  __shared__ double s_p[kRedBlocks], s_flags[kRedBlocks], s_bad[kRedBlocks];
+  for (int b = threadIdx.x; b < parts; b += kRedThreads) {
+    s_p[b] = r.partials[4 * b];
+    s_flags[b] = r.partials[4 * b + 1];
+    s_bad[b] = r.partials[4 * b + 2];
+  }
+  __syncthreads();
   if (threadIdx.x == 0) {
     SerialFold all{__builtin_inf(), 0, 0};
-    for (int b = 0; b < (int)gridDim.x; ++b) {
-      const int flags = (int)r.partials[2 * b + 1];
-      all = fold_join(all, SerialFold{r.partials[2 * b], flags & 1, flags >> 1});
+    double bad = 0.0;
+    for (int b = 0; b < parts; ++b) {
+      const int flags = (int)s_flags[b];
+      all = fold_join(all, SerialFold{s_p[b], flags & 1, flags >> 1});
+      bad += s_bad[b];
     }
     /* OpenMP's min combiner merges the thread's fold into max_dt: a fold
      * that ends on a NaN leaves max_dt */
     const double g = lesser(all.p, max_dt);
-    const double dt_h = r.dtp[1];
-    const double final_min = lesser(g, kCM * dt_h);
-    const double dt = 0.5 * (kCT * final_min + dt_h);
-    r.dtp[0] = dt;
-    r.dtp[1] = first_step ? dt : kCT * final_min;
+    const DtPair p = next_pair(g, r.dtp[1], first_step);
+    r.dtp[0] = p.dt;
+    r.dtp[1] = p.dt_h;
     r.sums[2] = g;
-    r.status[1] = atomicExch(r.status, 0);
-    *r.ticket = 0u;
+    r.status[1] = (int)bad;
   }
 }
 
 template <typename M, typename T>
 __global__ __launch_bounds__(kRedThreads) void k_conservation(
     M m, const T* __restrict__ rho, const T* __restrict__ e, FkReduce r) {
-  const int pad = m.pad, wx = m.nx - 2 * pad, wy = m.ny - 2 * pad;
-  const long n = (long)wx * wy;
+  const int pad = m.pad;
+  const unsigned int wx = m.nx - 2 * pad, n = wx * (unsigned int)(m.ny - 2 * pad);
   CSum ms{0.0, 0.0}, es{0.0, 0.0};
-  for (long k = (long)blockIdx.x * blockDim.x + threadIdx.x; k < n;
-       k += (long)gridDim.x * blockDim.x) {
+  for (unsigned int k = blockIdx.x * blockDim.x + threadIdx.x; k < n;
+       k += gridDim.x * blockDim.x) {
     const int i = pad + (int)(k / wx), j = pad + (int)(k % wx);
     const int c = i * m.nx + j;
     ms.add(double(rho[c]));
     es.add(double(rho[c]) * double(e[c]));
   }
-  finish_sums<kRedThreads>(ms, es, r);
+  publish_sums<kRedThreads>(ms, es, r);
 }
 
 int red_blocks(long n) {
@@ -177,58 +231,68 @@ using namespace flowhip;
 
 extern "C" {
 
-int fk_reduce_blocks(void) { return 4 * kMaxReduceBlocks; }
+int fk_reduce_blocks(void) { return kPartialsDoubles; }
+
+hipError_t fk_finish_timestep(FkReduce r, int parts, double max_dt, int first_step,
+                              hipStream_t s) {
+  hipLaunchKernelGGL(k_finish_timestep, dim3(1), dim3(kRedThreads), 0, s, r, parts, max_dt,
+                     first_step);
+  return hipGetLastError();
+}
+
+hipError_t fk_finish_sums(FkReduce r, int parts, hipStream_t s) {
+  hipLaunchKernelGGL(k_finish_sums, dim3(1), dim3(kRedThreads), 0, s, r, parts);
+  return hipGetLastError();
+}
 
 hipError_t fk_timestep(FkMesh m, const double* Qxx, const double* Qyy,
                        const double* rho, const double* e, FkReduce r,
                        double max_dt, int first_step, hipStream_t s) {
-  const long n = (long)(m.nx - 2 * m.pad) * (m.ny - 2 * m.pad);
-  hipLaunchKernelGGL((k_timestep<FkMesh, double>), dim3(red_blocks(n)),
-                     dim3(kRedThreads), 0, s, m, Qxx, Qyy, rho, e, r, max_dt,
-                     first_step);
-  return hipGetLastError();
+  const int grid = red_blocks((long)(m.nx - 2 * m.pad) * (m.ny - 2 * m.pad));
+  hipLaunchKernelGGL((k_timestep<FkMesh, double>), dim3(grid), dim3(kRedThreads), 0, s, m,
+                     Qxx, Qyy, rho, e, r, max_dt);
+  return fk_finish_timestep(r, grid, max_dt, first_step, s);
 }
 
 hipError_t fk_timestep_serial(FkMesh m, const double* cfl, const double* Qxx,
                               const double* Qyy, const double* rho,
                               const double* e, FkReduce r, double max_dt,
                               int first_step, hipStream_t s) {
-  const long n = (long)(m.nx - 2 * m.pad) * (m.ny - 2 * m.pad);
-  /* two partials per block, within fk_reduce_blocks() */
-  const int grid = red_blocks(n);
+  const int grid = red_blocks((long)(m.nx - 2 * m.pad) * (m.ny - 2 * m.pad));
   if (cfl)
     hipLaunchKernelGGL(k_timestep_serial<false>, dim3(grid), dim3(kRedThreads), 0, s, m,
-                       cfl, Qxx, Qyy, rho, e, r, max_dt, first_step);
+                       cfl, Qxx, Qyy, rho, e, r);
   else
     hipLaunchKernelGGL(k_timestep_serial<true>, dim3(grid), dim3(kRedThreads), 0, s, m,
-                       cfl, Qxx, Qyy, rho, e, r, max_dt, first_step);
+                       cfl, Qxx, Qyy, rho, e, r);
+  hipLaunchKernelGGL(k_finish_serial, dim3(1), dim3(kRedThreads), 0, s, r, grid, max_dt,
+                     first_step);
   return hipGetLastError();
 }
 
 hipError_t fk_conservation(FkMesh m, const double* rho, const double* e,
                            FkReduce r, hipStream_t s) {
-  const long n = (long)(m.nx - 2 * m.pad) * (m.ny - 2 * m.pad);
-  hipLaunchKernelGGL((k_conservation<FkMesh, double>), dim3(red_blocks(n)),
-                     dim3(kRedThreads), 0, s, m, rho, e, r);
-  return hipGetLastError();
+  const int grid = red_blocks((long)(m.nx - 2 * m.pad) * (m.ny - 2 * m.pad));
+  hipLaunchKernelGGL((k_conservation<FkMesh, double>), dim3(grid), dim3(kRedThreads), 0, s,
+                     m, rho, e, r);
+  return fk_finish_sums(r, grid, s);
 }
 
 hipError_t fk_timestep_f32(FkMesh32 m, const float* Qxx, const float* Qyy,
                            const float* rho, const float* e, FkReduce r,
                            double max_dt, int first_step, hipStream_t s) {
-  const long n = (long)(m.nx - 2 * m.pad) * (m.ny - 2 * m.pad);
-  hipLaunchKernelGGL((k_timestep<FkMesh32, float>), dim3(red_blocks(n)),
-                     dim3(kRedThreads), 0, s, m, Qxx, Qyy, rho, e, r, max_dt,
-                     first_step);
-  return hipGetLastError();
+  const int grid = red_blocks((long)(m.nx - 2 * m.pad) * (m.ny - 2 * m.pad));
+  hipLaunchKernelGGL((k_timestep<FkMesh32, float>), dim3(grid), dim3(kRedThreads), 0, s, m,
+                     Qxx, Qyy, rho, e, r, max_dt);
+  return fk_finish_timestep(r, grid, max_dt, first_step, s);
 }
 
 hipError_t fk_conservation_f32(FkMesh32 m, const float* rho, const float* e,
                                FkReduce r, hipStream_t s) {
-  const long n = (long)(m.nx - 2 * m.pad) * (m.ny - 2 * m.pad);
-  hipLaunchKernelGGL((k_conservation<FkMesh32, float>), dim3(red_blocks(n)),
-                     dim3(kRedThreads), 0, s, m, rho, e, r);
-  return hipGetLastError();
+  const int grid = red_blocks((long)(m.nx - 2 * m.pad) * (m.ny - 2 * m.pad));
+  hipLaunchKernelGGL((k_conservation<FkMesh32, float>), dim3(grid), dim3(kRedThreads), 0, s,
+                     m, rho, e, r);
+  return fk_finish_sums(r, grid, s);
 }
 
 }  // extern "C"

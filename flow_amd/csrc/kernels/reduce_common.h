@@ -1,8 +1,8 @@
 /*
- * reduce_common.h -- block-level reductions and the single-pass epilogues
- * (the last block to arrive combines what the others left) shared by the
- * reduction kernels, the fused kernels and the march kernels: the CFL
- * minimum, compensated per-block totals, and exact fixed-point totals.
+ * reduce_common.h -- block-level reductions, the partials that blocks leave
+ * for the next kernel and their folds, shared by the reduction kernels, the
+ * fused kernels and the march kernels: the CFL minimum, compensated
+ * per-block totals, and exact fixed-point totals.
  */
 #pragma once
 
@@ -11,24 +11,16 @@
 
 namespace flowhip {
 
-/* Upper bound on blocks of any launch that writes reduction partials; the
- * partials buffer holds 4 doubles per block. */
-constexpr int kMaxReduceBlocks = 8192;
-
-/* Returns true in the one block that arrives last (all others have
- * finished their work and published their partials). */
-__device__ __forceinline__ bool last_block_arrives(unsigned int* ticket) {
-  __shared__ bool last;
-  __threadfence(); /* release this block's partial */
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const unsigned int prev = atomicAdd(ticket, 1u);
-    last = (prev == gridDim.x - 1);
-  }
-  __syncthreads();
-  if (last) __threadfence(); /* acquire the other blocks' partials */
-  return last;
-}
+/* Upper bound on blocks of any launch that leaves reduction partials in
+ * FkReduce.partials. */
+constexpr int kMaxReduceBlocks = 2048;
+/* Layout of FkReduce.partials, in doubles: two per block of the kernel that
+ * evaluates the CFL candidates (its minimum and its count of undefined
+ * candidates), then 14 64-bit words per block of the kernel that leaves the
+ * totals (block_limbs; the kernels with plain compensated sums use 4). */
+constexpr int kTotalsOffset = 2 * kMaxReduceBlocks;
+constexpr int kTotalsWords = 14;
+constexpr int kPartialsDoubles = kTotalsOffset + kTotalsWords * kMaxReduceBlocks;
 
 template <int NT>
 __device__ __forceinline__ double block_min(double x) {
@@ -64,64 +56,90 @@ __device__ __forceinline__ CSum block_csum(CSum v) {
   return v; /* valid in wave 0 */
 }
 
-/* Per-block CFL minimum -> last block -> (dt, dt_h) update of
- * omp3/flow.c:103-105 and the undefined-candidate count. With r.cfl set the
- * candidates were also stored for k_timestep_serial, which then does the
- * update and publishes the count; this only leaves the minimum over the
- * defined candidates in r.sums[2]. */
-/* kSquared: the candidates are squared time steps (the FP32-state form);
- * the minimum's square root is taken once, here. */
-template <int NT, bool kSquared = false>
-__device__ void finish_timestep(double local_min, int nan_count, FkReduce r,
-                                double max_dt, int first_step) {
-  if (nan_count) atomicAdd(r.status, nan_count);
+/* ---- grid reductions ----
+ * A block leaves its partial in FkReduce.partials with plain stores and the
+ * next kernel on the stream folds them: the kernel boundary orders the two.
+ * The single-pass form this replaces (every block fences its partial and
+ * takes a ticket, the last one folds) cost 45-60 ns a block on MI355X, one
+ * block after the other (each device-scope fence writes back the XCD's L2),
+ * at the end of the kernel where nothing overlaps it: the pre-loop
+ * set_timestep of a 512^2 mesh (1024 blocks) took 70 us of which 64 were
+ * that, the 752-block Lagrangian march of a 1000^2 mesh about 45 of 117. */
+
+/* A block's CFL minimum and its count of undefined candidates. */
+template <int NT>
+__device__ __forceinline__ void publish_min(double local_min, int nan_count, FkReduce r) {
+  __shared__ int s_nan[NT / kWave];
+  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) nan_count += __shfl_xor(nan_count, off, kWave);
+  if (lane == 0) s_nan[w] = nan_count;
   const double bmin = block_min<NT>(local_min);
-  if (threadIdx.x == 0) r.partials[blockIdx.x] = bmin;
-  if (!last_block_arrives(r.ticket)) return;
-  double g = kSquared ? max_dt * max_dt : max_dt;
-  for (int b = threadIdx.x; b < (int)gridDim.x; b += NT)
-    g = lesser(g, r.partials[b]);
-  g = block_min<NT>(g);
-  if (kSquared) g = __builtin_sqrt(g);
   if (threadIdx.x == 0) {
-    if (!r.cfl) {
-      const double dt_h = r.dtp[1];
-      const double final_min = lesser(g, kCM * dt_h);
-      const double dt = 0.5 * (kCT * final_min + dt_h);
-      r.dtp[0] = dt;
-      r.dtp[1] = first_step ? dt : kCT * final_min;
-      r.status[1] = atomicExch(r.status, 0);
-    }
-    r.sums[2] = g;
-    *r.ticket = 0u;
+    int bad = 0;
+    for (int k = 0; k < NT / kWave; ++k) bad += s_nan[k];
+    r.partials[2 * blockIdx.x] = bmin;
+    r.partials[2 * blockIdx.x + 1] = (double)bad;
   }
 }
 
-/* Per-block compensated sums -> last block -> r.sums[0..1]. */
+/* The minimum over parts blocks' partials and max_dt, and the undefined
+ * candidates' count; the same in every thread of the block. kSquared: the
+ * candidates are squared time steps (the FP32-state form); the minimum's
+ * square root is taken once, here. */
+template <int NT, bool kSquared>
+__device__ __forceinline__ void fold_min(const FkReduce& r, int parts, double max_dt,
+                                         double& g_out, double& bad_out) {
+  __shared__ double s_min[NT / kWave], s_bad[NT / kWave];
+  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
+  double g = kSquared ? max_dt * max_dt : max_dt, bad = 0.0;
+  for (int b = threadIdx.x; b < parts; b += NT) {
+    const double2 p = reinterpret_cast<const double2*>(r.partials)[b];
+    g = lesser(g, p.x);
+    bad += p.y;
+  }
+  g = wave_min(g);
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) bad += __shfl_xor(bad, off, kWave);
+  if (lane == 0) {
+    s_min[w] = g;
+    s_bad[w] = bad;
+  }
+  __syncthreads();
+  g = s_min[0];
+  bad = s_bad[0];
+#pragma unroll
+  for (int k = 1; k < NT / kWave; ++k) {
+    g = lesser(g, s_min[k]);
+    bad += s_bad[k];
+  }
+  g_out = kSquared ? __builtin_sqrt(g) : g;
+  bad_out = bad;
+}
+
+/* The (dt, dt_h) update of omp3/flow.c:103-105 from the grid minimum g. */
+struct DtPair {
+  double dt, dt_h;
+};
+__device__ __forceinline__ DtPair next_pair(double g, double dt_h, int first_step) {
+  const double final_min = lesser(g, kCM * dt_h);
+  DtPair p;
+  p.dt = 0.5 * (kCT * final_min + dt_h);
+  p.dt_h = first_step ? p.dt : kCT * final_min;
+  return p;
+}
+
+/* A block's compensated sums of the mass and energy. */
 template <int NT>
-__device__ void finish_sums(CSum ms, CSum es, FkReduce r) {
+__device__ void publish_sums(CSum ms, CSum es, FkReduce r) {
   ms = block_csum<NT>(ms);
   es = block_csum<NT>(es);
   if (threadIdx.x == 0) {
-    double* p = r.partials + 4 * blockIdx.x;
+    double* p = r.partials + kTotalsOffset + 4 * blockIdx.x;
     p[0] = ms.s;
     p[1] = ms.c;
     p[2] = es.s;
     p[3] = es.c;
-  }
-  if (!last_block_arrives(r.ticket)) return;
-  CSum gm{0.0, 0.0}, ge{0.0, 0.0};
-  for (int b = threadIdx.x; b < (int)gridDim.x; b += NT) {
-    const double* p = r.partials + 4 * b;
-    gm.merge(CSum{p[0], p[1]});
-    ge.merge(CSum{p[2], p[3]});
-  }
-  gm = block_csum<NT>(gm);
-  ge = block_csum<NT>(ge);
-  if (threadIdx.x == 0) {
-    r.sums[0] = gm.s + gm.c;
-    r.sums[1] = ge.s + ge.c;
-    *r.ticket = 0u;
   }
 }
 
@@ -181,12 +199,6 @@ __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long x)
   return x;
 }
 
-/* Accumulator word k of total q lives at r.totals[(8 q + k) * kTotalsStride],
- * one per 128-byte line, so the blocks' atomics on different words do not
- * queue on one line. */
-constexpr int kTotalsStride = 16;
-static_assert(16 * kTotalsStride <= FK_TOTALS_WORDS, "totals words");
-
 /* The double nearest (to within an ulp; the same bits every time) to the
  * fixed-point total held in 6 limb counters t[0..5] (t[k] counts units of
  * 2^(32k - 64), any size below 2^63) and its bad count t[6]. */
@@ -215,16 +227,12 @@ __host__ __device__ inline double fixed_total(const unsigned long long* t) {
   return neg ? -r : r;
 }
 
-/* Per-lane exact totals (rho in fm, rho * e in fe) -> r.totals -> last
- * block -> r.sums[0..1]. The block sums its lanes' 32-bit limbs (integer
- * sums, in any order) and its first 14 threads add them to the counters
- * with 64-bit atomics; the last block reads and clears the counters. The
- * totals are the same bits whichever waves and blocks added which values.
- * (One atomic per wave and limb, on counters sharing a line, cost the
- * mass/energy march 2-3%.) */
+/* Per-lane exact totals (rho in fm, rho * e in fe) -> the block's 14 words:
+ * the sums of its lanes' 32-bit limbs (integer sums, in any order) and of
+ * the bad marks, mass first. */
 template <int NT>
-__device__ void finish_fixed_sums(const FixSum& fm, const FixSum& fe, FkReduce r) {
-  __shared__ unsigned long long part[NT / kWave][14];
+__device__ void publish_limbs(const FixSum& fm, const FixSum& fe, FkReduce r) {
+  __shared__ unsigned long long part[NT / kWave][kTotalsWords];
   const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
   const FixSum* f[2] = {&fm, &fe};
 #pragma unroll
@@ -240,22 +248,38 @@ __device__ void finish_fixed_sums(const FixSum& fm, const FixSum& fe, FkReduce r
     }
   }
   __syncthreads();
-  if (threadIdx.x < 14) {
+  if (threadIdx.x < kTotalsWords) {
     unsigned long long v = 0;
     for (int b = 0; b < NT / kWave; ++b) v += part[b][threadIdx.x];
-    const int q = threadIdx.x / 7, k = threadIdx.x % 7;
-    if (v) atomicAdd(&r.totals[(8 * q + k) * kTotalsStride], v);
+    unsigned long long* p = (unsigned long long*)(r.partials + kTotalsOffset);
+    p[kTotalsWords * blockIdx.x + threadIdx.x] = v;
   }
-  if (!last_block_arrives(r.ticket)) return;
-  if (threadIdx.x == 0) {
-    for (int q = 0; q < 2; ++q) {
-      unsigned long long t[7];
-      for (int k = 0; k < 7; ++k)
-        t[k] = atomicExch(&r.totals[(8 * q + k) * kTotalsStride], 0ull);
-      r.sums[q] = fixed_total(t);
-    }
-    *r.ticket = 0u;
+}
+
+/* The totals of parts blocks' words -> r.sums[0..1], by one block. Thread
+ * t < 252 adds word t % 14 of every 18th block, so a wave reads consecutive
+ * words. The totals are the same bits whichever waves and blocks added
+ * which values. */
+template <int NT>
+__device__ void fold_limbs(const FkReduce& r, int parts) {
+  constexpr int kSlices = NT / kTotalsWords;
+  __shared__ unsigned long long s_sum[kSlices][kTotalsWords];
+  const unsigned long long* p = (const unsigned long long*)(r.partials + kTotalsOffset);
+  const int slice = threadIdx.x / kTotalsWords, word = threadIdx.x % kTotalsWords;
+  if (slice < kSlices) {
+    unsigned long long v = 0;
+#pragma unroll 4
+    for (int b = slice; b < parts; b += kSlices) v += p[kTotalsWords * b + word];
+    s_sum[slice][word] = v;
   }
+  __syncthreads();
+  if (threadIdx.x < kTotalsWords) {
+    unsigned long long v = 0;
+    for (int k = 0; k < kSlices; ++k) v += s_sum[k][threadIdx.x];
+    s_sum[0][threadIdx.x] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) r.sums[threadIdx.x] = fixed_total(&s_sum[0][7 * threadIdx.x]);
 }
 
 }  // namespace flowhip

@@ -59,31 +59,27 @@ typedef struct FkMesh32 {
   int pairs;   /* as in FkMesh (8-byte alignment) */
 } FkMesh32;
 
-/* Device scratch for the single-pass grid reductions. */
+/* Device scratch of a mesh's reductions and work queues. */
 typedef struct FkReduce {
-  double* partials;      /* fk_reduce_blocks() doubles */
-  unsigned int* ticket;  /* one counter, zero between launches */
-  double* dtp;           /* {dt, dt_h} */
+  double* partials;      /* fk_reduce_blocks() doubles: what the blocks of a
+                            launch leave for the launch that folds it */
+  double* dtp;           /* {dt, dt_h}, then the pair the march schedule's
+                            mass/energy kernel hands to the momentum kernel */
   double* sums;          /* {mass, energy, unclamped min dt, spare} */
-  int* status;           /* [0] NaN CFL candidates being counted, [1] the
-                            count of the last fk_timestep launch */
-  int max_blocks;
-  /* FK_MARCH_QUEUE_WORDS words holding the counters from which the waves
-   * of a march kernel claim work items; zero between launches (the last
-   * wave resets them). */
+  int* status;           /* [1] undefined CFL candidates of the last dt
+                            computation */
+  /* FK_MARCH_QUEUE_WORDS words: a set of counters for each stage of a march
+   * step, from which the waves of its kernel claim work items. A stage's
+   * set is zero when its kernel starts; each kernel zeroes the others. */
   unsigned int* queue;
-  /* FK_TOTALS_WORDS exact fixed-point accumulators of the mass/energy
-   * march's totals; zero between launches (the last block clears them). */
-  unsigned long long* totals;
   /* NULL, or a cell-layout array (nx * ny doubles) that the FP64
    * Lagrangian kernels fill with every interior CFL candidate. When set,
-   * those kernels leave the (dt, dt_h) update and the status count to a
-   * following fk_timestep_serial launch that reads the candidates. */
+   * the (dt, dt_h) update and the count are left to a following
+   * fk_timestep_serial launch that reads the candidates. */
   double* cfl;
 } FkReduce;
 
-#define FK_MARCH_QUEUE_WORDS 512
-#define FK_TOTALS_WORDS 256
+#define FK_MARCH_QUEUE_WORDS 768
 
 /* Number of doubles FkReduce.partials must hold. */
 int fk_reduce_blocks(void);
@@ -117,18 +113,23 @@ hipError_t fk_shock_heating(FkMesh m, const double* dtp, double* e,
                             const double* rho, const double* Qxx,
                             const double* Qyy, hipStream_t s);
 /* omp3/flow.c:77-105: grid minimum of the CFL candidates, seeded with
- * max_dt, then the (dt, dt_h) update written to r->dtp. One launch. */
+ * max_dt, then the (dt, dt_h) update written to r->dtp. Two launches: the
+ * candidates, then fk_finish_timestep's fold of the blocks' minima. */
 hipError_t fk_timestep(FkMesh m, const double* Qxx, const double* Qyy,
                        const double* rho, const double* e, FkReduce r,
                        double max_dt, int first_step, hipStream_t s);
+/* The folds of what `parts` blocks left in r.partials: the dt update from
+ * their minima, the totals (r.sums[0..1]) from their compensated sums. */
+hipError_t fk_finish_timestep(FkReduce r, int parts, double max_dt, int first_step,
+                              hipStream_t s);
+hipError_t fk_finish_sums(FkReduce r, int parts, hipStream_t s);
 /* omp3/flow.c:77-105 with the candidates folded as one OpenMP thread folds
  * them: every interior candidate in row-major order with min(a, b) = a < b ?
  * a : b from +inf (a NaN candidate makes the running value NaN and the next
  * candidate replaces it), then merged into max_dt by OpenMP's min combiner
  * out = in < out ? in : out; then the (dt, dt_h) update. Candidates come from
  * cfl (cell layout, as left by a Lagrangian kernel with FkReduce.cfl set),
- * or, with cfl NULL, are computed from e, Qxx, Qyy and rho; undefined
- * candidates are counted into r.status in the second case only. */
+ * or, with cfl NULL, are computed from e, Qxx, Qyy and rho. */
 hipError_t fk_timestep_serial(FkMesh m, const double* cfl, const double* Qxx,
                               const double* Qyy, const double* rho,
                               const double* e, FkReduce r, double max_dt,
@@ -184,7 +185,7 @@ hipError_t fk_conservation(FkMesh m, const double* rho, const double* e,
  * (dt, dt_h) in r.dtp; writes the momenta after the viscous step (mx1, my1,
  * interior faces), the velocities after it (u0, v0, with ghosts), the
  * energy after shock heating (e1, with ghosts), rho_old = rho, and the new
- * (dt, dt_h) into r.dtp. One launch. */
+ * (dt, dt_h) into r.dtp. */
 hipError_t fk_lagrangian(FkMesh m, const double* rho, const double* e,
                          const double* mom_x, const double* mom_y, double* mx1,
                          double* my1, double* u0, double* v0, double* e1,
@@ -216,18 +217,28 @@ hipError_t fk_advect_momentum_y(FkMesh m, int tt, const double* u1,
                                 const double* dtp, hipStream_t s);
 
 /* ---- row-marching forms (march.hip) ----
- * Same contracts as the fused kernels above; one wave marches a strip of
- * columns down chunks of chunk_rows rows. */
+ * One wave marches a strip of columns down chunks of chunk_rows rows. The
+ * arrays' contracts are those of the fused kernels above; a step's scalars
+ * go through the three kernels of a step, launched in this order on one
+ * stream with the same r:
+ *   fk_march_lagrangian reads the pair in r.dtp and leaves its blocks' CFL
+ *     minima in r.partials (*parts blocks);
+ *   fk_march_mass_energy folds the lag_parts blocks' minima into the new
+ *     pair (lag_parts 0: r.dtp holds it already) and leaves its blocks'
+ *     totals (*parts blocks);
+ *   fk_march_momentum folds the parts blocks' totals into r.sums and leaves
+ *     the new pair in r.dtp. */
 hipError_t fk_march_mass_energy(FkMesh m, int tt, const double* u0,
                                 const double* v0, const double* rho0,
                                 const double* e1, double* rho, double* e,
-                                double* F_x, double* F_y, FkReduce r,
+                                double* F_x, double* F_y, FkReduce r, double max_dt,
+                                int first_step, int lag_parts, int* parts,
                                 int chunk_rows, hipStream_t s);
 hipError_t fk_march_lagrangian(FkMesh m, const double* rho, const double* e,
                                const double* mom_x, const double* mom_y, double* mx1,
                                double* my1, double* u0, double* v0, double* e1,
-                               double* rho_old, FkReduce r, double max_dt,
-                               int first_step, int chunk_rows, hipStream_t s);
+                               double* rho_old, FkReduce r, double max_dt, int* parts,
+                               int chunk_rows, hipStream_t s);
 /* omp3/flow.c:557-775: both momentum directions in one row march (the y
  * direction reads the u the x direction has just computed in the same
  * wave); the result equals fk_march_momentum_x then _y. */
@@ -235,7 +246,7 @@ hipError_t fk_march_momentum(FkMesh m, int tt, const double* u0, const double* v
                              const double* F_x, const double* F_y, const double* rho,
                              const double* mx1, const double* my1, double* mom_x,
                              double* mom_y, double* u, double* v, FkReduce r,
-                             int chunk_rows, hipStream_t s);
+                             int parts, int chunk_rows, hipStream_t s);
 hipError_t fk_march_momentum_x(FkMesh m, int tt, const double* u0,
                                const double* v0, const double* F_x,
                                const double* F_y, const double* rho,
@@ -260,18 +271,19 @@ hipError_t fk_march_lagrangian_f32(FkMesh32 m, const float* rho, const float* e,
                                    const float* mom_x, const float* mom_y,
                                    float* mx1, float* my1, float* u0, float* v0,
                                    float* e1, float* rho_old, FkReduce r,
-                                   double max_dt, int first_step, int chunk_rows,
+                                   double max_dt, int* parts, int chunk_rows,
                                    hipStream_t s);
 hipError_t fk_march_mass_energy_f32(FkMesh32 m, int tt, const float* u0,
                                     const float* v0, const float* rho0,
                                     const float* e1, float* rho, float* e,
-                                    float* F_x, float* F_y, FkReduce r,
+                                    float* F_x, float* F_y, FkReduce r, double max_dt,
+                                    int first_step, int lag_parts, int* parts,
                                     int chunk_rows, hipStream_t s);
 hipError_t fk_march_momentum_f32(FkMesh32 m, int tt, const float* u0, const float* v0,
                                  const float* F_x, const float* F_y, const float* rho,
                                  const float* mx1, const float* my1, float* mom_x,
                                  float* mom_y, float* u, float* v, FkReduce r,
-                                 int chunk_rows, hipStream_t s);
+                                 int parts, int chunk_rows, hipStream_t s);
 hipError_t fk_march_momentum_x_f32(FkMesh32 m, int tt, const float* u0,
                                    const float* v0, const float* F_x,
                                    const float* F_y, const float* rho,
@@ -320,7 +332,7 @@ typedef struct FkEnsLaunch {
                               (they hold one value throughout) */
   int fused_momentum;      /* both momentum directions in one march */
   unsigned int* queue;     /* FK_MARCH_QUEUE_WORDS work-queue words, zero
-                              between launches (each kernel resets them) */
+                              between steps (the epilogue kernels zero them) */
   FkEnsPartials part;
   FkEnsHistory hist;
 } FkEnsLaunch;
@@ -340,7 +352,7 @@ hipError_t fk_ens_set_counter(int* counter, int value, hipStream_t s);
  * device address it looks up once per device; max_side is the largest
  * interior side those buffers serve, bytes the array's size. Every caller
  * on one device gets the same memory. fk_static_begin zeroes r's counter
- * words (ticket, status, queue, totals) and sets r.dtp = {dt, dt_h}. */
+ * words (status, queue) and sets r.dtp = {dt, dt_h}. */
 hipError_t fk_static_scratch(FkReduce* r, double** inv_edgedx, double** inv_edgedy,
                              int* max_side, size_t* bytes);
 hipError_t fk_static_begin(FkReduce r, double dt, double dt_h, hipStream_t s);
