@@ -168,7 +168,9 @@ FlowHipEnsemble* flowhip_ensemble_new(int ninst, const int* global_nx,
   E->ninst = ninst;
   E->fp32 = fp32 ? 1 : 0;
   E->esize = fp32 ? (int)sizeof(float) : (int)sizeof(double);
-  E->chunk_rows = 48;
+  double cells = 0.0;
+  for (int i = 0; i < ninst; ++i) cells += (double)global_nx[i] * (double)global_ny[i];
+  E->chunk_rows = fk_ens_default_rows(cells, E->fp32);
   E->order = ENS_ORDER_LARGEST;
   E->fused_momentum = 1;
   E->gnx = (int*)malloc(sizeof(int) * (size_t)ninst);
@@ -510,7 +512,7 @@ int flowhip_ensemble_run(FlowHipEnsemble* E, int niters, int tt0, int pre_timest
   return niters;
 }
 
-/* Try every chunk height in {16, 20, 24, 32, 48, 64}, work order (instance,
+/* Try every chunk height in {4, 8, 12, 16, 20, 24, 32}, work order (instance,
  * largest first, round robin) and momentum schedule (fused, x then y) for
  * trial_steps steps from the current state; keep the fastest and put the
  * state back. */
@@ -523,7 +525,7 @@ int flowhip_ensemble_autotune(FlowHipEnsemble* E, int trial_steps, int tt0,
   HIPCHECK(hipMemcpy(E->snap, E->pool, E->pool_bytes, hipMemcpyDeviceToDevice));
   HIPCHECK(hipMemcpy((char*)E->snap + E->pool_bytes, E->d_dtp,
                      sizeof(double) * 2 * (size_t)n, hipMemcpyDeviceToDevice));
-  const int rows[] = {16, 20, 24, 32, 48, 64};
+  const int rows[] = {4, 8, 12, 16, 20, 24, 32};
   double best = 1e300;
   int brow = E->chunk_rows, bord = E->order, bfm = E->fused_momentum;
   hipEvent_t a, b;

@@ -18,6 +18,8 @@
  * are appended to device history buffers at a device-side step counter,
  * so a step can be captured once in a hipGraph and replayed.
  */
+#include <cmath>
+
 #include "march.h"
 
 namespace flowhip {
@@ -58,13 +60,6 @@ __device__ __forceinline__ MarchList ens_list(const FkEnsInst& in, int H) {
   ml.nstrips = in.nstrips;
   ml.nchunks = in.nchunks;
   ml.nitems = in.nitems;
-  /* uniform chunks of H rows */
-  ml.G = 1;
-  ml.cpb = in.nchunks;
-  ml.H2 = H;
-  ml.k = 1;
-  ml.nsmall = 0;
-  ml.R = in.ny - 2 * kPad;
   return ml;
 }
 
@@ -414,6 +409,16 @@ using namespace flowhip;
 extern "C" {
 
 int fk_ens_strip_width(void) { return kEnsW; }
+
+/* The single-mesh rule for chunk heights (march.hip) on the cells of the whole
+ * ensemble, with one height for all stages (prologue 4.5 rows, at most the 20
+ * rows the autotuner picks for the 256-instance ensemble). */
+int fk_ens_default_rows(double cells, int fp32) {
+  const double slots =
+      (double)march_cus() * kMWaves * (fp32 ? kMarchMaxWaves<float> : kMarchMaxWaves<double>);
+  const int H = (int)(std::sqrt(4.5 * cells / (kEnsW * slots)) + 0.5);
+  return H < 4 ? 4 : H > 20 ? 20 : H;
+}
 
 hipError_t fk_ens_step(FkEnsLaunch L, int tt, int fp32, hipStream_t s) {
   if (L.chunk_rows < 4 || L.chunk_rows > kMaxChunkRows) return hipErrorInvalidValue;

@@ -82,47 +82,25 @@ constexpr int kLagPairWaves = sizeof(T) == 8 ? 2 : FLOWHIP_LAG_PAIR_WAVES;
 template <typename T>
 constexpr int kMassPairWaves = sizeof(T) == 8 ? 2 : FLOWHIP_MASS_PAIR_WAVES;
 
-/* The work items of a march kernel: strips of W columns by chunks of rows.
- * The interior rows are cut into G row bands (one per XCD band of the
- * item list, MarchQueue), each into units of H2 rows. A band's chunks are
- * k units tall (H = k * H2 rows) except its last `nsmall`, one unit each:
- * the waves claim tall chunks first, which re-read few prologue rows per
- * row marched, and finish on short ones, which keeps the band's tail short.
- * Every band has cpb chunk slots (a shorter band leaves its last slot
- * empty); items run strip-fastest within a chunk, band by band. Every chunk
- * but the mesh's first starts at least H2 rows above the south wall. With
- * G = 1, k = 1 and nsmall = 0 the chunks are uniform, H2 rows each. */
+/* The work items of a march kernel: strips of W columns by chunks of H rows
+ * (the last chunk may be shorter), strip-fastest. */
 struct MarchList {
-  int W, H;           /* strip width (output columns), tall chunk height (rows) */
+  int W, H;           /* strip width (output columns), chunk height (rows) */
   int nstrips, nchunks, nitems;
-  int G, cpb;         /* row bands, chunk slots per band */
-  int H2, k, nsmall;  /* unit rows, units per tall chunk, short chunks per band */
-  int R;              /* interior rows */
 };
 
-/* Columns and rows of one item; y0 == y1 for an empty slot. */
+/* Columns and rows of one item. */
 struct ItemBox {
   int x0, x1, y0, y1;
 };
 
-__device__ __forceinline__ ItemBox item_box(const MarchList& ml, int nx, int item) {
-  const int strip = item % ml.nstrips, slot = item / ml.nstrips;
-  const int g = slot / ml.cpb, c = slot - g * ml.cpb;
-  const int r0 = kPad + g * ml.R / ml.G, r1 = kPad + (g + 1) * ml.R / ml.G;
-  const int units = (r1 - r0 + ml.H2 - 1) / ml.H2;
-  const int ub = max(units - ml.nsmall, 0);           /* units in tall chunks */
-  const int nbig = (ub + ml.k - 1) / ml.k;
+__device__ __forceinline__ ItemBox item_box(const MarchList& ml, int nx, int ny, int item) {
+  const int chunk = item / ml.nstrips, strip = item - chunk * ml.nstrips;
   ItemBox b;
   b.x0 = kPad + strip * ml.W;
   b.x1 = min(b.x0 + ml.W, nx - kPad);
-  if (c < nbig) {
-    b.y0 = r0 + c * ml.k * ml.H2;
-    b.y1 = min(r0 + min((c + 1) * ml.k, ub) * ml.H2, r1);
-  } else {
-    const int u = ub + (c - nbig);
-    b.y0 = min(r0 + u * ml.H2, r1);
-    b.y1 = u < units ? min(b.y0 + ml.H2, r1) : b.y0;
-  }
+  b.y0 = kPad + chunk * ml.H;
+  b.y1 = min(b.y0 + ml.H, ny - kPad);
   return b;
 }
 
@@ -258,26 +236,13 @@ struct MarchBlockQueue : MarchQueue<true> {
   }
 };
 
-/* Items of a mesh: H2-row units in tall chunks of k units, the last nsmall
- * chunks of each of G row bands one unit each (G is lowered until every
- * band holds at least 4 units; k = 1, nsmall = 0 gives uniform chunks). */
-inline MarchList make_march(int nx, int ny, int W, int H2, int k = 1, int nsmall = 0,
-                            int G = 1) {
+/* Items of a mesh. */
+inline MarchList make_march(int nx, int ny, int W, int H) {
   MarchList m;
   m.W = W;
-  m.H2 = H2;
-  m.k = k;
-  m.nsmall = nsmall;
-  m.H = k * H2;
-  m.R = ny - 2 * kPad;
-  m.G = G;
-  while (m.G > 1 && m.R / m.G < 4 * H2) --m.G;
-  const int rmax = (m.R + m.G - 1) / m.G;
-  const int units = (rmax + H2 - 1) / H2;
-  const int ub = units > nsmall ? units - nsmall : 0;
-  m.cpb = (ub + k - 1) / k + (units < nsmall ? units : nsmall);
+  m.H = H;
   m.nstrips = (nx - 2 * kPad + W - 1) / W;
-  m.nchunks = m.G * m.cpb;
+  m.nchunks = (ny - 2 * kPad + H - 1) / H;
   m.nitems = m.nstrips * m.nchunks;
   return m;
 }
@@ -331,8 +296,8 @@ __device__ __forceinline__ bool item_xedge(const MarchList& ml, int nx, int item
  * other items, all but the mesh's outer ring of items, run the
  * straight-line interior form of their kernel. */
 __device__ __forceinline__ bool item_edge(const MarchList& ml, int nx, int ny, int item) {
-  const ItemBox b = item_box(ml, nx, item);
-  return item_xedge(ml, nx, item) || (b.y0 == kPad) || (b.y1 + 3 > ny - kPad);
+  const ItemBox b = item_box(ml, nx, ny, item);
+  return item_xedge(ml, nx, item) || (b.y0 < kPad + 3) || (b.y1 + 3 > ny - kPad);
 }
 
 /* ---- per-row geometry of a chunk held across the lanes ----
@@ -340,6 +305,11 @@ __device__ __forceinline__ bool item_edge(const MarchList& ml, int nx, int ny, i
  * with v_readlane (k is uniform), so the row loop issues no memory load for
  * geometry. Chunks are at most kMaxChunkRows rows. */
 constexpr int kMaxChunkRows = 120;
+/* Least height the rules choose: the x stage of the momentum march at a
+ * chunk that starts two rows above the south wall reads a ghost row as its
+ * mirror, and at one row above it the Lagrangian's first y face would be a
+ * ghost face (item_edge). */
+constexpr int kMinChunkRows = 2;
 
 __device__ __forceinline__ double lane_value(double v, int k) {
   const long long b = __double_as_longlong(v);
@@ -632,7 +602,6 @@ __device__ __forceinline__ void mass_xy_box(const MGeo<T>& g, const MMassIO<T>& 
   (void)dt;
   (void)sx;
   const int x0 = box.x0, x1 = box.x1, y0 = box.y0, y1 = box.y1;
-  if (y0 >= y1) return;
   const bool edge = EDGE && ((x0 == kPad) || (x1 + 3 > nx - kPad) || (y0 == kPad) ||
                              (y1 + 3 > ny - kPad));
   const int q = x0 - 2 + lane;
@@ -761,7 +730,7 @@ template <typename T, bool P2, bool EDGE = true, bool UNI = false, typename Acc 
 __device__ __forceinline__ void mass_xy_item(const MGeo<T>& g, const MMassIO<T>& io, T dt,
                                              T dt_h, const MarchList& ml, int item, int lane,
                                              Acc& ms, Acc& es) {
-  mass_xy_box<T, P2, EDGE, UNI, Acc>(g, io, dt, dt_h, item_box(ml, g.nx, item), lane, ms, es);
+  mass_xy_box<T, P2, EDGE, UNI, Acc>(g, io, dt, dt_h, item_box(ml, g.nx, g.ny, item), lane, ms, es);
 }
 
 /* The x-first mass/energy march of an interior item, two columns per lane
@@ -772,7 +741,6 @@ __device__ __forceinline__ void mass_xy_pair(const MGeo<T>& g, const MMassIO<T>&
                                              Acc& es) {
   const int nx = g.nx, ny = g.ny, sx = nx + 1;
   const int x0 = box.x0, x1 = box.x1, y0 = box.y0, y1 = box.y1;
-  if (y0 >= y1) return;
   const int qb = x0 - 2 + 2 * lane; /* the lane's first column */
   /* x0 and the strip width are even, so a lane owns both columns or neither */
   const bool own = qb >= x0 && qb < x1;
@@ -927,7 +895,7 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_mass_xy(
   for (int item = mq.first(); item < mq.end; item = mq.next()) {
     ItemSum<T> ms{0.0, 0.0}, es{0.0, 0.0};
     if constexpr (PAIR) {
-      const ItemBox b = item_box(ml, g.nx, item);
+      const ItemBox b = item_box(ml, g.nx, g.ny, item);
       if (item_edge(ml, g.nx, g.ny, item)) {
         for (int sx0 = b.x0; sx0 < b.x1; sx0 += kMassW) {
           const ItemBox sb{sx0, min(sx0 + kMassW, b.x1), b.y0, b.y1};
@@ -963,7 +931,6 @@ __device__ __forceinline__ void mass_yx_box(const MGeo<T>& g, const MMassIO<T>& 
   (void)dt;
   (void)sx;
   const int x0 = box.x0, x1 = box.x1, y0 = box.y0, y1 = box.y1;
-  if (y0 >= y1) return;
   const bool edge = EDGE && ((x0 == kPad) || (x1 + 3 > nx - kPad) || (y0 == kPad) ||
                              (y1 + 3 > ny - kPad));
   const int q = x0 - 2 + lane;
@@ -1073,7 +1040,7 @@ template <typename T, bool P2, bool EDGE = true, bool UNI = false, typename Acc 
 __device__ __forceinline__ void mass_yx_item(const MGeo<T>& g, const MMassIO<T>& io, T dt,
                                              T dt_h, const MarchList& ml, int item, int lane,
                                              Acc& ms, Acc& es) {
-  mass_yx_box<T, P2, EDGE, UNI, Acc>(g, io, dt, dt_h, item_box(ml, g.nx, item), lane, ms, es);
+  mass_yx_box<T, P2, EDGE, UNI, Acc>(g, io, dt, dt_h, item_box(ml, g.nx, g.ny, item), lane, ms, es);
 }
 
 /* The y-first mass/energy march of an interior item, two columns per lane
@@ -1084,7 +1051,6 @@ __device__ __forceinline__ void mass_yx_pair(const MGeo<T>& g, const MMassIO<T>&
                                              Acc& es) {
   const int nx = g.nx, ny = g.ny, sx = nx + 1;
   const int x0 = box.x0, x1 = box.x1, y0 = box.y0, y1 = box.y1;
-  if (y0 >= y1) return;
   const int qb = x0 - 2 + 2 * lane;
   const bool own = qb >= x0 && qb < x1;
   bool face[2];
@@ -1241,7 +1207,7 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_mass_yx(
   for (int item = mq.first(); item < mq.end; item = mq.next()) {
     ItemSum<T> ms{0.0, 0.0}, es{0.0, 0.0};
     if constexpr (PAIR) {
-      const ItemBox b = item_box(ml, g.nx, item);
+      const ItemBox b = item_box(ml, g.nx, g.ny, item);
       if (item_edge(ml, g.nx, g.ny, item)) {
         for (int sx0 = b.x0; sx0 < b.x1; sx0 += kMassW) {
           const ItemBox sb{sx0, min(sx0 + kMassW, b.x1), b.y0, b.y1};
@@ -1311,9 +1277,8 @@ __device__ __forceinline__ void momx_xy_item(const MGeo<T>& g, const MMomIO<T>& 
   const int nx = g.nx, ny = g.ny, sx = nx + 1;
   (void)dt;
   (void)sx;
-  const ItemBox box = item_box(ml, nx, item);
+  const ItemBox box = item_box(ml, nx, ny, item);
   const int x0 = box.x0, x1 = box.x1, y0 = box.y0, y1 = box.y1;
-  if (y0 >= y1) return;
   const bool edge = (x0 == kPad) || (x1 + 3 > nx - kPad) || (y0 == kPad) ||
                     (y1 + 3 > ny - kPad);
   const bool xedge = (x0 - 3 < kPad) || (x1 + 3 > nx - kPad);
@@ -1420,9 +1385,8 @@ __device__ __forceinline__ void momx_yx_item(const MGeo<T>& g, const MMomIO<T>& 
   const int nx = g.nx, ny = g.ny, sx = nx + 1;
   (void)dt;
   (void)sx;
-  const ItemBox box = item_box(ml, nx, item);
+  const ItemBox box = item_box(ml, nx, ny, item);
   const int x0 = box.x0, x1 = box.x1, y0 = box.y0, y1 = box.y1;
-  if (y0 >= y1) return;
   const bool edge = (x0 == kPad) || (x1 + 3 > nx - kPad) || (y0 == kPad) ||
                     (y1 + 3 > ny - kPad);
   const bool xedge = (x0 - 3 < kPad) || (x1 + 3 > nx - kPad);
@@ -1517,9 +1481,8 @@ __device__ __forceinline__ void momy_xy_item(const MGeo<T>& g, const MMomIO<T>& 
   const int nx = g.nx, ny = g.ny, sx = nx + 1;
   (void)dt;
   (void)sx;
-  const ItemBox box = item_box(ml, nx, item);
+  const ItemBox box = item_box(ml, nx, ny, item);
   const int x0 = box.x0, x1 = box.x1, y0 = box.y0, y1 = box.y1;
-  if (y0 >= y1) return;
   const bool edge = (x0 == kPad) || (x1 + 3 > nx - kPad) || (y0 == kPad) ||
                     (y1 + 3 > ny - kPad);
   const int gend = (y1 == ny - kPad) ? y1 + 1 : y1;
@@ -1660,9 +1623,8 @@ __device__ __forceinline__ void momy_yx_item(const MGeo<T>& g, const MMomIO<T>& 
   const int nx = g.nx, ny = g.ny, sx = nx + 1;
   (void)dt;
   (void)sx;
-  const ItemBox box = item_box(ml, nx, item);
+  const ItemBox box = item_box(ml, nx, ny, item);
   const int x0 = box.x0, x1 = box.x1, y0 = box.y0, y1 = box.y1;
-  if (y0 >= y1) return;
   const bool edge = (x0 == kPad) || (x1 + 3 > nx - kPad) || (y0 == kPad) ||
                     (y1 + 3 > ny - kPad);
   const bool xedge = (x0 - 3 < kPad) || (x1 + 3 > nx - kPad);
@@ -1796,7 +1758,6 @@ __device__ __forceinline__ void lagrangian_box(const MGeo<T>& g, const MLagIO<T>
   (void)dt;
   (void)sx;
   const int x0 = box.x0, x1 = box.x1, y0 = box.y0, y1 = box.y1;
-  if (y0 >= y1) return;
   const bool edge = EDGE && ((x0 == kPad) || (x1 + 3 > nx - kPad) || (y0 == kPad) ||
                              (y1 + 3 > ny - kPad));
   /* strips within three columns of a wall hold ghost lanes; XE fixes that at
@@ -2019,7 +1980,7 @@ template <typename T, bool P2, int XE = -1, bool EDGE = true, bool UNI = false>
 __device__ __forceinline__ void lagrangian_item(const MGeo<T>& g, const MLagIO<T>& io, T dt,
                                                 T dt_h, const MarchList& ml, int item,
                                                 int lane, double& local_min, int& nan_count) {
-  lagrangian_box<T, P2, XE, EDGE, UNI>(g, io, dt, dt_h, item_box(ml, g.nx, item), lane,
+  lagrangian_box<T, P2, XE, EDGE, UNI>(g, io, dt, dt_h, item_box(ml, g.nx, g.ny, item), lane,
                                        local_min, nan_count);
 }
 
@@ -2040,7 +2001,6 @@ __device__ __forceinline__ void lagrangian_pair(const MGeo<T>& g, const MLagIO<T
   using P = T[2];
   const int nx = g.nx, ny = g.ny, sx = nx + 1;
   const int x0 = box.x0, x1 = box.x1, y0 = box.y0, y1 = box.y1;
-  if (y0 >= y1) return;
   const int qb = x0 - 4 + 2 * lane;
   const bool own = qb >= x0 && qb < x1; /* both columns: x0 and the width even */
   T edx_q[2], cdx_q[2], cdx_qm[2], iedx_q[2], rcdx_q[2];
@@ -2273,7 +2233,7 @@ void k_march_lagrangian(MGeo<T> g, MLagIO<T> io, FkReduce red, double max_dt, Ma
     if constexpr (PAIR) {
       /* interior items two columns per lane; edge items in one-column
        * sub-strips */
-      const ItemBox b = item_box(ml, g.nx, item);
+      const ItemBox b = item_box(ml, g.nx, g.ny, item);
       if (!item_edge(ml, g.nx, g.ny, item)) {
         lagrangian_pair<T, P2, UNI>(g, io, dt, dt_h, b, lane, local_min, nan_count);
       } else {
@@ -2331,9 +2291,8 @@ __device__ __forceinline__ void momxy_xy_item(const MGeo<T>& g, const MMom2IO<T>
                                               int item, int lane) {
   const int nx = g.nx, ny = g.ny, sx = nx + 1;
   (void)dt;
-  const ItemBox box = item_box(ml, nx, item);
+  const ItemBox box = item_box(ml, nx, ny, item);
   const int x0 = box.x0, x1 = box.x1, y0 = box.y0, y1 = box.y1;
-  if (y0 >= y1) return;
   const bool edge = EDGE && ((x0 == kPad) || (x1 + 3 > nx - kPad) || (y0 == kPad) ||
                              (y1 + 3 > ny - kPad));
   /* strips within three columns of a wall hold ghost lanes; XE fixes that at
@@ -2528,9 +2487,8 @@ __device__ __forceinline__ void momxy_yx_item(const MGeo<T>& g, const MMom2IO<T>
                                               int item, int lane) {
   const int nx = g.nx, ny = g.ny, sx = nx + 1;
   (void)dt;
-  const ItemBox box = item_box(ml, nx, item);
+  const ItemBox box = item_box(ml, nx, ny, item);
   const int x0 = box.x0, x1 = box.x1, y0 = box.y0, y1 = box.y1;
-  if (y0 >= y1) return;
   const bool edge = EDGE && ((x0 == kPad) || (x1 + 3 > nx - kPad) || (y0 == kPad) ||
                              (y1 + 3 > ny - kPad));
   /* strips within three columns of a wall hold ghost lanes; XE fixes that at
@@ -2724,13 +2682,8 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_momxy_yx(
   }
 }
 
-/* Persistent grid of a march kernel: as many blocks as stay resident on the
- * device (per_cu per CU, from the occupancy query on first use, at most
- * max_per_cu when that is positive), and no more than give every band a wave
- * for each of its items (a grid of nitems / kMWaves blocks left some bands an
- * item short of waves, and the launch took two rounds of items for one). */
-template <typename K>
-int march_grid(K kernel, int& per_cu, int nitems, int max_per_cu = 0) {
+/* compute units of the device, asked for once */
+inline int march_cus() {
   static int cus = 0;
   if (cus == 0) {
     int dev = 0;
@@ -2741,6 +2694,17 @@ int march_grid(K kernel, int& per_cu, int nitems, int max_per_cu = 0) {
     else
       cus = p.multiProcessorCount;
   }
+  return cus;
+}
+
+/* Persistent grid of a march kernel: as many blocks as stay resident on the
+ * device (per_cu per CU, from the occupancy query on first use, at most
+ * max_per_cu when that is positive), and no more than give every band a wave
+ * for each of its items (a grid of nitems / kMWaves blocks left some bands an
+ * item short of waves, and the launch took two rounds of items for one). */
+template <typename K>
+int march_grid(K kernel, int& per_cu, int nitems, int max_per_cu = 0) {
+  const int cus = march_cus();
   if (per_cu == 0 &&
       (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kMNT, 0) !=
            hipSuccess ||

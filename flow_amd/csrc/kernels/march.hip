@@ -2,99 +2,75 @@
  * march.hip -- launchers of the row-marching kernels on one mesh (FP64 and
  * the FP32-state form). The kernels are in march.h.
  */
+#include <cmath>
+
 #include "march.h"
 
 namespace flowhip {
 
-/* Chunking of a march kernel when no chunk height is given (chunk_rows 0):
- * units of H2 rows, chunks of k units, and nsmall one-unit chunks at the end
- * of each of the 8 XCD row bands (MarchList). Measured on MI355X at 8192^2,
- * uniform chunks (k = 1, nsmall = 0) of 24 / 20 / 16 rows (Lagrangian /
- * mass-energy / momentum; 24 / 16 / 16 in FP32; with two columns per lane
- * 12 / 12 for the FP64 Lagrangian and mass/energy marches, 10 / 10 in
- * FP32) are fastest (FP32 momentum: 16 rows 2.8% faster than 20 once the
- * last row of a chunk loads nothing, 12 and 14 the same as 16): tapering from
- * tall chunks (48-80 rows) down to 12-24-row ones cut the re-read prologue
- * rows but made the Lagrangian and mass/energy marches 5-10% slower. An
- * explicit chunk_rows > 0 gives uniform chunks of that height. Every
- * chunking gives bitwise the same result. */
-struct Taper {
-  int H2, k, nsmall;
+/* Chunk height of a march kernel when none is given. An item costs its H rows
+ * and about p more (prologue rows, first loads); C cells in strips of W
+ * columns on S waves then take (C / (W H S)) (H + p) row times, and the last
+ * items to finish leave the GPU partly idle for about H + p more, which is
+ * least at H = sqrt(p C / (W S)). So the height follows the square root of
+ * the mesh's cells, up to the height measured fastest at 8192^2, beyond which
+ * the rows in flight leave the last-level cache. p is fitted per kernel to
+ * sweeps of 2 to 24 rows at 64^2, 300x200, 512^2, 1000^2, 3000x150, 1536^2,
+ * 2048^2, 3001x2999 and 4096^2. Measured on MI355X (us a step, FP64; FP32),
+ * fixed heights of 24 / 20 / 16 rows (24 / 16 / 16) before and this rule
+ * after: 64^2 168 -> 64; 138 -> 52, 512^2 180 -> 83; 144 -> 60, 1000^2 197
+ * -> 130; 156 -> 90, 3000x150 195 -> 96; 156 -> 72, 2048^2 323 -> 323; 191 ->
+ * 166, 3001x2999 and up within 2%. */
+struct Rows {
+  double p;  /* prologue, in rows */
+  int most;  /* height on large meshes */
 };
-#ifndef FLOWHIP_TAPER_LAG
-#define FLOWHIP_TAPER_LAG 24, 1, 0
-#endif
-#ifndef FLOWHIP_TAPER_MASS
-#define FLOWHIP_TAPER_MASS 20, 1, 0
-#endif
-#ifndef FLOWHIP_TAPER_MOM
-#define FLOWHIP_TAPER_MOM 16, 1, 0
-#endif
-#ifndef FLOWHIP_TAPER_LAG32
-#define FLOWHIP_TAPER_LAG32 24, 1, 0
-#endif
-#ifndef FLOWHIP_TAPER_MASS32
-#define FLOWHIP_TAPER_MASS32 16, 1, 0
-#endif
-#ifndef FLOWHIP_TAPER_MOM32
-#define FLOWHIP_TAPER_MOM32 16, 1, 0
-#endif
-/* the FP32 mass/energy march with two columns per lane (three waves per
- * SIMD): 10 rows (measured 8 to 32; 14 rows +0.3%, 20 +3%) */
-#ifndef FLOWHIP_TAPER_MASS32P
-#define FLOWHIP_TAPER_MASS32P 10, 1, 0
-#endif
-/* the FP32 Lagrangian march with two columns per lane (three waves per
- * SIMD): 10 rows (measured 4 to 24; 12 rows +0.5%, 16 +4%, 20 +5%) */
-#ifndef FLOWHIP_TAPER_LAG32P
-#define FLOWHIP_TAPER_LAG32P 10, 1, 0
-#endif
-/* the FP64 Lagrangian and mass/energy marches with two columns per lane
- * (two waves per SIMD): 12 rows each (measured 8 to 24; 8 rows +2-5%,
- * 24 +3%, 10 to 20 within 1%) */
-#ifndef FLOWHIP_TAPER_LAG64P
-#define FLOWHIP_TAPER_LAG64P 12, 1, 0
-#endif
-#ifndef FLOWHIP_TAPER_MASS64P
-#define FLOWHIP_TAPER_MASS64P 12, 1, 0
-#endif
 enum { kKLag = 0, kKMass = 1, kKMom = 2 };
 template <typename T>
-constexpr Taper taper_of(int kernel) {
-  return sizeof(T) == 8 ? (kernel == kKLag    ? Taper{FLOWHIP_TAPER_LAG}
-                           : kernel == kKMass ? Taper{FLOWHIP_TAPER_MASS}
-                                              : Taper{FLOWHIP_TAPER_MOM})
-                        : (kernel == kKLag    ? Taper{FLOWHIP_TAPER_LAG32}
-                           : kernel == kKMass ? Taper{FLOWHIP_TAPER_MASS32}
-                                              : Taper{FLOWHIP_TAPER_MOM32});
+constexpr Rows rows_of(int kernel) {
+  return sizeof(T) == 8 ? (kernel == kKLag    ? Rows{2.9, 24}
+                           : kernel == kKMass ? Rows{5.7, 20}
+                                              : Rows{6.2, 16})
+                        : (kernel == kKLag    ? Rows{2.1, 24}
+                           : kernel == kKMass ? Rows{8.5, 16}
+                                              : Rows{5.2, 16});
 }
 
-inline MarchList march_items(int nx, int ny, int W, int chunk_rows, Taper t) {
+/* the marches with two columns per lane (12 rows in FP64, measured 8 to 24; 10
+ * in FP32, measured 4 to 24) run on large meshes, or where a caller asks */
+template <typename T>
+constexpr Rows pair_rows() {
+  return sizeof(T) == 8 ? Rows{2.9, 12} : Rows{2.1, 10};
+}
+
+inline MarchList march_items(int nx, int ny, int W, int chunk_rows, Rows r, int waves_per_simd,
+                             int least = kMinChunkRows) {
   if (chunk_rows > 0)
     return make_march(nx, ny, W, chunk_rows < kMaxChunkRows ? chunk_rows : kMaxChunkRows);
-  const int k = t.k * t.H2 <= kMaxChunkRows ? t.k : kMaxChunkRows / t.H2;
-  return make_march(nx, ny, W, t.H2, k, t.nsmall, kMarchBands);
+  const double cells = (double)(nx - 2 * kPad) * (ny - 2 * kPad);
+  const double slots = (double)march_cus() * kMWaves * waves_per_simd;
+  const int H = (int)(std::sqrt(r.p * cells / (W * slots)) + 0.5);
+  return make_march(nx, ny, W, H < least ? least : H > r.most ? r.most : H);
 }
 
 template <typename T, bool P2, bool UNI, bool PAIR = false>
 hipError_t launch_march_mass_p(MGeo<T> g, MMassIO<T> io, int tt, FkReduce r, MarchStep st,
                                int* parts, int chunk_rows, hipStream_t s) {
-  const MarchList ml = march_items(
-      g.nx, g.ny, PAIR ? kMassW2 : kMassW, chunk_rows,
-      PAIR ? (sizeof(T) == 8 ? Taper{FLOWHIP_TAPER_MASS64P} : Taper{FLOWHIP_TAPER_MASS32P})
-           : taper_of<T>(kKMass));
+  constexpr int kWaves = PAIR ? kMassPairWaves<T> : kMarchMaxWaves<T>;
+  const MarchList ml = march_items(g.nx, g.ny, PAIR ? kMassW2 : kMassW, chunk_rows,
+                                   PAIR ? pair_rows<T>() : rows_of<T>(kKMass), kWaves);
   if (ml.nitems < 1 || !r.queue) return hipErrorInvalidValue;
   if (tt % 2 == 0) {
     static int per_cu = 0;
     const int grid = march_grid(k_march_mass_xy<T, P2, UNI, PAIR>, per_cu, ml.nitems,
-                                PAIR ? kMassPairWaves<T> : kMarchMaxWaves<T>);
+                                kWaves);
     hipLaunchKernelGGL((k_march_mass_xy<T, P2, UNI, PAIR>), dim3(grid), dim3(kMNT), 0, s,
                        g, io, r, st, ml);
     *parts = grid;
   } else {
     static int per_cu = 0;
     const int grid = march_grid(k_march_mass_yx<T, P2, UNI, PAIR>, per_cu, ml.nitems,
-                                PAIR ? kMassPairWaves<T> : kMarchMaxWaves<T>);
+                                kWaves);
     hipLaunchKernelGGL((k_march_mass_yx<T, P2, UNI, PAIR>), dim3(grid), dim3(kMNT), 0, s,
                        g, io, r, st, ml);
     *parts = grid;
@@ -124,14 +100,13 @@ inline bool pairs_fit(const MGeo<T>& g, const MMassIO<T>& io) {
 template <typename T, bool P2, bool UNI, bool PAIR = false>
 hipError_t launch_march_lagrangian_p(MGeo<T> g, MLagIO<T> io, FkReduce r, double max_dt,
                                      int* parts, int chunk_rows, hipStream_t s) {
-  const MarchList ml = march_items(
-      g.nx, g.ny, PAIR ? kLagW2 : kLagW, chunk_rows,
-      PAIR ? (sizeof(T) == 8 ? Taper{FLOWHIP_TAPER_LAG64P} : Taper{FLOWHIP_TAPER_LAG32P})
-           : taper_of<T>(kKLag));
+  constexpr int kWaves = PAIR ? kLagPairWaves<T> : kLagMaxWaves<T>;
+  const MarchList ml = march_items(g.nx, g.ny, PAIR ? kLagW2 : kLagW, chunk_rows,
+                                   PAIR ? pair_rows<T>() : rows_of<T>(kKLag), kWaves);
   if (ml.nitems < 1 || !r.queue) return hipErrorInvalidValue;
   static int per_cu = 0;
   const int grid = march_grid(k_march_lagrangian<T, P2, UNI, PAIR>, per_cu, ml.nitems,
-                              PAIR ? kLagPairWaves<T> : kLagMaxWaves<T>);
+                              kWaves);
   hipLaunchKernelGGL((k_march_lagrangian<T, P2, UNI, PAIR>), dim3(grid), dim3(kMNT), 0, s,
                      g, io, r, max_dt, ml);
   *parts = grid;
@@ -160,7 +135,7 @@ hipError_t launch_march_momentum_p(MGeo<T> g, MMomIO<T> io, int tt, int ydir,
   const bool odd = (tt % 2) != 0;
   const MarchList ml =
       march_items(g.nx, g.ny, (!ydir && !odd) ? kMomXW : kMomW, chunk_rows,
-                  taper_of<T>(kKMom));
+                  rows_of<T>(kKMom), kMarchMaxWaves<T>, 4);
   if (ml.nitems < 1) return hipErrorInvalidValue;
   if (!ydir && odd) {
     static int per_cu = 0;
@@ -189,7 +164,8 @@ constexpr int kMomXYW = kWave - 5;
 template <typename T, bool P2, bool UNI>
 hipError_t launch_march_momxy_p(MGeo<T> g, MMom2IO<T> io, int tt, FkReduce r, int parts,
                                 int chunk_rows, hipStream_t s) {
-  const MarchList ml = march_items(g.nx, g.ny, kMomXYW, chunk_rows, taper_of<T>(kKMom));
+  const MarchList ml = march_items(g.nx, g.ny, kMomXYW, chunk_rows, rows_of<T>(kKMom),
+                                   kMarchMaxWaves<T>);
   if (ml.nitems < 1 || !r.queue) return hipErrorInvalidValue;
   /* one block more, for the step's epilogue */
   if (tt % 2) {

@@ -42,11 +42,12 @@ typedef struct FkMesh {
   int pairs;
 } FkMesh;
 
-/* Interior cells from which the two-column marches are the faster form
- * (measured on MI355X: slower at 1024^2, where the mesh does not fill the
- * GPU and a two-column item is the longer critical path; faster from
- * 2048^2) */
-#define FK_PAIR_MIN_CELLS (2048L * 2048L)
+/* Interior cells from which the two-column marches are the faster form.
+ * Measured on MI355X, two columns / one column at their best heights (us a
+ * step): 2048^2 364 / 320 FP64 and 191 / 166 FP32, 4096^2 975 / 955 and 577 /
+ * 537, 6144^2 2350 / 2360 and 1140 / 1150, 8192^2 3300 / 3390 and 1730 /
+ * 1800. */
+#define FK_PAIR_MIN_CELLS (6144L * 6144L)
 
 /* Geometry of the FP32-state precision form: the same arrays rounded to
  * FP32 (the reciprocals are rounded from the FP64 reciprocals). */
@@ -339,6 +340,8 @@ typedef struct FkEnsLaunch {
 
 /* Strip width of the ensemble work items. */
 int fk_ens_strip_width(void);
+/* Chunk height of an ensemble of so many interior cells, all instances. */
+int fk_ens_default_rows(double cells, int fp32);
 /* One step (omp3/flow.c:10-52) of every instance: Lagrangian stage, dt,
  * mass/energy advection, totals, x and y momentum, counter advance. */
 hipError_t fk_ens_step(FkEnsLaunch L, int tt, int fp32, hipStream_t s);
