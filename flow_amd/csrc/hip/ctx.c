@@ -77,12 +77,11 @@ FlowHipCtx* flowhip_ctx(Mesh* mesh) {
   HIPCHECK(hipMemset(h->red.sums, 0, sizeof(double) * 4));
   HIPCHECK(hipMemset(h->red.status, 0, sizeof(int) * 4));
   HIPCHECK(hipMemset(h->red.queue, 0, sizeof(unsigned int) * FK_MARCH_QUEUE_WORDS));
-  HIPCHECK(hipHostMalloc((void**)&h->h_stage, sizeof(double) * 8,
-                         hipHostMallocDefault));
-  HIPCHECK(hipHostMalloc((void**)&h->h_status, sizeof(int) * 4,
-                         hipHostMallocDefault));
-  memset(h->h_stage, 0, sizeof(double) * 8);
-  memset(h->h_status, 0, sizeof(int) * 4);
+  const size_t mail = sizeof(double) * FK_MAIL_WORDS * FLOWHIP_AHEAD;
+  HIPCHECK(hipHostMalloc((void**)&h->h_stage, sizeof(double) * 2, hipHostMallocDefault));
+  HIPCHECK(hipHostMalloc((void**)&h->mail, mail, hipHostMallocDefault));
+  memset(h->mail, 0, mail);
+  flowhip_post_to(h, 0);
   h->schedule = FLOWHIP_MARCH;
   h->march_rows = 0; /* each march kernel's own chunk height */
   schedule_from_env(h);
@@ -130,10 +129,42 @@ void flowhip_ctx_destroy(Mesh* mesh) {
   hipFree(h->red.status);
   hipFree(h->red.queue);
   hipHostFree(h->h_stage);
-  hipHostFree(h->h_status);
+  hipHostFree(h->mail);
   hipStreamDestroy(h->stream);
   free(h);
   mesh->hip = NULL;
+}
+
+void flowhip_push_pair(FlowHipCtx* h, const Mesh* mesh) {
+  const double want[2] = {mesh->dt, mesh->dt_h};
+  if (h->pair_known && memcmp(h->pair, want, sizeof(want)) == 0) return;
+  memcpy(h->h_stage, want, sizeof(want));
+  HIPCHECK(hipMemcpyAsync(h->red.dtp, h->h_stage, sizeof(want), hipMemcpyHostToDevice,
+                          h->stream));
+  memcpy(h->pair, want, sizeof(want));
+  h->pair_known = 1;
+}
+
+void flowhip_post_to(FlowHipCtx* h, int slot) {
+  h->red.mail = h->mail + (size_t)slot * FK_MAIL_WORDS;
+}
+
+void flowhip_wait(FlowHipCtx* h) {
+  HIPCHECK(hipStreamSynchronize(h->stream));
+  flowhip_timer_collect(h);
+}
+
+void flowhip_take_pair(FlowHipCtx* h, Mesh* mesh, int slot, const char* what) {
+  const double* m = h->mail + (size_t)slot * FK_MAIL_WORDS;
+  mesh->dt = h->pair[0] = m[0];
+  mesh->dt_h = h->pair[1] = m[1];
+  h->pair_known = 1;
+  h->undefined = (int)m[4];
+  if (!isfinite(mesh->dt) || !(mesh->dt > 0.0) || !isfinite(mesh->dt_h))
+    TERMINATE("%s: non-finite or non-positive timestep "
+              "(dt=%.12e dt_h=%.12e, %d undefined CFL candidates): the "
+              "state has diverged",
+              what, mesh->dt, mesh->dt_h, h->undefined);
 }
 
 /* Whether every value is a power of two with |exponent| <= emax. */
@@ -249,7 +280,7 @@ int flowhip_set_cfl_rule(Mesh* mesh, int rule) {
 
 int flowhip_get_cfl_rule(Mesh* mesh) { return flowhip_ctx(mesh)->cfl_rule; }
 
-int flowhip_undefined_candidates(Mesh* mesh) { return flowhip_ctx(mesh)->h_status[1]; }
+int flowhip_undefined_candidates(Mesh* mesh) { return flowhip_ctx(mesh)->undefined; }
 
 static int timer_index(FlowHipCtx* h, const char* name) {
   for (int k = 0; k < h->ntimers; ++k)

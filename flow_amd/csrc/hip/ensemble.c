@@ -37,6 +37,9 @@ struct FlowHipEnsemble {
   void* geo;           /* geometry of all instances */
   double* d_dtp;       /* 2 per instance */
   double* h_dtp;       /* pinned */
+  double* set_dtp;     /* pinned: pairs set by the caller, on their way */
+  char* is_set;        /* per instance: set_dtp holds a pair to upload */
+  int any_set;
   int* d_work;
   int nwork;
   int chunk_rows, order;
@@ -55,6 +58,23 @@ struct FlowHipEnsemble {
 };
 
 static size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
+
+/* The pairs that flowhip_ensemble_set_dt left, uploaded in runs of
+ * neighbouring instances (one copy when all were set). */
+static void ens_push_dt(FlowHipEnsemble* E) {
+  if (!E->any_set) return;
+  for (int i = 0; i < E->ninst; ++i) {
+    if (!E->is_set[i]) continue;
+    int j = i;
+    while (j < E->ninst && E->is_set[j]) E->is_set[j++] = 0;
+    HIPCHECK(hipMemcpyAsync(E->d_dtp + 2 * i, E->set_dtp + 2 * i,
+                            2 * sizeof(double) * (size_t)(j - i), hipMemcpyHostToDevice,
+                            E->stream));
+    i = j;
+  }
+  HIPCHECK(hipStreamSynchronize(E->stream));
+  E->any_set = 0;
+}
 
 static void ens_drop_graphs(FlowHipEnsemble* E) {
   for (int k = 0; k < 2; ++k) {
@@ -202,6 +222,10 @@ FlowHipEnsemble* flowhip_ensemble_new(int ninst, const int* global_nx,
   HIPCHECK(hipMalloc((void**)&E->d_dtp, sizeof(double) * 2 * (size_t)ninst));
   HIPCHECK(hipHostMalloc((void**)&E->h_dtp, sizeof(double) * 2 * (size_t)ninst,
                          hipHostMallocDefault));
+  HIPCHECK(hipHostMalloc((void**)&E->set_dtp, sizeof(double) * 2 * (size_t)ninst,
+                         hipHostMallocDefault));
+  E->is_set = (char*)calloc((size_t)ninst, 1);
+  if (!E->is_set) TERMINATE("ensemble: out of host memory");
 
   /* geometry: arch's uniform spacing (width / global_nx for every entry),
    * its reciprocals by a correctly rounded division, FP32 copies if asked */
@@ -295,6 +319,8 @@ void flowhip_ensemble_delete(FlowHipEnsemble* E) {
   HIPCHECK(hipFree(E->geo));
   HIPCHECK(hipFree(E->d_dtp));
   HIPCHECK(hipHostFree(E->h_dtp));
+  HIPCHECK(hipHostFree(E->set_dtp));
+  free(E->is_set);
   HIPCHECK(hipFree(E->d_work));
   HIPCHECK(hipFree(E->d_insts));
   HIPCHECK(hipFree(E->part.min));
@@ -374,11 +400,11 @@ int flowhip_ensemble_get_array(FlowHipEnsemble* E, int inst, int which, double* 
 
 int flowhip_ensemble_set_dt(FlowHipEnsemble* E, int inst, double dt, double dt_h) {
   if (!E || inst < 0 || inst >= E->ninst) return -1;
-  HIPCHECK(hipStreamSynchronize(E->stream));
-  E->h_dtp[0] = dt;
-  E->h_dtp[1] = dt_h;
-  HIPCHECK(hipMemcpy(E->d_dtp + 2 * inst, E->h_dtp, 2 * sizeof(double),
-                     hipMemcpyHostToDevice));
+  /* uploaded by the next call that uses the pairs, all at once */
+  E->set_dtp[2 * inst] = dt;
+  E->set_dtp[2 * inst + 1] = dt_h;
+  E->is_set[inst] = 1;
+  E->any_set = 1;
   return 0;
 }
 
@@ -458,6 +484,7 @@ int flowhip_ensemble_run(FlowHipEnsemble* E, int niters, int tt0, int pre_timest
                          double* wall_seconds, int* undefined) {
   if (!E || niters < 0) return -1;
   const int n = E->ninst;
+  ens_push_dt(E);
   ens_reserve_history(E, niters > 0 ? niters : 1);
   if (pre_timestep) HIPCHECK(fk_ens_timestep(ens_launch(E), E->fp32, E->stream));
   HIPCHECK(hipMemcpyAsync(E->h_dtp, E->d_dtp, sizeof(double) * 2 * (size_t)n,
@@ -520,6 +547,7 @@ int flowhip_ensemble_autotune(FlowHipEnsemble* E, int trial_steps, int tt0,
                               double* best_ms) {
   if (!E || trial_steps < 1) return -1;
   const int n = E->ninst;
+  ens_push_dt(E);
   if (!E->snap) HIPCHECK(hipMalloc(&E->snap, E->pool_bytes + sizeof(double) * 2 * (size_t)n));
   HIPCHECK(hipStreamSynchronize(E->stream));
   HIPCHECK(hipMemcpy(E->snap, E->pool, E->pool_bytes, hipMemcpyDeviceToDevice));

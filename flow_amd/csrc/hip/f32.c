@@ -9,10 +9,6 @@
  * the EOS pressure of near-vacuum cells (rho < 1e-6). The dt pair stays on
  * the device in FP64 and is rounded to FP32 inside each kernel.
  */
-#include <math.h>
-#include <stdio.h>
-#include <time.h>
-
 #include "schedules.h"
 
 int flowhip_f32_alloc(float** buf, size_t len) {
@@ -59,33 +55,6 @@ int flowhip_f32_boundary(Mesh* mesh, float* arr, int nxp, int nyp, int invert) {
   return 0;
 }
 
-static void push_dt32(FlowHipCtx* h, const Mesh* mesh) {
-  h->h_stage[0] = mesh->dt;
-  h->h_stage[1] = mesh->dt_h;
-  HIPCHECK(hipMemcpyAsync(h->red.dtp, h->h_stage, 2 * sizeof(double),
-                          hipMemcpyHostToDevice, h->stream));
-}
-
-/* dt pair, and the totals when with_sums, in one transfer + sync */
-static void pull32(FlowHipCtx* h, Mesh* mesh, int with_sums) {
-  HIPCHECK(hipMemcpyAsync(h->h_stage, h->red.dtp, 2 * sizeof(double),
-                          hipMemcpyDeviceToHost, h->stream));
-  if (with_sums)
-    HIPCHECK(hipMemcpyAsync(h->h_stage + 2, h->red.sums, 2 * sizeof(double),
-                            hipMemcpyDeviceToHost, h->stream));
-  HIPCHECK(hipMemcpyAsync(h->h_status, h->red.status, 2 * sizeof(int),
-                          hipMemcpyDeviceToHost, h->stream));
-  HIPCHECK(hipStreamSynchronize(h->stream));
-  flowhip_timer_collect(h);
-  mesh->dt = h->h_stage[0];
-  mesh->dt_h = h->h_stage[1];
-  if (!isfinite(mesh->dt) || !(mesh->dt > 0.0) || !isfinite(mesh->dt_h))
-    TERMINATE("hip kernel set (FP32 state): non-finite or non-positive "
-              "timestep (dt=%.12e dt_h=%.12e, %d undefined CFL candidates): "
-              "the state has diverged",
-              mesh->dt, mesh->dt_h, h->h_status[1]);
-}
-
 /* One step of omp3/flow.c:10-52 on FP32 state, in the march schedule's four
  * kernels (the same ping-pong use of P, Qxx, Qyy, uF_x, uF_y as the FP64
  * fused schedule). */
@@ -109,10 +78,22 @@ static void step_f32(FlowHipCtx* h, Mesh* mesh, FkMesh32 m, int tt, float** a) {
                                   flowhip_rows(h, FLOWHIP_K_MOMENTUM, 1), s));
 }
 
-static double now_seconds(void) {
-  struct timespec ts;
-  clock_gettime(CLOCK_MONOTONIC, &ts);
-  return (double)ts.tv_sec + 1e-9 * (double)ts.tv_nsec;
+typedef struct RunArgs32 {
+  FlowHipCtx* h;
+  Mesh* mesh;
+  float** a;
+  FkMesh32 m;
+} RunArgs32;
+
+static void enqueue_f32(void* arg, int tt) {
+  RunArgs32* r = (RunArgs32*)arg;
+  FlowHipCtx* h = r->h;
+  if (tt < 0)
+    FK_LAUNCH(h, "timestep_f32",
+              fk_timestep_f32(r->m, r->a[8], r->a[9], r->a[1], r->a[3], h->red,
+                              r->mesh->max_dt, 0, h->stream));
+  else
+    step_f32(h, r->mesh, r->m, tt, r->a);
 }
 
 /* main.c:64-115 on FP32 state; the arguments mean what flowhip_run's do. */
@@ -122,48 +103,10 @@ int flowhip_run_f32(Mesh* mesh, float** a, int niters, int tt0,
   if (niters < 0 || !a) return -1;
   if (mesh->local_nx - 2 * mesh->pad < 2 || mesh->local_ny - 2 * mesh->pad < 2)
     TERMINATE("flowhip_run_f32: the mesh needs at least 2x2 interior cells");
-  FlowHipCtx* h = flowhip_ctx(mesh);
-  const FkMesh32 m = flowhip_fkmesh32(mesh);
-  h->sums_valid = 0;
-  if (pre_timestep) {
-    push_dt32(h, mesh);
-    FK_LAUNCH(h, "timestep_f32",
-              fk_timestep_f32(m, a[8], a[9], a[1], a[3], h->red, mesh->max_dt,
-                              0, h->stream));
-    pull32(h, mesh, 0);
-  }
-  if (dt_pairs) {
-    dt_pairs[0] = mesh->dt;
-    dt_pairs[1] = mesh->dt_h;
-  }
-  if (undefined) undefined[0] = pre_timestep ? h->h_status[1] : 0;
-  double wall = 0.0, elapsed = 0.0;
-  int k;
-  for (k = 0; k < niters; ++k) {
-    const int tt = tt0 + k;
-    const double w0 = now_seconds();
-    push_dt32(h, mesh);
-    step_f32(h, mesh, m, tt, a);
-    pull32(h, mesh, 1);
-    wall += now_seconds() - w0;
-    if (mesh->rank == MASTER && mesh->verbose) {
-      printf("\nIteration %d\n", tt + 1);
-      printf("Total mass:      %.12e\n", h->h_stage[2]);
-      printf("Total energy:    %.12e\n", h->h_stage[3]);
-    }
-    if (dt_pairs) {
-      dt_pairs[2 * (k + 1)] = mesh->dt;
-      dt_pairs[2 * (k + 1) + 1] = mesh->dt_h;
-    }
-    if (mass) mass[k] = h->h_stage[2];
-    if (energy) energy[k] = h->h_stage[3];
-    if (undefined) undefined[k + 1] = h->h_status[1];
-    elapsed += mesh->dt;
-    if (elapsed >= mesh->sim_end) {
-      ++k;
-      break;
-    }
-  }
-  if (wall_seconds) *wall_seconds = wall;
-  return k;
+  RunArgs32 r = {flowhip_ctx(mesh), mesh, a, {0}};
+  r.m = flowhip_fkmesh32(mesh);
+  r.h->sums_valid = 0;
+  return flowhip_run_loop(r.h, mesh, enqueue_f32, &r, "hip kernel set (FP32 state)", niters,
+                          tt0, pre_timestep, dt_pairs, mass, energy, wall_seconds,
+                          undefined);
 }

@@ -57,8 +57,12 @@ typedef struct FlowHipCtx {
   float* geo32;
   const double* geo32_src[4];
   int geo32_nx, geo32_ny;
-  double* h_stage;      /* pinned: [0..1] dt pair, [2..5] sums */
-  int* h_status;        /* pinned */
+  double* h_stage;      /* pinned: a dt pair on its way to the device */
+  double* mail;         /* pinned: FK_MAIL_WORDS for each step in flight */
+  double pair[2];       /* the device's dt pair, when pair_known */
+  int pair_known;
+  double totals[2];     /* mass and energy of the last step or conservation call */
+  int undefined;        /* of the last dt computation */
   int schedule;
   int march_rows;       /* chunk height of every march kernel; 0: each its own */
   /* rule for undefined CFL candidates (FLOWHIP_CFL_*); under the serial
@@ -94,6 +98,20 @@ FlowHipCtx* flowhip_ctx(Mesh* mesh);
 void flowhip_ctx_destroy(Mesh* mesh);
 FkMesh flowhip_fkmesh(const Mesh* mesh);
 FkMesh32 flowhip_fkmesh32(Mesh* mesh);
+
+/* Steps that may be in flight at once (flowhip_run), a mail slot each. */
+#define FLOWHIP_AHEAD 64
+
+/* The device's dt pair made the mesh's (which the caller may have set);
+ * nothing is copied where they are the same bits. */
+void flowhip_push_pair(FlowHipCtx* h, const Mesh* mesh);
+/* Work enqueued from here on posts its results in a mail slot. */
+void flowhip_post_to(FlowHipCtx* h, int slot);
+/* Waits for the stream. */
+void flowhip_wait(FlowHipCtx* h);
+/* The pair and count of a slot whose work is done, into mesh and h; a
+ * diverged pair is fatal. */
+void flowhip_take_pair(FlowHipCtx* h, Mesh* mesh, int slot, const char* what);
 
 /* Timing brackets around one launch; no-ops unless timing is on. */
 int flowhip_timer_begin(FlowHipCtx* h, const char* name);

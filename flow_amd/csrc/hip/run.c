@@ -37,34 +37,138 @@ static double now_seconds(void) {
   return (double)ts.tv_sec + 1e-9 * (double)ts.tv_nsec;
 }
 
+/* How many of the next `most` steps can be enqueued before the host knows
+ * their dt: none but the last of them may be the one after which elapsed
+ * reaches sim_end. set_timestep's update gives dt = (C_T m + dt_h) / 2 and
+ * dt_h' = C_T m or (first step) dt with m <= min(max_dt, C_M dt_h), which
+ * grow with dt_h, so the largest values bound every later step's dt. */
+static int steps_ahead(const Mesh* mesh, double elapsed, int most) {
+  double dt_h = mesh->dt_h;
+  int n = 0;
+  while (n < most) {
+    const double m = C_T * min(mesh->max_dt, C_M * dt_h);
+    const double dt = 0.5 * (m + dt_h);
+    elapsed += dt * (1.0 + 1.0e-9);
+    dt_h = max(m, dt) * (1.0 + 1.0e-9);
+    ++n;
+    if (elapsed >= mesh->sim_end) break;
+  }
+  return n;
+}
+
+int flowhip_run_loop(FlowHipCtx* h, Mesh* mesh, void (*enqueue)(void*, int), void* arg,
+                     const char* who, int niters, int tt0, int pre_timestep,
+                     double* dt_pairs, double* mass, double* energy, double* wall_seconds,
+                     int* undefined) {
+  /* replayed graphs post to the slot they were captured with; printed steps
+   * wait their turn */
+  const int alone = h->use_graphs || (mesh->rank == MASTER && mesh->verbose);
+  double wall = 0.0, elapsed = 0.0;
+  int k = 0;
+  flowhip_push_pair(h, mesh);
+  if (pre_timestep) {
+    flowhip_post_to(h, 0);
+    enqueue(arg, -1);
+    flowhip_wait(h);
+    flowhip_take_pair(h, mesh, 0, who);
+  }
+  if (dt_pairs) {
+    dt_pairs[0] = mesh->dt;
+    dt_pairs[1] = mesh->dt_h;
+  }
+  if (undefined) undefined[0] = pre_timestep ? h->undefined : 0;
+  while (k < niters) {
+    const int left = min(niters - k, FLOWHIP_AHEAD);
+    const int n = alone ? 1 : steps_ahead(mesh, elapsed, left);
+    const double w0 = now_seconds();
+    for (int q = 0; q < n; ++q) {
+      flowhip_post_to(h, q);
+      enqueue(arg, tt0 + k + q);
+    }
+    flowhip_wait(h);
+    wall += now_seconds() - w0;
+    for (int q = 0; q < n; ++q, ++k) {
+      flowhip_take_pair(h, mesh, q, who);
+      const double* m = h->mail + (size_t)q * FK_MAIL_WORDS;
+      memcpy(h->totals, m + 2, sizeof(h->totals));
+      if (mesh->rank == MASTER && mesh->verbose) {
+        printf("\nIteration %d\n", tt0 + k + 1);
+        printf("Total mass:      %.12e\n", h->totals[0]);
+        printf("Total energy:    %.12e\n", h->totals[1]);
+      }
+      if (dt_pairs) {
+        dt_pairs[2 * (k + 1)] = mesh->dt;
+        dt_pairs[2 * (k + 1) + 1] = mesh->dt_h;
+      }
+      if (mass) mass[k] = h->totals[0];
+      if (energy) energy[k] = h->totals[1];
+      if (undefined) undefined[k + 1] = h->undefined;
+      elapsed += mesh->dt;
+      if (elapsed >= mesh->sim_end) {
+        ++k;
+        niters = k;
+        break;
+      }
+    }
+  }
+  flowhip_post_to(h, 0);
+  if (wall_seconds) *wall_seconds = wall;
+  return k;
+}
+
+typedef struct RunArgs {
+  FlowHipCtx* h;
+  FlowHipStep st;
+} RunArgs;
+
+static void enqueue_f64(void* arg, int tt) {
+  RunArgs* r = (RunArgs*)arg;
+  FlowHipCtx* h = r->h;
+  FlowHipStep* st = &r->st;
+  if (tt < 0) {
+    flowhip_enqueue_timestep(h, st->m, st->Qxx, st->Qyy, st->rho, st->e, st->max_dt, 0);
+    return;
+  }
+  st->tt = tt;
+  h->sums_valid = 0;
+  flowhip_enqueue_step(h, st);
+  if (!h->sums_valid)
+    FK_LAUNCH(h, "conservation", fk_conservation(st->m, st->rho, st->e, h->red, h->stream));
+  h->sums_valid = 0; /* posted: print_conservation computes its own again */
+}
+
 /* main.c:64-115 */
 int flowhip_run(Mesh* mesh, double** a, int niters, int tt0, int pre_timestep,
                 double* dt_pairs, double* mass, double* energy,
                 double* wall_seconds, int* undefined) {
   if (niters < 0 || !a) return -1;
+  if (!(mesh->rank == MASTER && mesh->verbose)) {
+    RunArgs r;
+    r.h = flowhip_ctx(mesh);
+    r.st = flowhip_step_of(mesh, tt0, a);
+    if (niters > 0) flowhip_check_size(mesh);
+    return flowhip_run_loop(r.h, mesh, enqueue_f64, &r, "hip kernel set", niters, tt0,
+                            pre_timestep, dt_pairs, mass, energy, wall_seconds, undefined);
+  }
+  /* the calls main.c makes, with their prints */
   const int nx = mesh->local_nx, ny = mesh->local_ny;
-  double *P = a[0], *rho = a[1], *rho_old = a[2], *e = a[3], *u = a[4],
-         *v = a[5], *mom_x = a[6], *mom_y = a[7], *Qxx = a[8], *Qyy = a[9],
-         *F_x = a[10], *F_y = a[11], *uF_x = a[12], *uF_y = a[13],
-         *vF_x = a[14], *vF_y = a[15];
+  double wall = 0.0, elapsed = 0.0;
   if (pre_timestep)
-    set_timestep(nx, ny, Qxx, Qyy, rho, e, mesh, NULL, 0, mesh->celldx,
+    set_timestep(nx, ny, a[8], a[9], a[1], a[3], mesh, NULL, 0, mesh->celldx,
                  mesh->celldy);
   if (dt_pairs) {
     dt_pairs[0] = mesh->dt;
     dt_pairs[1] = mesh->dt_h;
   }
   if (undefined) undefined[0] = pre_timestep ? flowhip_undefined_candidates(mesh) : 0;
-  double wall = 0.0, elapsed = 0.0;
   int k;
   for (k = 0; k < niters; ++k) {
     const int tt = tt0 + k;
-    if (mesh->rank == MASTER && mesh->verbose)
-      printf("\nIteration %d\n", tt + 1);
+    printf("\nIteration %d\n", tt + 1);
     const double w0 = now_seconds();
-    solve_hydro_2d(mesh, tt, P, rho, rho_old, e, u, v, mom_x, mom_y, Qxx, Qyy,
-                   F_x, F_y, uF_x, uF_y, vF_x, vF_y, NULL);
-    print_conservation(nx, ny, rho, e, NULL, mesh);
+    solve_hydro_2d(mesh, tt, a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8], a[9],
+                   a[10], a[11], a[12], a[13], a[14], a[15], NULL);
+    print_conservation(nx, ny, a[1], a[3], NULL, mesh);
     wall += now_seconds() - w0;
     if (dt_pairs) {
       dt_pairs[2 * (k + 1)] = mesh->dt;

@@ -582,7 +582,12 @@ __device__ __forceinline__ DtPair mass_pair(const FkReduce& red, const MarchStep
 /* Block 0 of the momentum march; parts: blocks of the mass/energy march. */
 __device__ __forceinline__ void step_epilogue(const FkReduce& red, int parts) {
   march_queue_reset(red.queue, kStageMom);
-  if (threadIdx.x < 2) red.dtp[threadIdx.x] = red.dtp[2 + threadIdx.x];
+  if (threadIdx.x < 2) {
+    const double v = red.dtp[2 + threadIdx.x];
+    red.dtp[threadIdx.x] = v;
+    post(red, threadIdx.x, v);
+  }
+  if (threadIdx.x == 2) post(red, 4, (double)red.status[1]);
   fold_limbs<kMNT>(red, parts);
 }
 

@@ -78,6 +78,7 @@ hipError_t fk_static_scratch(FkReduce* r, double** inv_edgedx, double** inv_edge
   q.queue = reinterpret_cast<unsigned int*>(base + kOffQueue);
   q.dtp = reinterpret_cast<double*>(base + kOffPair);
   q.sums = q.dtp + 4; /* right after the dt pairs: one copy reads both */
+  q.mail = nullptr;
   q.cfl = nullptr;
   *r = q;
   *inv_edgedx = reinterpret_cast<double*>(base + kOffInvX);

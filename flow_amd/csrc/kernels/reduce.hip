@@ -59,6 +59,9 @@ __global__ __launch_bounds__(kRedThreads) void k_finish_timestep(FkReduce r, int
     r.dtp[1] = p.dt_h;
     r.sums[2] = g;
     r.status[1] = (int)bad;
+    post(r, 0, p.dt);
+    post(r, 1, p.dt_h);
+    post(r, 4, bad);
   }
 }
 
@@ -75,6 +78,8 @@ __global__ __launch_bounds__(kRedThreads) void k_finish_sums(FkReduce r, int par
   if (threadIdx.x == 0) {
     r.sums[0] = gm.s + gm.c;
     r.sums[1] = ge.s + ge.c;
+    post(r, 2, r.sums[0]);
+    post(r, 3, r.sums[1]);
   }
 }
 
@@ -199,6 +204,9 @@ __global__ __launch_bounds__(kRedThreads) void k_finish_serial(FkReduce r, int p
     r.dtp[1] = p.dt_h;
     r.sums[2] = g;
     r.status[1] = (int)bad;
+    post(r, 0, p.dt);
+    post(r, 1, p.dt_h);
+    post(r, 4, bad);
   }
 }
 

@@ -256,6 +256,12 @@ __device__ void publish_limbs(const FixSum& fm, const FixSum& fe, FkReduce r) {
   }
 }
 
+/* A value of the dt pair (k 0, 1), a total (2, 3) or the undefined
+ * candidates (4), for the host. */
+__device__ __forceinline__ void post(const FkReduce& r, int k, double v) {
+  if (r.mail) r.mail[k] = v;
+}
+
 /* The totals of parts blocks' words -> r.sums[0..1], by one block. Thread
  * t < 252 adds word t % 14 of every 18th block, so a wave reads consecutive
  * words. The totals are the same bits whichever waves and blocks added
@@ -279,7 +285,11 @@ __device__ void fold_limbs(const FkReduce& r, int parts) {
     s_sum[0][threadIdx.x] = v;
   }
   __syncthreads();
-  if (threadIdx.x < 2) r.sums[threadIdx.x] = fixed_total(&s_sum[0][7 * threadIdx.x]);
+  if (threadIdx.x < 2) {
+    const double v = fixed_total(&s_sum[0][7 * threadIdx.x]);
+    r.sums[threadIdx.x] = v;
+    post(r, 2 + threadIdx.x, v);
+  }
 }
 
 }  // namespace flowhip

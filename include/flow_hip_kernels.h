@@ -73,6 +73,10 @@ typedef struct FkReduce {
    * step, from which the waves of its kernel claim work items. A stage's
    * set is zero when its kernel starts; each kernel zeroes the others. */
   unsigned int* queue;
+  /* NULL, or FK_MAIL_WORDS doubles of pinned host memory to which the
+   * kernel that settles a value also writes it: {dt, dt_h, mass, energy,
+   * undefined CFL candidates}. */
+  double* mail;
   /* NULL, or a cell-layout array (nx * ny doubles) that the FP64
    * Lagrangian kernels fill with every interior CFL candidate. When set,
    * the (dt, dt_h) update and the count are left to a following
@@ -81,6 +85,7 @@ typedef struct FkReduce {
 } FkReduce;
 
 #define FK_MARCH_QUEUE_WORDS 768
+#define FK_MAIL_WORDS 8
 
 /* Number of doubles FkReduce.partials must hold. */
 int fk_reduce_blocks(void);
