@@ -89,8 +89,8 @@ FlowHipCtx* flowhip_ctx(Mesh* mesh) {
    * meshes (the results are the same bits either way) */
   const char* p2 = getenv("FLOWHIP_POW2");
   h->no_pow2 = (p2 && !strcmp(p2, "0")) ? 1 : 0;
-  /* FLOWHIP_UNIFORM=0 keeps the per-row geometry loads on uniform meshes
-   * (the same bits either way) */
+  /* FLOWHIP_UNIFORM=0 keeps the geometry loads on uniform meshes (the same
+   * bits either way) */
   const char* un = getenv("FLOWHIP_UNIFORM");
   h->no_uniform = (un && !strcmp(un, "0")) ? 1 : 0;
   /* two columns per lane in the Lagrangian and mass/energy marches (the
@@ -182,15 +182,28 @@ static int all_pow2(const double* dev, int n, int emax) {
   return ok;
 }
 
-/* Whether all n values are the same. */
-static int all_equal(const double* dev, int n) {
+/* Whether all n values are the same; *value is the first. */
+static int all_equal(const double* dev, int n, double* value) {
   double* host = (double*)malloc(sizeof(double) * (size_t)n);
   if (!host) TERMINATE("hip kernel set: out of host memory");
   HIPCHECK(hipMemcpy(host, dev, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost));
   int ok = 1;
   for (int k = 1; k < n && ok; ++k) ok = (host[k] == host[0]);
+  *value = host[0];
   free(host);
   return ok;
+}
+
+FkUniform flowhip_uniform(double edx, double edy, double cdx, double cdy) {
+  const FkUniform u = {edx, edy, cdx, cdy, 1.0 / edx, 1.0 / edy, 1.0 / cdx, 1.0 / cdy};
+  return u;
+}
+
+FkUniform flowhip_uniform32(double edx, double edy, double cdx, double cdy) {
+  const float cx = (float)cdx, cy = (float)cdy;
+  const FkUniform u = {(float)edx,         (float)edy,         cx,        cy,
+                       (float)(1.0 / edx), (float)(1.0 / edy), 1.0f / cx, 1.0f / cy};
+  return u;
 }
 
 /* 1/edgedx and 1/edgedy, recomputed when the geometry arrays change, and
@@ -209,8 +222,11 @@ static void ensure_reciprocals(FlowHipCtx* h, const Mesh* mesh) {
   h->pow2_f32 = h->pow2 && all_pow2(mesh->edgedx, lx, 40) &&
                 all_pow2(mesh->edgedy, ly, 40) && all_pow2(mesh->celldx, lx, 40) &&
                 all_pow2(mesh->celldy, ly, 40);
-  h->uniform = all_equal(mesh->edgedx, lx) && all_equal(mesh->edgedy, ly) &&
-               all_equal(mesh->celldx, lx) && all_equal(mesh->celldy, ly);
+  double edx = 0.0, edy = 0.0, cdx = 0.0, cdy = 0.0;
+  h->uniform = all_equal(mesh->edgedx, lx, &edx) && all_equal(mesh->edgedy, ly, &edy) &&
+               all_equal(mesh->celldx, lx, &cdx) && all_equal(mesh->celldy, ly, &cdy);
+  h->uni = flowhip_uniform(edx, edy, cdx, cdy);
+  h->uni32 = flowhip_uniform32(edx, edy, cdx, cdy);
   h->inv_src_cx = mesh->celldx;
   h->inv_src_cy = mesh->celldy;
   hipFree(h->inv_edgedx);
@@ -233,13 +249,15 @@ FkMesh flowhip_fkmesh(const Mesh* mesh) {
     m.inv_edgedx = h->inv_edgedx;
     m.inv_edgedy = h->inv_edgedy;
     m.pow2 = h->pow2 && !h->no_pow2;
-    m.uniform = m.pow2 && h->uniform && !h->no_uniform;
+    m.uniform = h->uniform && !h->no_uniform;
+    m.u = h->uni;
     m.pairs = h->pairs;
   } else {
     m.inv_edgedx = m.inv_edgedy = NULL;
     m.pow2 = 0;
     m.uniform = 0;
     m.pairs = 0;
+    memset(&m.u, 0, sizeof(m.u));
   }
   m.nx = mesh->local_nx;
   m.ny = mesh->local_ny;
@@ -406,7 +424,8 @@ FkMesh32 flowhip_fkmesh32(Mesh* mesh) {
   f.inv_edgedx = h->geo32 + 2 * (lx + ly);
   f.inv_edgedy = h->geo32 + 3 * lx + 2 * ly;
   f.pow2 = h->pow2_f32 && !h->no_pow2;
-  f.uniform = f.pow2 && h->uniform && !h->no_uniform;
+  f.uniform = h->uniform && !h->no_uniform;
+  f.u = h->uni32;
   f.pairs = h->pairs;
   return f;
 }

@@ -268,6 +268,8 @@ FlowHipEnsemble* flowhip_ensemble_new(int ninst, const int* global_nx,
     in->nx = global_nx[i] + 4;
     in->ny = global_ny[i] + 4;
     for (int k = 0; k < 16; ++k) in->a[k] = (char*)E->pool + aoff[16 * i + k];
+    const double dx = width[i] / global_nx[i], dy = height[i] / global_ny[i];
+    in->u = fp32 ? flowhip_uniform32(dx, dy, dx, dy) : flowhip_uniform(dx, dy, dx, dy);
     in->dtp = E->d_dtp + 2 * i;
     in->max_dt = max_dt[i];
     E->h_dtp[2 * i] = C_T * dt_param[i];

@@ -49,8 +49,9 @@ typedef struct FlowHipCtx {
   int inv_nx, inv_ny;
   int pow2, pow2_f32; /* every spacing a power of two (FP64 / FP32 range) */
   int uniform;        /* each spacing array holds one value throughout */
+  FkUniform uni, uni32; /* and these are they */
   int no_pow2;        /* keep the quotients anyway */
-  int no_uniform;     /* keep the per-row geometry loads anyway */
+  int no_uniform;     /* keep the geometry loads anyway */
   int pairs;          /* FkMesh.pairs: 0 never, 1 large meshes, 2 always */
   /* FP32 copies of the geometry for the precision form: edgedx, edgedy,
    * celldx, celldy, 1/edgedx, 1/edgedy, each (L+1) floats */
@@ -98,6 +99,9 @@ FlowHipCtx* flowhip_ctx(Mesh* mesh);
 void flowhip_ctx_destroy(Mesh* mesh);
 FkMesh flowhip_fkmesh(const Mesh* mesh);
 FkMesh32 flowhip_fkmesh32(Mesh* mesh);
+/* FkUniform of four spacings, for FP64 and FP32 kernels. */
+FkUniform flowhip_uniform(double edx, double edy, double cdx, double cdy);
+FkUniform flowhip_uniform32(double edx, double edy, double cdx, double cdy);
 
 /* Steps that may be in flight at once (flowhip_run), a mail slot each. */
 #define FLOWHIP_AHEAD 64

@@ -41,6 +41,7 @@ __device__ __forceinline__ MGeo<T> ens_geo(const FkEnsInst& in) {
   g.cdy = (const T*)in.geo[3];
   g.iedx = (const T*)in.geo[4];
   g.iedy = (const T*)in.geo[5];
+  g.u = uniform_of<T>(in.u);
   return g;
 }
 

@@ -24,6 +24,20 @@
 
 namespace flowhip {
 
+/* The spacings of a uniform mesh (each spacing array holds one value
+ * throughout), passed by value: the uniform forms (template flag UNI) load no
+ * geometry at all. The host compares the arrays when it sees a mesh's geometry
+ * first; the values are the arrays' own, the reciprocals the same quotients.
+ * What that saves is a round trip to memory at the head of every item, before
+ * its first rows can be loaded, and 2 to 20 registers a lane. Measured on
+ * MI355X (us a step): FP32 1000^2 69.2 -> 64.3, 1536^2 104.8 -> 98.0,
+ * 3001x2999 338 -> 327, FP64 1000^2 105.2 -> 101.4, 3001x2999 608 -> 595,
+ * 8192^2 3528 -> 3507. */
+template <typename T>
+struct MUni {
+  T edx, edy, cdx, cdy, iedx, iedy, rcdx, rcdy;
+};
+
 template <typename T>
 struct MGeo {
   int nx, ny;
@@ -33,7 +47,23 @@ struct MGeo {
   const T* __restrict__ cdy;
   const T* __restrict__ iedx;
   const T* __restrict__ iedy;
+  MUni<T> u; /* UNI forms only */
 };
+
+/* a column's spacing */
+template <bool UNI, typename T>
+__device__ __forceinline__ T geo_at(const T* arr, T uniform, int k) {
+  if constexpr (UNI)
+    return uniform;
+  else
+    return arr[k];
+}
+
+template <typename T>
+inline __host__ __device__ MUni<T> uniform_of(const FkUniform& u) {
+  return MUni<T>{T(u.edx),  T(u.edy),  T(u.cdx),  T(u.cdy),
+                 T(u.iedx), T(u.iedy), T(u.rcdx), T(u.rcdy)};
+}
 
 template <typename T>
 struct MMassIO {
@@ -325,6 +355,8 @@ template <typename T>
 struct RowGeo {
   T a, b;
   int base;
+  __device__ RowGeo(const T* arr, T, int base_row, int last_row, int lane, bool recip)
+      : RowGeo(arr, base_row, last_row, lane, recip) {}
   __device__ RowGeo(const T* arr, int base_row, int last_row, int lane,
                     bool recip = false)
       : base(base_row) {
@@ -354,7 +386,7 @@ template <typename T>
 struct RowScalar {
   const __attribute__((address_space(4))) T* p;
   int last;
-  __device__ RowScalar(const T* arr, int, int last_row, int)
+  __device__ RowScalar(const T* arr, T, int, int last_row, int)
       : p((const __attribute__((address_space(4))) T*)(unsigned long long)arr),
         last(last_row) {}
   /* value at row r (wave-uniform) */
@@ -369,8 +401,8 @@ template <typename T, bool P2>
 struct RowRecip {
   RowScalar<T> d;
   /* (the flag matches RowGeo's constructor; these are always reciprocals) */
-  __device__ RowRecip(const T* arr, int base_row, int last_row, int lane, bool = true)
-      : d(arr, base_row, last_row, lane) {}
+  __device__ RowRecip(const T* arr, T, int base_row, int last_row, int lane, bool = true)
+      : d(arr, T(0), base_row, last_row, lane) {}
   __device__ __forceinline__ T operator()(int r) const {
     if constexpr (P2)
       return recip_pow2(d(r));
@@ -379,36 +411,19 @@ struct RowRecip {
   }
 };
 
-/* Row geometry of a uniform mesh (each spacing array holds one value
- * throughout): the value is read once per work item and every row reads it
- * from a scalar register. Same values as RowScalar / RowRecip at every row.
- * Measured on MI355X at 8192^2: the fused momentum march 5% faster, the
- * mass/energy march 0.5-1%; the Lagrangian march was not (it keeps the
- * per-row loads). */
+/* Row geometry of a uniform mesh: the same value at every row, from a scalar
+ * register. */
 template <typename T>
 struct RowConst {
   T v;
-  __device__ RowConst(const T* arr, int, int, int, bool = false)
-      : v(((const __attribute__((address_space(4))) T*)(unsigned long long)arr)[0]) {}
-  __device__ __forceinline__ T operator()(int) const { return v; }
-};
-template <typename T, bool P2>
-struct RowConstRecip {
-  T v;
-  __device__ RowConstRecip(const T* arr, int, int, int, bool = true) {
-    const T d = ((const __attribute__((address_space(4))) T*)(unsigned long long)arr)[0];
-    if constexpr (P2)
-      v = recip_pow2(d);
-    else
-      v = T(1.0) / d;
-  }
+  __device__ RowConst(const T*, T value, int, int, int, bool = false) : v(value) {}
   __device__ __forceinline__ T operator()(int) const { return v; }
 };
 /* UNI selects the uniform-mesh forms */
 template <typename T, bool UNI>
 using RowS = typename std::conditional<UNI, RowConst<T>, RowScalar<T>>::type;
 template <typename T, bool P2, bool UNI>
-using RowR = typename std::conditional<UNI, RowConstRecip<T, P2>, RowRecip<T, P2>>::type;
+using RowR = typename std::conditional<UNI, RowConst<T>, RowRecip<T, P2>>::type;
 
 /* ---- boundary-strip writers (ghost writes only in edge items) ---- */
 template <typename T>
@@ -618,14 +633,18 @@ __device__ __forceinline__ void mass_xy_box(const MGeo<T>& g, const MMassIO<T>& 
   const int qf = q <= nx ? q : nx;             /* a valid x face for loads */
   /* per-lane geometry, loaded once per item: no load inside the row loop
    * other than the next row's prefetch */
-  const T cdx_q = g.cdx[qc], edx_q = g.edx[qc], edx_q1 = g.edx[qc + 1];
+  const T cdx_q = geo_at<UNI>(g.cdx, g.u.cdx, qc);
+  const T edx_q = geo_at<UNI>(g.edx, g.u.edx, qc);
+  const T edx_q1 = geo_at<UNI>(g.edx, g.u.edx, qc + 1);
   const int qg = face ? q : x0;
-  const T cdx_qm1 = g.cdx[qg - 1], iedx_q = g.iedx[qg];
-  const RowS<T, UNI> edy(g.edy, y0 - 4, ny, lane), cdy(g.cdy, y0 - 4, ny, lane);
-  const RowS<T, UNI> iedy(g.iedy, y0 - 4, ny, lane);
+  const T cdx_qm1 = geo_at<UNI>(g.cdx, g.u.cdx, qg - 1);
+  const T iedx_q = geo_at<UNI>(g.iedx, g.u.iedx, qg);
+  const RowS<T, UNI> edy(g.edy, g.u.edy, y0 - 4, ny, lane);
+  const RowS<T, UNI> cdy(g.cdy, g.u.cdy, y0 - 4, ny, lane);
+  const RowS<T, UNI> iedy(g.iedy, g.u.iedy, y0 - 4, ny, lane);
   /* reciprocal spacings, used in place of quotients on power-of-two meshes */
-  const T rcdx_q = T(1.0) / cdx_q;
-  const RowR<T, P2, UNI> rcdy(g.cdy, y0 - 4, ny, lane);
+  const T rcdx_q = UNI ? g.u.rcdx : T(1.0) / cdx_q;
+  const RowR<T, P2, UNI> rcdy(g.cdy, g.u.rcdy, y0 - 4, ny, lane);
 
   /* rows of the x-updated fields for this lane's column: w[0] oldest */
   T wr[4], we[4];
@@ -755,17 +774,18 @@ __device__ __forceinline__ void mass_xy_pair(const MGeo<T>& g, const MMassIO<T>&
   for (int c = 0; c < 2; ++c) {
     const int q = qb + c;
     face[c] = q >= x0 && q <= x1;
-    cdx_q[c] = g.cdx[q];
-    edx_q[c] = g.edx[q];
-    edx_q1[c] = g.edx[q + 1];
+    cdx_q[c] = geo_at<UNI>(g.cdx, g.u.cdx, q);
+    edx_q[c] = geo_at<UNI>(g.edx, g.u.edx, q);
+    edx_q1[c] = geo_at<UNI>(g.edx, g.u.edx, q + 1);
     const int qg = face[c] ? q : x0;
-    cdx_qm1[c] = g.cdx[qg - 1];
-    iedx_q[c] = g.iedx[qg];
-    rcdx_q[c] = T(1.0) / cdx_q[c];
+    cdx_qm1[c] = geo_at<UNI>(g.cdx, g.u.cdx, qg - 1);
+    iedx_q[c] = geo_at<UNI>(g.iedx, g.u.iedx, qg);
+    rcdx_q[c] = UNI ? g.u.rcdx : T(1.0) / cdx_q[c];
   }
-  const RowS<T, UNI> edy(g.edy, y0 - 4, ny, lane), cdy(g.cdy, y0 - 4, ny, lane);
-  const RowS<T, UNI> iedy(g.iedy, y0 - 4, ny, lane);
-  const RowR<T, P2, UNI> rcdy(g.cdy, y0 - 4, ny, lane);
+  const RowS<T, UNI> edy(g.edy, g.u.edy, y0 - 4, ny, lane);
+  const RowS<T, UNI> cdy(g.cdy, g.u.cdy, y0 - 4, ny, lane);
+  const RowS<T, UNI> iedy(g.iedy, g.u.iedy, y0 - 4, ny, lane);
+  const RowR<T, P2, UNI> rcdy(g.cdy, g.u.rcdy, y0 - 4, ny, lane);
   auto ldc = [&](const T* a, int row, T(&x)[2]) { ld_pair(a, (long)row * nx + qb, x); };
   auto ldx = [&](const T* a, int row, T(&x)[2]) { ld_xpair(a, (long)row * sx + qb, x); };
 
@@ -947,15 +967,19 @@ __device__ __forceinline__ void mass_yx_box(const MGeo<T>& g, const MMassIO<T>& 
   const int qm = !EDGE ? q : (inq ? mirror(q, nx) : nx - kPad - 1);
   const int qc = inq ? q : nx - 1;
   const int qf = q <= nx ? q : nx;
-  const T cdx_m = g.cdx[qm], edx_m = g.edx[qm], edx_m1 = g.edx[qm + 1];
-  const T cdx_q = g.cdx[qc];
+  const T cdx_m = geo_at<UNI>(g.cdx, g.u.cdx, qm);
+  const T edx_m = geo_at<UNI>(g.edx, g.u.edx, qm);
+  const T edx_m1 = geo_at<UNI>(g.edx, g.u.edx, qm + 1);
+  const T cdx_q = geo_at<UNI>(g.cdx, g.u.cdx, qc);
   const int qg = face ? q : x0;
-  const T cdx_qm1 = g.cdx[qg - 1], iedx_q = g.iedx[qg];
-  const RowS<T, UNI> edy(g.edy, y0 - 4, ny, lane), cdy(g.cdy, y0 - 4, ny, lane);
-  const RowS<T, UNI> iedy(g.iedy, y0 - 4, ny, lane);
+  const T cdx_qm1 = geo_at<UNI>(g.cdx, g.u.cdx, qg - 1);
+  const T iedx_q = geo_at<UNI>(g.iedx, g.u.iedx, qg);
+  const RowS<T, UNI> edy(g.edy, g.u.edy, y0 - 4, ny, lane);
+  const RowS<T, UNI> cdy(g.cdy, g.u.cdy, y0 - 4, ny, lane);
+  const RowS<T, UNI> iedy(g.iedy, g.u.iedy, y0 - 4, ny, lane);
   /* reciprocal spacings, used in place of quotients on power-of-two meshes */
-  const T rcdx_q = T(1.0) / cdx_q, rcdx_m = T(1.0) / cdx_m;
-  const RowR<T, P2, UNI> rcdy(g.cdy, y0 - 4, ny, lane);
+  const T rcdx_q = UNI ? g.u.rcdx : T(1.0) / cdx_q, rcdx_m = UNI ? g.u.rcdx : T(1.0) / cdx_m;
+  const RowR<T, P2, UNI> rcdy(g.cdy, g.u.rcdy, y0 - 4, ny, lane);
 
   /* rho0, e1 at rows r-1 .. r+2 and v0 at faces r .. r+2 of column qm */
   T wr[4], we[4], wv[3];
@@ -1064,17 +1088,18 @@ __device__ __forceinline__ void mass_yx_pair(const MGeo<T>& g, const MMassIO<T>&
   for (int c = 0; c < 2; ++c) {
     const int q = qb + c;
     face[c] = q >= x0 && q <= x1;
-    cdx_q[c] = g.cdx[q];
-    edx_q[c] = g.edx[q];
-    edx_q1[c] = g.edx[q + 1];
+    cdx_q[c] = geo_at<UNI>(g.cdx, g.u.cdx, q);
+    edx_q[c] = geo_at<UNI>(g.edx, g.u.edx, q);
+    edx_q1[c] = geo_at<UNI>(g.edx, g.u.edx, q + 1);
     const int qg = face[c] ? q : x0;
-    cdx_qm1[c] = g.cdx[qg - 1];
-    iedx_q[c] = g.iedx[qg];
-    rcdx_q[c] = T(1.0) / cdx_q[c];
+    cdx_qm1[c] = geo_at<UNI>(g.cdx, g.u.cdx, qg - 1);
+    iedx_q[c] = geo_at<UNI>(g.iedx, g.u.iedx, qg);
+    rcdx_q[c] = UNI ? g.u.rcdx : T(1.0) / cdx_q[c];
   }
-  const RowS<T, UNI> edy(g.edy, y0 - 4, ny, lane), cdy(g.cdy, y0 - 4, ny, lane);
-  const RowS<T, UNI> iedy(g.iedy, y0 - 4, ny, lane);
-  const RowR<T, P2, UNI> rcdy(g.cdy, y0 - 4, ny, lane);
+  const RowS<T, UNI> edy(g.edy, g.u.edy, y0 - 4, ny, lane);
+  const RowS<T, UNI> cdy(g.cdy, g.u.cdy, y0 - 4, ny, lane);
+  const RowS<T, UNI> iedy(g.iedy, g.u.iedy, y0 - 4, ny, lane);
+  const RowR<T, P2, UNI> rcdy(g.cdy, g.u.rcdy, y0 - 4, ny, lane);
   auto ldc = [&](const T* a, int row, T(&x)[2]) { ld_pair(a, (long)row * nx + qb, x); };
   auto ldx = [&](const T* a, int row, T(&x)[2]) { ld_xpair(a, (long)row * sx + qb, x); };
 
@@ -1777,17 +1802,20 @@ __device__ __forceinline__ void lagrangian_box(const MGeo<T>& g, const MLagIO<T>
   const int mf_lane = mirror_lane(lane, q, sx), mc_lane = mirror_lane(lane, q, nx);
   const bool own_face = q >= x0 && (q < x1 || (q == x1 && x1 == nx - kPad));
   const bool own = q >= x0 && q < x1;
-  const T edx_q = g.edx[qg], cdx_q = g.cdx[qg], cdx_qm = g.cdx[qg - 1];
-  const RowS<T, UNI> edy(g.edy, y0 - 4, ny, lane), cdy(g.cdy, y0 - 4, ny, lane);
+  const T edx_q = geo_at<UNI>(g.edx, g.u.edx, qg);
+  const T cdx_q = geo_at<UNI>(g.cdx, g.u.cdx, qg);
+  const T cdx_qm = geo_at<UNI>(g.cdx, g.u.cdx, qg - 1);
+  const RowS<T, UNI> edy(g.edy, g.u.edy, y0 - 4, ny, lane);
+  const RowS<T, UNI> cdy(g.cdy, g.u.cdy, y0 - 4, ny, lane);
   /* reciprocal spacings, used in place of quotients on power-of-two meshes */
-  const T iedx_q = g.iedx[qg], rcdx_q = T(1.0) / cdx_q;
-  const RowS<T, UNI> iedy(g.iedy, y0 - 4, ny, lane);
+  const T iedx_q = geo_at<UNI>(g.iedx, g.u.iedx, qg), rcdx_q = UNI ? g.u.rcdx : T(1.0) / cdx_q;
+  const RowS<T, UNI> iedy(g.iedy, g.u.iedy, y0 - 4, ny, lane);
   /* lane-held reciprocals in FP32: 2% faster there than RowRecip */
   using Recip = typename std::conditional<
-      UNI, RowConstRecip<T, P2>,
+      UNI, RowConst<T>,
       typename std::conditional<std::is_same<T, float>::value, RowGeo<T>,
                                 RowRecip<T, P2>>::type>::type;
-  const Recip rcdy(g.cdy, y0 - 4, ny, lane, true);
+  const Recip rcdy(g.cdy, g.u.rcdy, y0 - 4, ny, lane, true);
 
   /* y face k of the lane's column after pressure acceleration, from cell
    * rows k (rk, ek) and k-1 (rs, es) and mom_y at face k */
@@ -2012,19 +2040,20 @@ __device__ __forceinline__ void lagrangian_pair(const MGeo<T>& g, const MLagIO<T
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
     const int q = qb + c;
-    edx_q[c] = g.edx[q];
-    cdx_q[c] = g.cdx[q];
-    cdx_qm[c] = g.cdx[q - 1];
-    iedx_q[c] = g.iedx[q];
-    rcdx_q[c] = T(1.0) / cdx_q[c];
+    edx_q[c] = geo_at<UNI>(g.edx, g.u.edx, q);
+    cdx_q[c] = geo_at<UNI>(g.cdx, g.u.cdx, q);
+    cdx_qm[c] = geo_at<UNI>(g.cdx, g.u.cdx, q - 1);
+    iedx_q[c] = geo_at<UNI>(g.iedx, g.u.iedx, q);
+    rcdx_q[c] = UNI ? g.u.rcdx : T(1.0) / cdx_q[c];
   }
-  const RowS<T, UNI> edy(g.edy, y0 - 4, ny, lane), cdy(g.cdy, y0 - 4, ny, lane);
-  const RowS<T, UNI> iedy(g.iedy, y0 - 4, ny, lane);
+  const RowS<T, UNI> edy(g.edy, g.u.edy, y0 - 4, ny, lane);
+  const RowS<T, UNI> cdy(g.cdy, g.u.cdy, y0 - 4, ny, lane);
+  const RowS<T, UNI> iedy(g.iedy, g.u.iedy, y0 - 4, ny, lane);
   using Recip = typename std::conditional<
-      UNI, RowConstRecip<T, P2>,
+      UNI, RowConst<T>,
       typename std::conditional<std::is_same<T, float>::value, RowGeo<T>,
                                 RowRecip<T, P2>>::type>::type;
-  const Recip rcdy(g.cdy, y0 - 4, ny, lane, true);
+  const Recip rcdy(g.cdy, g.u.rcdy, y0 - 4, ny, lane, true);
   auto ldc = [&](const T* a, int row, P& x) { ld_pair(a, (long)row * nx + qb, x); };
   auto ldx = [&](const T* a, int row, P& x) { ld_xpair(a, (long)row * sx + qb, x); };
 
@@ -2314,13 +2343,16 @@ __device__ __forceinline__ void momxy_xy_item(const MGeo<T>& g, const MMom2IO<T>
   const int mc_lane = mirror_lane(lane, q, nx);
   const bool own_x = q >= x0 && (q < x1 || (q == x1 && x1 == nx - kPad));
   const bool own_y = q >= x0 && q < x1;
-  const T edx_q = g.edx[qg], cdx_q = g.cdx[qg], cdx_qm = g.cdx[qg - 1];
-  const T iedx_q = g.iedx[qg];
-  const RowS<T, UNI> edy(g.edy, y0 - 4, ny, lane), cdy(g.cdy, y0 - 4, ny, lane);
-  const RowS<T, UNI> iedy(g.iedy, y0 - 4, ny, lane);
+  const T edx_q = geo_at<UNI>(g.edx, g.u.edx, qg);
+  const T cdx_q = geo_at<UNI>(g.cdx, g.u.cdx, qg);
+  const T cdx_qm = geo_at<UNI>(g.cdx, g.u.cdx, qg - 1);
+  const T iedx_q = geo_at<UNI>(g.iedx, g.u.iedx, qg);
+  const RowS<T, UNI> edy(g.edy, g.u.edy, y0 - 4, ny, lane);
+  const RowS<T, UNI> cdy(g.cdy, g.u.cdy, y0 - 4, ny, lane);
+  const RowS<T, UNI> iedy(g.iedy, g.u.iedy, y0 - 4, ny, lane);
   /* reciprocal spacings, used in place of quotients on power-of-two meshes */
-  const T rcdx_q = T(1.0) / cdx_q;
-  const RowR<T, P2, UNI> rcdy(g.cdy, y0 - 4, ny, lane);
+  const T rcdx_q = UNI ? g.u.rcdx : T(1.0) / cdx_q;
+  const RowR<T, P2, UNI> rcdy(g.cdy, g.u.rcdy, y0 - 4, ny, lane);
 
   /* x stage: u1 and m1 of cell row i from that row's u0, F_x, mx1, rho */
   auto xrow = [&](int i, T a_u, T a_fx, T a_m1, T a_r, T& m1, T& u1) {
@@ -2509,13 +2541,16 @@ __device__ __forceinline__ void momxy_yx_item(const MGeo<T>& g, const MMom2IO<T>
   const int mf_lane = mirror_lane(lane, q, sx), mc_lane = mirror_lane(lane, q, nx);
   const bool own_x = q >= x0 && (q < x1 || (q == x1 && x1 == nx - kPad));
   const bool own_y = q >= x0 && q < x1;
-  const T edx_q = g.edx[qg], cdx_q = g.cdx[qg], cdx_qm = g.cdx[qg - 1];
-  const T iedx_q = g.iedx[qg];
-  const RowS<T, UNI> edy(g.edy, y0 - 4, ny, lane), cdy(g.cdy, y0 - 4, ny, lane);
-  const RowS<T, UNI> iedy(g.iedy, y0 - 4, ny, lane);
+  const T edx_q = geo_at<UNI>(g.edx, g.u.edx, qg);
+  const T cdx_q = geo_at<UNI>(g.cdx, g.u.cdx, qg);
+  const T cdx_qm = geo_at<UNI>(g.cdx, g.u.cdx, qg - 1);
+  const T iedx_q = geo_at<UNI>(g.iedx, g.u.iedx, qg);
+  const RowS<T, UNI> edy(g.edy, g.u.edy, y0 - 4, ny, lane);
+  const RowS<T, UNI> cdy(g.cdy, g.u.cdy, y0 - 4, ny, lane);
+  const RowS<T, UNI> iedy(g.iedy, g.u.iedy, y0 - 4, ny, lane);
   /* reciprocal spacings, used in place of quotients on power-of-two meshes */
-  const T rcdx_q = T(1.0) / cdx_q;
-  const RowR<T, P2, UNI> rcdy(g.cdy, y0 - 4, ny, lane);
+  const T rcdx_q = UNI ? g.u.rcdx : T(1.0) / cdx_q;
+  const RowR<T, P2, UNI> rcdy(g.cdy, g.u.rcdy, y0 - 4, ny, lane);
 
   /* x stage: x flux in y at corner row gf from u0 rows gf-2 .. gf+1 */
   auto corner = [&](int gf, T w0, T w1, T w2, T w3, T a_v, T a_fy) {

@@ -185,34 +185,39 @@ hipError_t launch_march_momxy_p(MGeo<T> g, MMom2IO<T> io, int tt, FkReduce r, in
 }
 
 /* Dispatch on whether every mesh spacing is a power of two (quotients by
- * spacings become products with exact reciprocals) and, for the mass/energy
- * and fused momentum marches, whether such a mesh is also uniform (row
- * geometry read once per item). */
+ * spacings become products with exact reciprocals) and whether the mesh is
+ * uniform (MUni): launch<P2, UNI>. */
+template <typename F>
+hipError_t by_geometry(int pow2, int uniform, F&& launch) {
+  using Yes = std::true_type;
+  using No = std::false_type;
+  if (uniform) return pow2 ? launch(Yes{}, Yes{}) : launch(No{}, Yes{});
+  return pow2 ? launch(Yes{}, No{}) : launch(No{}, No{});
+}
+
 template <typename T>
 hipError_t launch_march_mass(MGeo<T> g, MMassIO<T> io, int tt, FkReduce r, MarchStep st,
                              int* parts, int chunk_rows, int pow2, int uniform, int pairs,
                              hipStream_t s) {
   if (pairs_wanted(pairs, g.nx, g.ny) && pow2 && uniform && pairs_fit(g, io))
     return launch_march_mass_p<T, true, true, true>(g, io, tt, r, st, parts, chunk_rows, s);
-  if (pow2 && uniform) return launch_march_mass_p<T, true, true>(g, io, tt, r, st, parts, chunk_rows, s);
-  return pow2 ? launch_march_mass_p<T, true, false>(g, io, tt, r, st, parts, chunk_rows, s)
-              : launch_march_mass_p<T, false, false>(g, io, tt, r, st, parts, chunk_rows, s);
+  return by_geometry(pow2, uniform, [&](auto p2, auto uni) {
+    return launch_march_mass_p<T, decltype(p2)::value, decltype(uni)::value>(
+        g, io, tt, r, st, parts, chunk_rows, s);
+  });
 }
 
-/* The Lagrangian march takes the uniform-mesh form in FP32 only (in FP64 it
- * measured 1% slower than the per-row loads). */
 template <typename T>
 hipError_t launch_march_lagrangian(MGeo<T> g, MLagIO<T> io, FkReduce r, double max_dt,
                                    int* parts, int chunk_rows, int pow2, int uniform,
                                    int pairs, hipStream_t s) {
   if (pairs_wanted(pairs, g.nx, g.ny) && pow2 && uniform && lag_pairs_fit(g, io))
-    return launch_march_lagrangian_p<T, true, true, true>(g, io, r, max_dt, parts, chunk_rows, s);
-  if constexpr (sizeof(T) == 4) {
-    if (pow2 && uniform)
-      return launch_march_lagrangian_p<T, true, true>(g, io, r, max_dt, parts, chunk_rows, s);
-  }
-  return pow2 ? launch_march_lagrangian_p<T, true, false>(g, io, r, max_dt, parts, chunk_rows, s)
-              : launch_march_lagrangian_p<T, false, false>(g, io, r, max_dt, parts, chunk_rows, s);
+    return launch_march_lagrangian_p<T, true, true, true>(g, io, r, max_dt, parts,
+                                                          chunk_rows, s);
+  return by_geometry(pow2, uniform, [&](auto p2, auto uni) {
+    return launch_march_lagrangian_p<T, decltype(p2)::value, decltype(uni)::value>(
+        g, io, r, max_dt, parts, chunk_rows, s);
+  });
 }
 
 template <typename T>
@@ -226,10 +231,10 @@ hipError_t launch_march_momentum(MGeo<T> g, MMomIO<T> io, int tt, int ydir,
 template <typename T>
 hipError_t launch_march_momxy(MGeo<T> g, MMom2IO<T> io, int tt, FkReduce r, int parts,
                               int chunk_rows, int pow2, int uniform, hipStream_t s) {
-  if (pow2 && uniform)
-    return launch_march_momxy_p<T, true, true>(g, io, tt, r, parts, chunk_rows, s);
-  return pow2 ? launch_march_momxy_p<T, true, false>(g, io, tt, r, parts, chunk_rows, s)
-              : launch_march_momxy_p<T, false, false>(g, io, tt, r, parts, chunk_rows, s);
+  return by_geometry(pow2, uniform, [&](auto p2, auto uni) {
+    return launch_march_momxy_p<T, decltype(p2)::value, decltype(uni)::value>(
+        g, io, tt, r, parts, chunk_rows, s);
+  });
 }
 
 }  // namespace flowhip
@@ -238,7 +243,7 @@ using namespace flowhip;
 
 static MGeo<double> mgeo64(FkMesh m) {
   MGeo<double> g{m.nx, m.ny, m.edgedx, m.edgedy, m.celldx, m.celldy,
-                 m.inv_edgedx, m.inv_edgedy};
+                 m.inv_edgedx, m.inv_edgedy, uniform_of<double>(m.u)};
   return g;
 }
 
@@ -296,7 +301,7 @@ hipError_t fk_march_mass_energy(FkMesh m, int tt, const double* u0,
 
 static MGeo<float> mgeo32(FkMesh32 m) {
   MGeo<float> g{m.nx, m.ny, m.edgedx, m.edgedy, m.celldx, m.celldy,
-                m.inv_edgedx, m.inv_edgedy};
+                m.inv_edgedx, m.inv_edgedy, uniform_of<float>(m.u)};
   return g;
 }
 

@@ -20,6 +20,15 @@
 extern "C" {
 #endif
 
+/* The spacings of a mesh whose four spacing arrays each hold one value
+ * throughout: edgedx, edgedy, celldx, celldy, 1 / edgedx, 1 / edgedy, 1 /
+ * celldx and 1 / celldy. In an FP32-state form the values are the FP32 ones
+ * (spacings rounded, 1 / edge rounded from the FP64 quotient, 1 / cell the
+ * FP32 quotient), which a double holds exactly. */
+typedef struct FkUniform {
+  double edx, edy, cdx, cdy, iedx, iedy, rcdx, rcdy;
+} FkUniform;
+
 typedef struct FkMesh {
   int nx, ny, pad;
   const double *edgedx, *edgedy, *celldx, *celldy; /* device, L+1 each */
@@ -30,10 +39,10 @@ typedef struct FkMesh {
   /* 1 when every spacing above is a power of two (the march kernels then
    * divide by spacings as products with exact reciprocals), else 0 */
   int pow2;
-  /* 1 when, besides, each of the four spacing arrays holds one value
-   * throughout (the mass/energy and momentum marches then read the row
-   * geometry once per work item instead of once per row), else 0 */
+  /* 1 when each of the four spacing arrays holds one value throughout (the
+   * march kernels then take the values in u and load no geometry), else 0 */
   int uniform;
+  FkUniform u;
   /* Whether the Lagrangian and mass/energy marches hold two columns per
    * lane on uniform power-of-two meshes (each can when nx is even and the
    * cell and y-face arrays it reads and writes are 16-byte aligned):
@@ -57,6 +66,7 @@ typedef struct FkMesh32 {
   const float *inv_edgedx, *inv_edgedy;
   int pow2;
   int uniform; /* as in FkMesh */
+  FkUniform u;
   int pairs;   /* as in FkMesh (8-byte alignment) */
 } FkMesh32;
 
@@ -309,6 +319,7 @@ hipError_t fk_march_momentum_y_f32(FkMesh32 m, int tt, const float* u1,
 typedef struct FkEnsInst {
   int nx, ny;              /* local sizes, pad included */
   const void* geo[6];      /* edgedx, edgedy, celldx, celldy, 1/edgedx, 1/edgedy */
+  FkUniform u;             /* the same, by value */
   void* a[16];             /* solve_hydro_2d's arrays, in its order */
   double* dtp;             /* {dt, dt_h} of this instance (device) */
   double max_dt;
@@ -334,8 +345,8 @@ typedef struct FkEnsLaunch {
   const int* work;         /* device, nwork (instance, item) pairs */
   int ninst, nwork, chunk_rows;
   int pow2;                /* every instance's spacings are powers of two */
-  int uniform;             /* read each instance's spacings once per item
-                              (they hold one value throughout) */
+  int uniform;             /* take each instance's spacings by value (its
+                              arrays hold one value throughout) */
   int fused_momentum;      /* both momentum directions in one march */
   unsigned int* queue;     /* FK_MARCH_QUEUE_WORDS work-queue words, zero
                               between steps (the epilogue kernels zero them) */
