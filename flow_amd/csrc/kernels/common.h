@@ -29,14 +29,53 @@ inline dim3 sw_grid(const Domain& d) {
   return dim3(gx > 0 ? gx : 1, gy > 0 ? gy : 1, 1);
 }
 
-/* Wave64 reductions through cross-lane shuffles. */
+/* One step of a wave64 reduction as DPP moves: lane i of a row of 16 reads
+ * lane i - 1, 2, 4, 8 (row_shr), then rows 1 and 3 read lane 15 of the row
+ * before, then rows 2 and 3 read lane 31, so lane 63 ends with the whole
+ * wave's. A lane without a source reads old. Register moves, a few cycles
+ * each; the shuffles they replace go through LDS, 50 cycles and more a step. */
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned int dpp_step(unsigned int old, unsigned int v) {
+  return (unsigned int)__builtin_amdgcn_update_dpp((int)old, (int)v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned long long dpp_step(unsigned long long old,
+                                                       unsigned long long v) {
+  const unsigned int lo = dpp_step<CTRL, ROWS>((unsigned int)old, (unsigned int)v);
+  const unsigned int hi =
+      dpp_step<CTRL, ROWS>((unsigned int)(old >> 32), (unsigned int)(v >> 32));
+  return ((unsigned long long)hi << 32) | lo;
+}
+/* op(control, row mask) for each step of a wave's reduction */
+#define FLOWHIP_DPP_STEPS(op) \
+  op(0x111, 0xf) op(0x112, 0xf) op(0x114, 0xf) op(0x118, 0xf) op(0x142, 0xa) op(0x143, 0xc)
+
+/* lane 63's value, in every lane */
+__device__ __forceinline__ unsigned long long last_lane(unsigned long long v) {
+  const unsigned int lo = __builtin_amdgcn_readlane((int)(unsigned int)v, kWave - 1);
+  const unsigned int hi = __builtin_amdgcn_readlane((int)(unsigned int)(v >> 32), kWave - 1);
+  return ((unsigned long long)hi << 32) | lo;
+}
+
+/* The minimum over the wave (all lanes active), in every lane. */
 __device__ __forceinline__ double wave_min(double x) {
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) {
-    const double y = __shfl_xor(x, off, kWave);
-    x = (y < x) ? y : x;
+#define FLOWHIP_MIN_STEP(ctrl, rows)                                                 \
+  {                                                                                  \
+    const unsigned long long v = __builtin_bit_cast(unsigned long long, x);          \
+    const double y = __builtin_bit_cast(double, (dpp_step<ctrl, rows>(v, v)));       \
+    x = (y < x) ? y : x;                                                             \
   }
-  return x;
+  FLOWHIP_DPP_STEPS(FLOWHIP_MIN_STEP)
+#undef FLOWHIP_MIN_STEP
+  return __builtin_bit_cast(double, last_lane(__builtin_bit_cast(unsigned long long, x)));
+}
+
+/* The sum over the wave (all lanes active), in every lane. */
+__device__ __forceinline__ int wave_sum(int x) {
+#define FLOWHIP_SUM_STEP(ctrl, rows) x += (int)dpp_step<ctrl, rows>(0u, (unsigned int)x);
+  FLOWHIP_DPP_STEPS(FLOWHIP_SUM_STEP)
+#undef FLOWHIP_SUM_STEP
+  return __builtin_amdgcn_readlane(x, kWave - 1);
 }
 
 /* 1/x for a positive power of two x with a normal reciprocal, exactly: 2^-k

@@ -64,12 +64,6 @@ __device__ __forceinline__ MarchList ens_list(const FkEnsInst& in, int H) {
   return ml;
 }
 
-__device__ __forceinline__ int wave_sum_int(int x) {
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) x += __shfl_xor(x, off, kWave);
-  return x;
-}
-
 /* ---- the four stages ---- */
 
 template <typename T, bool P2, bool UNI>
@@ -103,7 +97,7 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_lagrangian(
       lagrangian_item<T, P2, -1, true, kUni>(g, io, dt, dt_h, ml, wi.y, lane, local_min,
                                              nan_count);
     local_min = wave_min(local_min);
-    nan_count = wave_sum_int(nan_count);
+    nan_count = wave_sum(nan_count);
     if (lane == 0) {
       part.min[in.item0 + wi.y] = local_min;
       part.nan[in.item0 + wi.y] = nan_count;
@@ -258,7 +252,7 @@ __global__ __launch_bounds__(kMNT) void k_ens_timestep(
       }
     }
     local_min = wave_min(local_min);
-    nan_count = wave_sum_int(nan_count);
+    nan_count = wave_sum(nan_count);
     if (lane == 0) {
       part.min[in.item0 + wi.y] = local_min;
       part.nan[in.item0 + wi.y] = nan_count;
@@ -290,7 +284,7 @@ __global__ __launch_bounds__(kWave) void k_ens_dt(const FkEnsInst* __restrict__ 
   }
   g = wave_min(g);
   if (squared) g = __builtin_sqrt(g);
-  bad = wave_sum_int(bad);
+  bad = wave_sum(bad);
   if (lane == 0) {
     const double dt_h = in.dtp[1];
     const double final_min = lesser(g, kCM * dt_h);

@@ -578,17 +578,20 @@ template <typename T>
 __device__ __forceinline__ DtPair mass_pair(const FkReduce& red, const MarchStep& st) {
   DtPair p{red.dtp[0], red.dtp[1]};
   if (blockIdx.x == 0) march_queue_reset(red.queue, kStageMass);
-  double g = 0.0, bad = 0.0;
+  double g = 0.0;
   if (st.lag_parts) {
-    fold_min<kMNT, std::is_same<T, float>::value>(red, st.lag_parts, st.max_dt, g, bad);
+    g = fold_min<std::is_same<T, float>::value>(red, st.lag_parts, st.max_dt);
     p = next_pair(g, p.dt_h, st.first_step);
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    red.dtp[2] = p.dt;
-    red.dtp[3] = p.dt_h;
-    if (st.lag_parts) {
-      red.sums[2] = g;
-      red.status[1] = (int)bad;
+  if (blockIdx.x == 0 && threadIdx.x < kWave) {
+    const int bad = st.lag_parts ? fold_undefined(red, st.lag_parts) : 0;
+    if (threadIdx.x == 0) {
+      red.dtp[2] = p.dt;
+      red.dtp[3] = p.dt_h;
+      if (st.lag_parts) {
+        red.sums[2] = g;
+        red.status[1] = bad;
+      }
     }
   }
   return p;
@@ -603,7 +606,7 @@ __device__ __forceinline__ void step_epilogue(const FkReduce& red, int parts) {
     post(red, threadIdx.x, v);
   }
   if (threadIdx.x == 2) post(red, 4, (double)red.status[1]);
-  fold_limbs<kMNT>(red, parts);
+  fold_totals<kMNT>(red, parts);
 }
 
 /* ======================================================================= */
@@ -937,7 +940,7 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_mass_xy(
     fm.add(ms.s + ms.c);
     fe.add(es.s + es.c);
   }
-  publish_limbs<kMNT>(fm, fe, red);
+  publish_totals<kMNT>(fm, fe, red);
 }
 
 /* ======================================================================= */
@@ -1254,7 +1257,7 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_mass_yx(
     fm.add(ms.s + ms.c);
     fe.add(es.s + es.c);
   }
-  publish_limbs<kMNT>(fm, fe, red);
+  publish_totals<kMNT>(fm, fe, red);
 }
 
 

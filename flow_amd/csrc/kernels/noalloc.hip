@@ -27,7 +27,7 @@ constexpr int kMaxSide = 46335;
 constexpr size_t kInvBytes = align256(sizeof(double) * (kMaxSide + 5));
 constexpr size_t kOffInvX = kOffPair + 256;
 constexpr size_t kOffInvY = kOffInvX + kInvBytes;
-constexpr size_t kScratchBytes = kOffInvY + kInvBytes;  /* 1007616 B, < 1 MiB */
+constexpr size_t kScratchBytes = kOffInvY + kInvBytes;  /* 909312 B, < 1 MiB */
 static_assert(kScratchBytes < (1u << 20), "scratch stays below 1 MiB");
 
 constexpr int kMaxDevices = 64;

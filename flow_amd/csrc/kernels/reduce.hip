@@ -48,20 +48,19 @@ __global__ __launch_bounds__(kRedThreads) void k_timestep(
 }
 
 /* The (dt, dt_h) update from parts blocks' minima. */
-__global__ __launch_bounds__(kRedThreads) void k_finish_timestep(FkReduce r, int parts,
-                                                                 double max_dt,
-                                                                 int first_step) {
-  double g, bad;
-  fold_min<kRedThreads, false>(r, parts, max_dt, g, bad);
+__global__ __launch_bounds__(kWave) void k_finish_timestep(FkReduce r, int parts,
+                                                           double max_dt, int first_step) {
+  const double g = fold_min<false>(r, parts, max_dt);
+  const int bad = fold_undefined(r, parts);
   if (threadIdx.x == 0) {
     const DtPair p = next_pair(g, r.dtp[1], first_step);
     r.dtp[0] = p.dt;
     r.dtp[1] = p.dt_h;
     r.sums[2] = g;
-    r.status[1] = (int)bad;
+    r.status[1] = bad;
     post(r, 0, p.dt);
     post(r, 1, p.dt_h);
-    post(r, 4, bad);
+    post(r, 4, (double)bad);
   }
 }
 
@@ -243,7 +242,7 @@ int fk_reduce_blocks(void) { return kPartialsDoubles; }
 
 hipError_t fk_finish_timestep(FkReduce r, int parts, double max_dt, int first_step,
                               hipStream_t s) {
-  hipLaunchKernelGGL(k_finish_timestep, dim3(1), dim3(kRedThreads), 0, s, r, parts, max_dt,
+  hipLaunchKernelGGL(k_finish_timestep, dim3(1), dim3(kWave), 0, s, r, parts, max_dt,
                      first_step);
   return hipGetLastError();
 }

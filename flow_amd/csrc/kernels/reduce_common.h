@@ -16,10 +16,10 @@ namespace flowhip {
 constexpr int kMaxReduceBlocks = 2048;
 /* Layout of FkReduce.partials, in doubles: two per block of the kernel that
  * evaluates the CFL candidates (its minimum and its count of undefined
- * candidates), then 14 64-bit words per block of the kernel that leaves the
- * totals (block_limbs; the kernels with plain compensated sums use 4). */
+ * candidates), then 8 64-bit words per block of the kernel that leaves the
+ * totals (publish_totals; the kernels with plain compensated sums use 4). */
 constexpr int kTotalsOffset = 2 * kMaxReduceBlocks;
-constexpr int kTotalsWords = 14;
+constexpr int kTotalsWords = 8;
 constexpr int kPartialsDoubles = kTotalsOffset + kTotalsWords * kMaxReduceBlocks;
 
 template <int NT>
@@ -71,8 +71,8 @@ template <int NT>
 __device__ __forceinline__ void publish_min(double local_min, int nan_count, FkReduce r) {
   __shared__ int s_nan[NT / kWave];
   const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) nan_count += __shfl_xor(nan_count, off, kWave);
+  /* almost always none */
+  if (__ballot(nan_count != 0)) nan_count = wave_sum(nan_count);
   if (lane == 0) s_nan[w] = nan_count;
   const double bmin = block_min<NT>(local_min);
   if (threadIdx.x == 0) {
@@ -83,38 +83,24 @@ __device__ __forceinline__ void publish_min(double local_min, int nan_count, FkR
   }
 }
 
-/* The minimum over parts blocks' partials and max_dt, and the undefined
- * candidates' count; the same in every thread of the block. kSquared: the
- * candidates are squared time steps (the FP32-state form); the minimum's
+/* The minimum over parts blocks' partials and max_dt; the same in every
+ * thread. Each wave folds all of them for itself: no LDS, no barrier. kSquared:
+ * the candidates are squared time steps (the FP32-state form); the minimum's
  * square root is taken once, here. */
-template <int NT, bool kSquared>
-__device__ __forceinline__ void fold_min(const FkReduce& r, int parts, double max_dt,
-                                         double& g_out, double& bad_out) {
-  __shared__ double s_min[NT / kWave], s_bad[NT / kWave];
-  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
-  double g = kSquared ? max_dt * max_dt : max_dt, bad = 0.0;
-  for (int b = threadIdx.x; b < parts; b += NT) {
-    const double2 p = reinterpret_cast<const double2*>(r.partials)[b];
-    g = lesser(g, p.x);
-    bad += p.y;
-  }
+template <bool kSquared>
+__device__ __forceinline__ double fold_min(const FkReduce& r, int parts, double max_dt) {
+  double g = kSquared ? max_dt * max_dt : max_dt;
+#pragma unroll 4
+  for (int b = threadIdx.x % kWave; b < parts; b += kWave) g = lesser(g, r.partials[2 * b]);
   g = wave_min(g);
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) bad += __shfl_xor(bad, off, kWave);
-  if (lane == 0) {
-    s_min[w] = g;
-    s_bad[w] = bad;
-  }
-  __syncthreads();
-  g = s_min[0];
-  bad = s_bad[0];
-#pragma unroll
-  for (int k = 1; k < NT / kWave; ++k) {
-    g = lesser(g, s_min[k]);
-    bad += s_bad[k];
-  }
-  g_out = kSquared ? __builtin_sqrt(g) : g;
-  bad_out = bad;
+  return kSquared ? __builtin_sqrt(g) : g;
+}
+
+/* The undefined candidates of parts blocks, by one wave. */
+__device__ __forceinline__ int fold_undefined(const FkReduce& r, int parts) {
+  int bad = 0;
+  for (int b = threadIdx.x % kWave; b < parts; b += kWave) bad += (int)r.partials[2 * b + 1];
+  return wave_sum(bad);
 }
 
 /* The (dt, dt_h) update of omp3/flow.c:103-105 from the grid minimum g. */
@@ -154,30 +140,17 @@ struct FixSum {
   unsigned int bad;
 
   __host__ __device__ void add(double v) {
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    const unsigned int E = (unsigned int)(u >> 52) & 0x7ffu;
-    if (E >= 1023u + 127u) { /* |v| >= 2^127, inf or NaN */
-      bad = 1u;
+    const double mag = __builtin_fabs(v);
+    unsigned long long a0 = 0, a1 = 0, a2 = 0;
+    if (mag < 0x1p62) {
+      /* whole part and fraction, each converted exactly (bits of the
+       * fraction below 2^-64 are cut off) */
+      a1 = (unsigned long long)mag;
+      a0 = (unsigned long long)((mag - (double)a1) * 0x1p64);
+    } else if (!words(v, a0, a1, a2)) {
       return;
     }
-    const unsigned long long mant = u & 0xfffffffffffffull;
-    const unsigned long long M = E ? (mant | (1ull << 52)) : mant;
-    /* v = M 2^(s - 64) */
-    const int s = (E ? (int)E : 1) - 1075 + 64;
-    unsigned long long a0 = 0, a1 = 0, a2 = 0;
-    if (s < 0) {
-      a0 = s > -64 ? (M >> -s) : 0ull;
-    } else if (s < 64) {
-      a0 = M << s;
-      a1 = s ? (M >> (64 - s)) : 0ull;
-    } else if (s < 128) {
-      const int t = s - 64;
-      a1 = M << t;
-      a2 = t ? (M >> (64 - t)) : 0ull;
-    } else {
-      a2 = M << (s - 128); /* s <= 138: below 2^63 */
-    }
-    if (u >> 63) {
+    if (v < 0.0) {
       const unsigned long long b0 = w0 < a0;
       w0 -= a0;
       const unsigned long long t1 = w1 - a1, b1 = (w1 < a1) + (t1 < b0);
@@ -191,11 +164,50 @@ struct FixSum {
       w2 += a2 + c1a + (w1 < c0);
     }
   }
+
+  /* |v| >= 2^62 in units of 2^-64; false, and the sum marked bad, if it is
+   * out of range */
+  __host__ __device__ bool words(double v, unsigned long long& a0, unsigned long long& a1,
+                                 unsigned long long& a2) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned int E = (unsigned int)(u >> 52) & 0x7ffu;
+    if (E >= 1023u + 127u) { /* |v| >= 2^127, inf or NaN */
+      bad = 1u;
+      return false;
+    }
+    const unsigned long long M = (u & 0xfffffffffffffull) | (1ull << 52);
+    const int s = (int)E - 1075 + 64; /* |v| = M 2^(s - 64), 73 <= s <= 138 */
+    if (s < 128) {
+      const int t = s - 64;
+      a1 = M << t;
+      a2 = M >> (64 - t);
+    } else {
+      a2 = M << (s - 128);
+    }
+    return true;
+  }
 };
 
-__device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long x) {
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) x += __shfl_xor(x, off, kWave);
+/* a += b, modulo 2^192 */
+struct Words192 {
+  unsigned long long w0, w1, w2;
+};
+__host__ __device__ __forceinline__ void add192(Words192& a, const Words192& b) {
+  a.w0 += b.w0;
+  const unsigned long long c0 = a.w0 < b.w0;
+  const unsigned long long t = a.w1 + b.w1;
+  const unsigned long long c1 = t < b.w1;
+  a.w1 = t + c0;
+  a.w2 += b.w2 + c1 + (a.w1 < c0);
+}
+
+/* The sum over the wave (all lanes active), valid in lane 63. */
+__device__ __forceinline__ Words192 wave_sum192(Words192 x) {
+#define FLOWHIP_ADD_STEP(ctrl, rows)                                              \
+  add192(x, Words192{dpp_step<ctrl, rows>(0ull, x.w0), dpp_step<ctrl, rows>(0ull, x.w1), \
+                     dpp_step<ctrl, rows>(0ull, x.w2)});
+  FLOWHIP_DPP_STEPS(FLOWHIP_ADD_STEP)
+#undef FLOWHIP_ADD_STEP
   return x;
 }
 
@@ -227,32 +239,39 @@ __host__ __device__ inline double fixed_total(const unsigned long long* t) {
   return neg ? -r : r;
 }
 
-/* Per-lane exact totals (rho in fm, rho * e in fe) -> the block's 14 words:
- * the sums of its lanes' 32-bit limbs (integer sums, in any order) and of
- * the bad marks, mass first. */
+/* Per-lane exact totals (rho in fm, rho * e in fe) -> the block's 8 words:
+ * mass, its bad mark, energy, its bad mark. Integer addition is associative,
+ * so the totals are the same bits whichever waves and blocks added which
+ * values. (As 14 sums of 32-bit limbs through shuffles this took 7800
+ * cycles, a quarter of the mass/energy march of a 512^2 mesh.) */
 template <int NT>
-__device__ void publish_limbs(const FixSum& fm, const FixSum& fe, FkReduce r) {
-  __shared__ unsigned long long part[NT / kWave][kTotalsWords];
+__device__ void publish_totals(const FixSum& fm, const FixSum& fe, FkReduce r) {
+  __shared__ Words192 part[NT / kWave][2];
+  __shared__ unsigned int s_bad[NT / kWave][2];
   const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
-  const FixSum* f[2] = {&fm, &fe};
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const unsigned long long limb[7] = {
-        f[q]->w0 & 0xffffffffull, f[q]->w0 >> 32, f[q]->w1 & 0xffffffffull,
-        f[q]->w1 >> 32,           f[q]->w2 & 0xffffffffull, f[q]->w2 >> 32,
-        (unsigned long long)f[q]->bad};
-#pragma unroll
-    for (int k = 0; k < 7; ++k) {
-      const unsigned long long v = wave_sum_u64(limb[k]);
-      if (lane == 0) part[w][7 * q + k] = v;
-    }
+  const Words192 m = wave_sum192(Words192{fm.w0, fm.w1, fm.w2});
+  const Words192 e = wave_sum192(Words192{fe.w0, fe.w1, fe.w2});
+  const bool bm = __ballot(fm.bad != 0u) != 0ull, be = __ballot(fe.bad != 0u) != 0ull;
+  if (lane == kWave - 1) {
+    part[w][0] = m;
+    part[w][1] = e;
+    s_bad[w][0] = bm;
+    s_bad[w][1] = be;
   }
   __syncthreads();
-  if (threadIdx.x < kTotalsWords) {
-    unsigned long long v = 0;
-    for (int b = 0; b < NT / kWave; ++b) v += part[b][threadIdx.x];
-    unsigned long long* p = (unsigned long long*)(r.partials + kTotalsOffset);
-    p[kTotalsWords * blockIdx.x + threadIdx.x] = v;
+  if (threadIdx.x < 2) {
+    Words192 t = part[0][threadIdx.x];
+    unsigned int bad = s_bad[0][threadIdx.x];
+    for (int k = 1; k < NT / kWave; ++k) {
+      add192(t, part[k][threadIdx.x]);
+      bad |= s_bad[k][threadIdx.x];
+    }
+    unsigned long long* p = (unsigned long long*)(r.partials + kTotalsOffset) +
+                            kTotalsWords * blockIdx.x + 4 * threadIdx.x;
+    p[0] = t.w0;
+    p[1] = t.w1;
+    p[2] = t.w2;
+    p[3] = bad;
   }
 }
 
@@ -262,33 +281,45 @@ __device__ __forceinline__ void post(const FkReduce& r, int k, double v) {
   if (r.mail) r.mail[k] = v;
 }
 
-/* The totals of parts blocks' words -> r.sums[0..1], by one block. Thread
- * t < 252 adds word t % 14 of every 18th block, so a wave reads consecutive
- * words. The totals are the same bits whichever waves and blocks added
- * which values. */
+/* The totals of parts blocks' words -> r.sums[0..1], by one block: its first
+ * half the mass, its second the energy. */
 template <int NT>
-__device__ void fold_limbs(const FkReduce& r, int parts) {
-  constexpr int kSlices = NT / kTotalsWords;
-  __shared__ unsigned long long s_sum[kSlices][kTotalsWords];
-  const unsigned long long* p = (const unsigned long long*)(r.partials + kTotalsOffset);
-  const int slice = threadIdx.x / kTotalsWords, word = threadIdx.x % kTotalsWords;
-  if (slice < kSlices) {
-    unsigned long long v = 0;
-#pragma unroll 4
-    for (int b = slice; b < parts; b += kSlices) v += p[kTotalsWords * b + word];
-    s_sum[slice][word] = v;
+__device__ void fold_totals(const FkReduce& r, int parts) {
+  constexpr int kHalf = NT / 2;
+  __shared__ Words192 s_sum[NT / kWave];
+  __shared__ unsigned int s_bad[NT / kWave];
+  const int q = threadIdx.x / kHalf, lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
+  const unsigned long long* p =
+      (const unsigned long long*)(r.partials + kTotalsOffset) + 4 * q;
+  Words192 t{0, 0, 0};
+  unsigned long long any = 0;
+#pragma unroll 2
+  for (int b = threadIdx.x % kHalf; b < parts; b += kHalf) {
+    const unsigned long long* v = p + kTotalsWords * b;
+    add192(t, Words192{v[0], v[1], v[2]});
+    any |= v[3];
+  }
+  t = wave_sum192(t);
+  const bool bad = __ballot(any != 0ull) != 0ull;
+  if (lane == kWave - 1) {
+    s_sum[w] = t;
+    s_bad[w] = bad;
   }
   __syncthreads();
-  if (threadIdx.x < kTotalsWords) {
-    unsigned long long v = 0;
-    for (int k = 0; k < kSlices; ++k) v += s_sum[k][threadIdx.x];
-    s_sum[0][threadIdx.x] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < 2) {
-    const double v = fixed_total(&s_sum[0][7 * threadIdx.x]);
-    r.sums[threadIdx.x] = v;
-    post(r, 2 + threadIdx.x, v);
+  if (threadIdx.x % kHalf == 0) {
+    constexpr int kPer = kHalf / kWave;
+    Words192 s = s_sum[q * kPer];
+    unsigned int b = s_bad[q * kPer];
+    for (int k = 1; k < kPer; ++k) {
+      add192(s, s_sum[q * kPer + k]);
+      b |= s_bad[q * kPer + k];
+    }
+    const unsigned long long limb[7] = {
+        s.w0 & 0xffffffffull, s.w0 >> 32, s.w1 & 0xffffffffull, s.w1 >> 32,
+        s.w2 & 0xffffffffull, s.w2 >> 32, (unsigned long long)b};
+    const double v = fixed_total(limb);
+    r.sums[q] = v;
+    post(r, 2 + q, v);
   }
 }
 

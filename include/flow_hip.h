@@ -169,7 +169,7 @@ int flowhip_ensemble_run(FlowHipEnsemble* ens, int niters, int tt0,
  * print_conservation prints) in *mass and *energy (either may be NULL).
  * It calls no hipMalloc, hipFree or other allocating routine and creates no
  * per-Mesh state: its scratch (reduction partials, counters, dt pair,
- * totals, reciprocal spacings) is one static device array of 1007616 bytes
+ * totals, reciprocal spacings) is one static device array of 909312 bytes
  * per GPU, held until the process ends. Meshes up to FLOWHIP_MAX_CELLS_SIDE
  * interior cells a side; the CFL rule is FLOWHIP_CFL_DEFINED. Reads
  * mesh->dt and dt_h, writes the next pair into them (as solve_hydro_2d
