@@ -91,6 +91,7 @@ static void ens_build_work(FlowHipEnsemble* E) {
   for (int i = 0; i < n; ++i) {
     FkEnsInst* in = &E->h_insts[i];
     in->nstrips = (E->gnx[i] + W - 1) / W;
+    in->strip_inv = fk_strip_inverse(in->nstrips);
     in->nchunks = (E->gny[i] + H - 1) / H;
     in->nitems = in->nstrips * in->nchunks;
     in->item0 = total;

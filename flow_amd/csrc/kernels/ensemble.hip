@@ -61,6 +61,7 @@ __device__ __forceinline__ MarchList ens_list(const FkEnsInst& in, int H) {
   ml.nstrips = in.nstrips;
   ml.nchunks = in.nchunks;
   ml.nitems = in.nitems;
+  ml.inv = in.strip_inv;
   return ml;
 }
 
@@ -90,12 +91,11 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_lagrangian(
      * uniform-geometry form in FP64 only (0.3% faster there, 1% slower in
      * FP32, where the per-row reciprocals are cheap) */
     constexpr bool kUni = UNI && sizeof(T) == 8;
-    if (!item_edge(ml, g.nx, g.ny, wi.y))
-      lagrangian_item<T, P2, 0, false, kUni>(g, io, dt, dt_h, ml, wi.y, lane, local_min,
-                                             nan_count);
+    const ItemBox b = item_box(ml, g.nx, g.ny, wi.y);
+    if (!box_edge(b, g.nx, g.ny))
+      lagrangian_box<T, P2, 0, false, kUni>(g, io, dt, dt_h, b, lane, local_min, nan_count);
     else
-      lagrangian_item<T, P2, -1, true, kUni>(g, io, dt, dt_h, ml, wi.y, lane, local_min,
-                                             nan_count);
+      lagrangian_box<T, P2, -1, true, kUni>(g, io, dt, dt_h, b, lane, local_min, nan_count);
     local_min = wave_min(local_min);
     nan_count = wave_sum(nan_count);
     if (lane == 0) {
@@ -122,17 +122,18 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_mass(
     CSum ms{0.0, 0.0}, es{0.0, 0.0};
     const MGeo<T> g = ens_geo<T>(in);
     const MarchList ml = ens_list(in, H);
-    const bool edge = item_edge(ml, g.nx, g.ny, wi.y);
+    const ItemBox b = item_box(ml, g.nx, g.ny, wi.y);
+    const bool edge = box_edge(b, g.nx, g.ny);
     if (tt % 2 == 0) {
       if (edge)
-        mass_xy_item<T, P2, true, UNI>(g, io, dt, dt_h, ml, wi.y, lane, ms, es);
+        mass_xy_box<T, P2, true, UNI>(g, io, dt, dt_h, b, lane, ms, es);
       else
-        mass_xy_item<T, P2, false, UNI>(g, io, dt, dt_h, ml, wi.y, lane, ms, es);
+        mass_xy_box<T, P2, false, UNI>(g, io, dt, dt_h, b, lane, ms, es);
     } else {
       if (edge)
-        mass_yx_item<T, P2, true, UNI>(g, io, dt, dt_h, ml, wi.y, lane, ms, es);
+        mass_yx_box<T, P2, true, UNI>(g, io, dt, dt_h, b, lane, ms, es);
       else
-        mass_yx_item<T, P2, false, UNI>(g, io, dt, dt_h, ml, wi.y, lane, ms, es);
+        mass_yx_box<T, P2, false, UNI>(g, io, dt, dt_h, b, lane, ms, es);
     }
     ms = wave_csum(ms);
     es = wave_csum(es);
@@ -203,17 +204,18 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_momentum_xy(
                         arr<T>(in, kU),   arr<T>(in, kV)};
     const MGeo<T> g = ens_geo<T>(in);
     const MarchList ml = ens_list(in, H);
-    const bool edge = item_edge(ml, g.nx, g.ny, wi.y);
+    const ItemBox b = item_box(ml, g.nx, g.ny, wi.y);
+    const bool edge = box_edge(b, g.nx, g.ny);
     if (tt % 2) {
       if (edge)
-        momxy_xy_item<T, P2, -1, true, UNI>(g, io, dt, dt_h, ml, wi.y, lane);
+        momxy_xy_box<T, P2, -1, true, UNI>(g, io, dt, dt_h, b, lane);
       else
-        momxy_xy_item<T, P2, 0, false, UNI>(g, io, dt, dt_h, ml, wi.y, lane);
+        momxy_xy_box<T, P2, 0, false, UNI>(g, io, dt, dt_h, b, lane);
     } else {
       if (edge)
-        momxy_yx_item<T, P2, -1, true, UNI>(g, io, dt, dt_h, ml, wi.y, lane);
+        momxy_yx_box<T, P2, -1, true, UNI>(g, io, dt, dt_h, b, lane);
       else
-        momxy_yx_item<T, P2, 0, false, UNI>(g, io, dt, dt_h, ml, wi.y, lane);
+        momxy_yx_box<T, P2, 0, false, UNI>(g, io, dt, dt_h, b, lane);
     }
   }
 }
@@ -231,10 +233,9 @@ __global__ __launch_bounds__(kMNT) void k_ens_timestep(
     const FkEnsInst& in = insts[wi.x];
     const MGeo<T> g = ens_geo<T>(in);
     const int nx = in.nx, ny = in.ny;
-    const int strip = wi.y % in.nstrips, chunk = wi.y / in.nstrips;
-    const int x0 = kPad + strip * kEnsW, x1 = min(x0 + kEnsW, nx - kPad);
-    const int y0 = kPad + chunk * H, y1 = min(y0 + H, ny - kPad);
-    const int j = x0 + lane;
+    const ItemBox b = item_box(ens_list(in, H), nx, ny, wi.y);
+    const int x1 = b.x1, y0 = b.y0, y1 = b.y1;
+    const int j = b.x0 + lane;
     const T *e = arr<T>(in, kE), *qxx = arr<T>(in, kQxx), *qyy = arr<T>(in, kQyy),
             *rho = arr<T>(in, kRho);
     double local_min = in.max_dt;
@@ -404,6 +405,8 @@ using namespace flowhip;
 extern "C" {
 
 int fk_ens_strip_width(void) { return kEnsW; }
+
+unsigned long long fk_strip_inverse(int nstrips) { return strip_inverse(nstrips); }
 
 /* The single-mesh rule for chunk heights (march.hip) on the cells of the whole
  * ensemble, with one height for all stages (prologue 4.5 rows, at most the 20

@@ -117,7 +117,16 @@ constexpr int kMassPairWaves = sizeof(T) == 8 ? 2 : FLOWHIP_MASS_PAIR_WAVES;
 struct MarchList {
   int W, H;           /* strip width (output columns), chunk height (rows) */
   int nstrips, nchunks, nitems;
+  unsigned long long inv; /* strip_inverse(nstrips) */
 };
+
+/* item / nstrips as (item * inv) >> 40, two scalar multiplies for a division
+ * of some thirty vector operations: with inv = floor(2^40 / n) + 1 the quotient
+ * is exact while item * n < 2^40 (a mesh of 46335 columns has 800 strips and
+ * fewer than 2^25 items). */
+inline __host__ __device__ unsigned long long strip_inverse(int nstrips) {
+  return (1ull << 40) / (unsigned int)nstrips + 1ull;
+}
 
 /* Columns and rows of one item. */
 struct ItemBox {
@@ -125,7 +134,8 @@ struct ItemBox {
 };
 
 __device__ __forceinline__ ItemBox item_box(const MarchList& ml, int nx, int ny, int item) {
-  const int chunk = item / ml.nstrips, strip = item - chunk * ml.nstrips;
+  const int chunk = (int)(((unsigned long long)item * ml.inv) >> 40);
+  const int strip = item - chunk * ml.nstrips;
   ItemBox b;
   b.x0 = kPad + strip * ml.W;
   b.x1 = min(b.x0 + ml.W, nx - kPad);
@@ -210,14 +220,14 @@ template <bool UNIFORM>
 struct MarchQueue {
   unsigned int* ctr;
   int lo, end, waves, head;
-  /* the queue of block blk of nblk marching blocks, on set `stage` */
+  /* the queue of block blk of nblk marching blocks (a multiple of the bands,
+   * march_grid), on set `stage` */
   __device__ MarchQueue(unsigned int* queue, int stage, int nitems, int blk, int nblk) {
-    const int bands = nblk < kMarchBands ? nblk : kMarchBands;
-    const int band = blk % bands, local = blk / bands;
+    const int band = blk % kMarchBands, local = blk / kMarchBands;
     ctr = queue + stage * kQueueSet + band * kQueueStride;
-    lo = (int)((long)band * nitems / bands);
-    end = (int)((long)(band + 1) * nitems / bands);
-    waves = (nblk - band + bands - 1) / bands * kMWaves;
+    lo = (int)(((long)band * nitems) / kMarchBands);
+    end = (int)(((long)(band + 1) * nitems) / kMarchBands);
+    waves = nblk / kMarchBands * kMWaves;
     head = lo + local * kMWaves;
   }
   /* the wave's first item (end or beyond: none) */
@@ -274,6 +284,7 @@ inline MarchList make_march(int nx, int ny, int W, int H) {
   m.nstrips = (nx - 2 * kPad + W - 1) / W;
   m.nchunks = (ny - 2 * kPad + H - 1) / H;
   m.nitems = m.nstrips * m.nchunks;
+  m.inv = strip_inverse(m.nstrips);
   return m;
 }
 
@@ -314,20 +325,18 @@ __device__ __forceinline__ T dn(T v, int d) {
 }
 
 
-/* Whether a work item's strip lies within three columns of a wall, where
- * some of its lanes are ghost columns. */
-__device__ __forceinline__ bool item_xedge(const MarchList& ml, int nx, int item) {
-  const int x0 = kPad + (item % ml.nstrips) * ml.W, x1 = min(x0 + ml.W, nx - kPad);
-  return (x0 - 3 < kPad) || (x1 + 3 > nx - kPad);
+/* Whether an item's strip lies within three columns of a wall, where some of
+ * its lanes are ghost columns. */
+__device__ __forceinline__ bool box_xedge(const ItemBox& b, int nx) {
+  return (b.x0 - 3 < kPad) || (b.x1 + 3 > nx - kPad);
 }
 
 /* Whether an item's stencils reach a ghost row or column anywhere (the
  * x test above, or a chunk within three rows of a north/south wall); the
  * other items, all but the mesh's outer ring of items, run the
  * straight-line interior form of their kernel. */
-__device__ __forceinline__ bool item_edge(const MarchList& ml, int nx, int ny, int item) {
-  const ItemBox b = item_box(ml, nx, ny, item);
-  return item_xedge(ml, nx, item) || (b.y0 < kPad + 3) || (b.y1 + 3 > ny - kPad);
+__device__ __forceinline__ bool box_edge(const ItemBox& b, int nx, int ny) {
+  return box_xedge(b, nx) || (b.y0 < kPad + 3) || (b.y1 + 3 > ny - kPad);
 }
 
 /* ---- per-row geometry of a chunk held across the lanes ----
@@ -338,7 +347,7 @@ constexpr int kMaxChunkRows = 120;
 /* Least height the rules choose: the x stage of the momentum march at a
  * chunk that starts two rows above the south wall reads a ghost row as its
  * mirror, and at one row above it the Lagrangian's first y face would be a
- * ghost face (item_edge). */
+ * ghost face (box_edge). */
 constexpr int kMinChunkRows = 2;
 
 __device__ __forceinline__ double lane_value(double v, int k) {
@@ -753,13 +762,6 @@ __device__ __forceinline__ void mass_xy_box(const MGeo<T>& g, const MMassIO<T>& 
   }
 }
 
-template <typename T, bool P2, bool EDGE = true, bool UNI = false, typename Acc = CSum>
-__device__ __forceinline__ void mass_xy_item(const MGeo<T>& g, const MMassIO<T>& io, T dt,
-                                             T dt_h, const MarchList& ml, int item, int lane,
-                                             Acc& ms, Acc& es) {
-  mass_xy_box<T, P2, EDGE, UNI, Acc>(g, io, dt, dt_h, item_box(ml, g.nx, g.ny, item), lane, ms, es);
-}
-
 /* The x-first mass/energy march of an interior item, two columns per lane
  * (mass_xy_box's interior form, column by column). */
 template <typename T, bool P2, bool UNI, typename Acc>
@@ -922,9 +924,10 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_mass_xy(
   MarchQueue<true> mq(red.queue, kStageMass, ml.nitems, blockIdx.x, gridDim.x);
   for (int item = mq.first(); item < mq.end; item = mq.next()) {
     ItemSum<T> ms{0.0, 0.0}, es{0.0, 0.0};
+    const ItemBox b = item_box(ml, g.nx, g.ny, item);
+    const bool edge = box_edge(b, g.nx, g.ny);
     if constexpr (PAIR) {
-      const ItemBox b = item_box(ml, g.nx, g.ny, item);
-      if (item_edge(ml, g.nx, g.ny, item)) {
+      if (edge) {
         for (int sx0 = b.x0; sx0 < b.x1; sx0 += kMassW) {
           const ItemBox sb{sx0, min(sx0 + kMassW, b.x1), b.y0, b.y1};
           mass_xy_box<T, P2, true, UNI, ItemSum<T>>(g, io, dt, dt_h, sb, lane, ms, es);
@@ -932,10 +935,10 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_mass_xy(
       } else {
         mass_xy_pair<T, P2, UNI>(g, io, dt, dt_h, b, lane, ms, es);
       }
-    } else if (item_edge(ml, g.nx, g.ny, item)) {
-      mass_xy_item<T, P2, true, UNI>(g, io, dt, dt_h, ml, item, lane, ms, es);
+    } else if (edge) {
+      mass_xy_box<T, P2, true, UNI>(g, io, dt, dt_h, b, lane, ms, es);
     } else {
-      mass_xy_item<T, P2, false, UNI>(g, io, dt, dt_h, ml, item, lane, ms, es);
+      mass_xy_box<T, P2, false, UNI>(g, io, dt, dt_h, b, lane, ms, es);
     }
     fm.add(ms.s + ms.c);
     fe.add(es.s + es.c);
@@ -1066,13 +1069,6 @@ __device__ __forceinline__ void mass_yx_box(const MGeo<T>& g, const MMassIO<T>& 
     wv[0] = wv[1];
     wv[1] = wv[2];
   }
-}
-
-template <typename T, bool P2, bool EDGE = true, bool UNI = false, typename Acc = CSum>
-__device__ __forceinline__ void mass_yx_item(const MGeo<T>& g, const MMassIO<T>& io, T dt,
-                                             T dt_h, const MarchList& ml, int item, int lane,
-                                             Acc& ms, Acc& es) {
-  mass_yx_box<T, P2, EDGE, UNI, Acc>(g, io, dt, dt_h, item_box(ml, g.nx, g.ny, item), lane, ms, es);
 }
 
 /* The y-first mass/energy march of an interior item, two columns per lane
@@ -1239,9 +1235,10 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_mass_yx(
   MarchQueue<true> mq(red.queue, kStageMass, ml.nitems, blockIdx.x, gridDim.x);
   for (int item = mq.first(); item < mq.end; item = mq.next()) {
     ItemSum<T> ms{0.0, 0.0}, es{0.0, 0.0};
+    const ItemBox b = item_box(ml, g.nx, g.ny, item);
+    const bool edge = box_edge(b, g.nx, g.ny);
     if constexpr (PAIR) {
-      const ItemBox b = item_box(ml, g.nx, g.ny, item);
-      if (item_edge(ml, g.nx, g.ny, item)) {
+      if (edge) {
         for (int sx0 = b.x0; sx0 < b.x1; sx0 += kMassW) {
           const ItemBox sb{sx0, min(sx0 + kMassW, b.x1), b.y0, b.y1};
           mass_yx_box<T, P2, true, UNI, ItemSum<T>>(g, io, dt, dt_h, sb, lane, ms, es);
@@ -1249,10 +1246,10 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_mass_yx(
       } else {
         mass_yx_pair<T, P2, UNI>(g, io, dt, dt_h, b, lane, ms, es);
       }
-    } else if (item_edge(ml, g.nx, g.ny, item)) {
-      mass_yx_item<T, P2, true, UNI>(g, io, dt, dt_h, ml, item, lane, ms, es);
+    } else if (edge) {
+      mass_yx_box<T, P2, true, UNI>(g, io, dt, dt_h, b, lane, ms, es);
     } else {
-      mass_yx_item<T, P2, false, UNI>(g, io, dt, dt_h, ml, item, lane, ms, es);
+      mass_yx_box<T, P2, false, UNI>(g, io, dt, dt_h, b, lane, ms, es);
     }
     fm.add(ms.s + ms.c);
     fe.add(es.s + es.c);
@@ -1780,7 +1777,7 @@ struct MLagIO {
  * i+3 computed this step), Qyy on cell rows i and i+1 and v after the
  * viscous acceleration on faces i and i+1. Ghost faces hold the negated
  * mirror (INVERT_X / INVERT_Y), ghost Q cells the mirror cell.
- * EDGE = false is the interior form, for items that item_edge clears: no
+ * EDGE = false is the interior form, for items that box_edge clears: no
  * ghost store, mirror or wall test is compiled, so each row is one
  * straight-line block. */
 template <typename T, bool P2, int XE = -1, bool EDGE = true, bool UNI = false>
@@ -2010,14 +2007,6 @@ __device__ __forceinline__ void lagrangian_box(const MGeo<T>& g, const MLagIO<T>
     wx[0] = wx[1];
     wx[1] = wx[2];
   }
-}
-
-template <typename T, bool P2, int XE = -1, bool EDGE = true, bool UNI = false>
-__device__ __forceinline__ void lagrangian_item(const MGeo<T>& g, const MLagIO<T>& io, T dt,
-                                                T dt_h, const MarchList& ml, int item,
-                                                int lane, double& local_min, int& nan_count) {
-  lagrangian_box<T, P2, XE, EDGE, UNI>(g, io, dt, dt_h, item_box(ml, g.nx, g.ny, item), lane,
-                                       local_min, nan_count);
 }
 
 /* ---- the Lagrangian march, two columns per lane (FP32 interior items) ----
@@ -2267,11 +2256,12 @@ void k_march_lagrangian(MGeo<T> g, MLagIO<T> io, FkReduce red, double max_dt, Ma
   for (int base = mq.first(); base < mq.end; base = mq.next()) {
     const int item = __builtin_amdgcn_readfirstlane(base + wave);
     if (item >= mq.end) continue;
+    const ItemBox b = item_box(ml, g.nx, g.ny, item);
+    const bool edge = box_edge(b, g.nx, g.ny);
     if constexpr (PAIR) {
       /* interior items two columns per lane; edge items in one-column
        * sub-strips */
-      const ItemBox b = item_box(ml, g.nx, g.ny, item);
-      if (!item_edge(ml, g.nx, g.ny, item)) {
+      if (!edge) {
         lagrangian_pair<T, P2, UNI>(g, io, dt, dt_h, b, lane, local_min, nan_count);
       } else {
         for (int sx0 = b.x0; sx0 < b.x1; sx0 += kLagW) {
@@ -2280,15 +2270,12 @@ void k_march_lagrangian(MGeo<T> g, MLagIO<T> io, FkReduce red, double max_dt, Ma
                                                nan_count);
         }
       }
-    } else if (!item_edge(ml, g.nx, g.ny, item)) {
-      lagrangian_item<T, P2, 0, false, UNI>(g, io, dt, dt_h, ml, item, lane, local_min,
-                                            nan_count);
-    } else if (item_xedge(ml, g.nx, item)) {
-      lagrangian_item<T, P2, 1, true, UNI>(g, io, dt, dt_h, ml, item, lane, local_min,
-                                           nan_count);
+    } else if (!edge) {
+      lagrangian_box<T, P2, 0, false, UNI>(g, io, dt, dt_h, b, lane, local_min, nan_count);
+    } else if (box_xedge(b, g.nx)) {
+      lagrangian_box<T, P2, 1, true, UNI>(g, io, dt, dt_h, b, lane, local_min, nan_count);
     } else {
-      lagrangian_item<T, P2, 0, true, UNI>(g, io, dt, dt_h, ml, item, lane, local_min,
-                                           nan_count);
+      lagrangian_box<T, P2, 0, true, UNI>(g, io, dt, dt_h, b, lane, local_min, nan_count);
     }
   }
   publish_min<kMNT>(local_min, nan_count, red);
@@ -2323,12 +2310,10 @@ struct MMom2IO {
  * stage's cell flux at x1 and u0 up to x1+2). The per-row arithmetic is the
  * two separate kernels', so the results are theirs bit for bit. */
 template <typename T, bool P2, int XE = -1, bool EDGE = true, bool UNI = false>
-__device__ __forceinline__ void momxy_xy_item(const MGeo<T>& g, const MMom2IO<T>& io,
-                                              T dt, T dt_h, const MarchList& ml,
-                                              int item, int lane) {
+__device__ __forceinline__ void momxy_xy_box(const MGeo<T>& g, const MMom2IO<T>& io, T dt,
+                                             T dt_h, const ItemBox box, int lane) {
   const int nx = g.nx, ny = g.ny, sx = nx + 1;
   (void)dt;
-  const ItemBox box = item_box(ml, nx, ny, item);
   const int x0 = box.x0, x1 = box.x1, y0 = box.y0, y1 = box.y1;
   const bool edge = EDGE && ((x0 == kPad) || (x1 + 3 > nx - kPad) || (y0 == kPad) ||
                              (y1 + 3 > ny - kPad));
@@ -2522,12 +2507,10 @@ __device__ __forceinline__ void momxy_xy_item(const MGeo<T>& g, const MMom2IO<T>
  * march; the y stage at row r reads u of rows r and r-1 from the x stage.
  * Lane l holds x face / column q = x0 - 3 + l (strips of 59 columns). */
 template <typename T, bool P2, int XE = -1, bool EDGE = true, bool UNI = false>
-__device__ __forceinline__ void momxy_yx_item(const MGeo<T>& g, const MMom2IO<T>& io,
-                                              T dt, T dt_h, const MarchList& ml,
-                                              int item, int lane) {
+__device__ __forceinline__ void momxy_yx_box(const MGeo<T>& g, const MMom2IO<T>& io, T dt,
+                                             T dt_h, const ItemBox box, int lane) {
   const int nx = g.nx, ny = g.ny, sx = nx + 1;
   (void)dt;
-  const ItemBox box = item_box(ml, nx, ny, item);
   const int x0 = box.x0, x1 = box.x1, y0 = box.y0, y1 = box.y1;
   const bool edge = EDGE && ((x0 == kPad) || (x1 + 3 > nx - kPad) || (y0 == kPad) ||
                              (y1 + 3 > ny - kPad));
@@ -2693,12 +2676,13 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_momxy_xy(
   for (int base = mq.first(); base < mq.end; base = mq.next()) {
     const int item = __builtin_amdgcn_readfirstlane(base + wave);
     if (item >= mq.end) continue;
-    if (!item_edge(ml, g.nx, g.ny, item))
-      momxy_xy_item<T, P2, 0, false, UNI>(g, io, dt, dt_h, ml, item, lane);
-    else if (item_xedge(ml, g.nx, item))
-      momxy_xy_item<T, P2, 1, true, UNI>(g, io, dt, dt_h, ml, item, lane);
+    const ItemBox b = item_box(ml, g.nx, g.ny, item);
+    if (!box_edge(b, g.nx, g.ny))
+      momxy_xy_box<T, P2, 0, false, UNI>(g, io, dt, dt_h, b, lane);
+    else if (box_xedge(b, g.nx))
+      momxy_xy_box<T, P2, 1, true, UNI>(g, io, dt, dt_h, b, lane);
     else
-      momxy_xy_item<T, P2, 0, true, UNI>(g, io, dt, dt_h, ml, item, lane);
+      momxy_xy_box<T, P2, 0, true, UNI>(g, io, dt, dt_h, b, lane);
   }
 }
 
@@ -2716,12 +2700,13 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_march_momxy_yx(
   for (int base = mq.first(); base < mq.end; base = mq.next()) {
     const int item = __builtin_amdgcn_readfirstlane(base + wave);
     if (item >= mq.end) continue;
-    if (!item_edge(ml, g.nx, g.ny, item))
-      momxy_yx_item<T, P2, 0, false, UNI>(g, io, dt, dt_h, ml, item, lane);
-    else if (item_xedge(ml, g.nx, item))
-      momxy_yx_item<T, P2, 1, true, UNI>(g, io, dt, dt_h, ml, item, lane);
+    const ItemBox b = item_box(ml, g.nx, g.ny, item);
+    if (!box_edge(b, g.nx, g.ny))
+      momxy_yx_box<T, P2, 0, false, UNI>(g, io, dt, dt_h, b, lane);
+    else if (box_xedge(b, g.nx))
+      momxy_yx_box<T, P2, 1, true, UNI>(g, io, dt, dt_h, b, lane);
     else
-      momxy_yx_item<T, P2, 0, true, UNI>(g, io, dt, dt_h, ml, item, lane);
+      momxy_yx_box<T, P2, 0, true, UNI>(g, io, dt, dt_h, b, lane);
   }
 }
 
@@ -2740,8 +2725,8 @@ inline int march_cus() {
   return cus;
 }
 
-/* Persistent grid of a march kernel: as many blocks as stay resident on the
- * device (per_cu per CU, from the occupancy query on first use, at most
+/* Persistent grid of a march kernel, a multiple of the bands: as many blocks
+ * as stay resident on the device (per_cu per CU, from the occupancy query on first use, at most
  * max_per_cu when that is positive), and no more than give every band a wave
  * for each of its items (a grid of nitems / kMWaves blocks left some bands an
  * item short of waves, and the launch took two rounds of items for one). */
@@ -2754,12 +2739,12 @@ int march_grid(K kernel, int& per_cu, int nitems, int max_per_cu = 0) {
        per_cu < 1))
     per_cu = 1;
   if (max_per_cu > 0 && per_cu > max_per_cu) per_cu = max_per_cu;
-  long gsz = (long)cus * per_cu;
+  long gsz = (long)cus * per_cu / kMarchBands * kMarchBands;
   const long band = (nitems + kMarchBands - 1) / kMarchBands;
   const long need = kMarchBands * ((band + kMWaves - 1) / kMWaves);
   if (gsz > need) gsz = need;
   if (gsz > kMaxReduceBlocks) gsz = kMaxReduceBlocks;
-  return gsz < 1 ? 1 : (int)gsz;
+  return gsz < kMarchBands ? kMarchBands : (int)gsz;
 }
 
 }  // namespace flowhip

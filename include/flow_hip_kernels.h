@@ -324,6 +324,7 @@ typedef struct FkEnsInst {
   double* dtp;             /* {dt, dt_h} of this instance (device) */
   double max_dt;
   int nstrips, nchunks, nitems;
+  unsigned long long strip_inv; /* fk_strip_inverse(nstrips) */
   int item0;               /* first partial slot of this instance */
 } FkEnsInst;
 
@@ -356,6 +357,8 @@ typedef struct FkEnsLaunch {
 
 /* Strip width of the ensemble work items. */
 int fk_ens_strip_width(void);
+/* The kernels' stand-in for a division by a number of strips. */
+unsigned long long fk_strip_inverse(int nstrips);
 /* Chunk height of an ensemble of so many interior cells, all instances. */
 int fk_ens_default_rows(double cells, int fp32);
 /* One step (omp3/flow.c:10-52) of every instance: Lagrangian stage, dt,
