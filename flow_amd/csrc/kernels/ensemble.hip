@@ -82,8 +82,7 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_lagrangian(
                        arr<T>(in, kUFx),   arr<T>(in, kUFy), arr<T>(in, kP),
                        arr<T>(in, kRhoOld)};
     const T dt = T(in.dtp[0]), dt_h = T(in.dtp[1]);
-    /* FP32 state: squared candidates (cell_timestep_sq) */
-    double local_min = std::is_same<T, float>::value ? in.max_dt * in.max_dt : in.max_dt;
+    double local_min = cfl_seed<T>(in.max_dt, in.dtp[1]);
     int nan_count = 0;
     const MGeo<T> g = ens_geo<T>(in);
     const MarchList ml = ens_list(in, H);

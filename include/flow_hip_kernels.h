@@ -76,7 +76,9 @@ typedef struct FkReduce {
                             launch leave for the launch that folds it */
   double* dtp;           /* {dt, dt_h}, then the pair the march schedule's
                             mass/energy kernel hands to the momentum kernel */
-  double* sums;          /* {mass, energy, unclamped min dt, spare} */
+  double* sums;          /* {mass, energy, grid minimum dt (the march kernels
+                            leave out candidates past the clamp C_M dt_h),
+                            spare} */
   int* status;           /* [1] undefined CFL candidates of the last dt
                             computation */
   /* FK_MARCH_QUEUE_WORDS words: a set of counters for each stage of a march
