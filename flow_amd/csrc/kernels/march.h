@@ -587,26 +587,24 @@ template <typename T>
 __device__ __forceinline__ DtPair mass_pair(const FkReduce& red, const MarchStep& st) {
   DtPair p{red.dtp[0], red.dtp[1]};
   if (blockIdx.x == 0) march_queue_reset(red.queue, kStageMass);
-  double g = 0.0;
+  MinFold m{0.0, 0};
   if (st.lag_parts) {
-    g = fold_min<std::is_same<T, float>::value>(red, st.lag_parts, st.max_dt);
-    p = next_pair(g, p.dt_h, st.first_step);
+    m = fold_min<std::is_same<T, float>::value>(red, st.lag_parts, st.max_dt);
+    p = next_pair(m.g, p.dt_h, st.first_step);
   }
-  if (blockIdx.x == 0 && threadIdx.x < kWave) {
-    const int bad = st.lag_parts ? fold_undefined(red, st.lag_parts) : 0;
-    if (threadIdx.x == 0) {
-      red.dtp[2] = p.dt;
-      red.dtp[3] = p.dt_h;
-      if (st.lag_parts) {
-        red.sums[2] = g;
-        red.status[1] = bad;
-      }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    red.dtp[2] = p.dt;
+    red.dtp[3] = p.dt_h;
+    if (st.lag_parts) {
+      red.sums[2] = m.g;
+      red.status[1] = m.bad;
     }
   }
   return p;
 }
 
-/* Block 0 of the momentum march; parts: blocks of the mass/energy march. */
+/* Block 0 of the momentum kernel (at least kMNT threads); parts: blocks of the
+ * mass/energy kernel. */
 __device__ __forceinline__ void step_epilogue(const FkReduce& red, int parts) {
   march_queue_reset(red.queue, kStageMom);
   if (threadIdx.x < 2) {
@@ -1764,6 +1762,46 @@ struct MLagIO {
   double* __restrict__ cfl; /* NULL, or every interior CFL candidate (FP64) */
 };
 
+/* dst = src at the ghost cells whose nearest interior cell is (i, j). */
+template <typename T>
+__device__ __forceinline__ void copy_ghosts(T* dst, const T* src, int nx, int ny, int i, int j) {
+  const int c = i * nx + j;
+  const bool w = (j == kPad), ea = (j == nx - kPad - 1);
+  const bool s = (i == kPad), no = (i == ny - kPad - 1);
+  for (int d = 1; d <= kPad; ++d) {
+    if (w) dst[c - d] = src[c - d];
+    if (ea) dst[c + d] = src[c + d];
+    if (s) dst[c - d * nx] = src[c - d * nx];
+    if (no) dst[c + d * nx] = src[c + d * nx];
+    for (int d2 = 1; d2 <= kPad; ++d2) {
+      if (s && w) dst[c - d * nx - d2] = src[c - d * nx - d2];
+      if (s && ea) dst[c - d * nx + d2] = src[c - d * nx + d2];
+      if (no && w) dst[c + d * nx - d2] = src[c + d * nx - d2];
+      if (no && ea) dst[c + d * nx + d2] = src[c + d * nx + d2];
+    }
+  }
+}
+
+/* Cell c's FP64 CFL candidate (squared in the FP32-state form) into the lane's
+ * minimum, unless it certainly cannot lower it (and none is dumped). */
+template <typename T>
+__device__ __forceinline__ void cfl_candidate(const MLagIO<T>& io, int c, T es, T qx, T qy, T rho,
+                                              T cdx, T cdy, double& local_min, int& nan_count) {
+  constexpr bool kSq = std::is_same<T, float>::value;
+  if (!io.cfl && cfl_above(double(es), double(qx), double(qy), double(rho), double(cdx),
+                           double(cdy), kSq ? local_min : local_min * local_min))
+    return;
+  const double cand = kSq ? cell_timestep_sq(double(es), double(qx), double(qy), double(rho),
+                                             double(cdx), double(cdy))
+                          : cell_timestep(double(es), double(qx), double(qy), double(rho),
+                                          double(cdx), double(cdy));
+  if (cand == cand)
+    local_min = lesser(local_min, cand);
+  else
+    ++nan_count;
+  if (io.cfl) io.cfl[c] = cand;
+}
+
 /* EOS, pressure acceleration, artificial viscosity, shock heating, the CFL
  * candidates and the copy of rho (omp3/flow.c:55-70, 110-290, 73-96,
  * 302-305). Lane l holds x face / cell column q = x0 - 3 + l (strips of 58
@@ -1957,38 +1995,8 @@ __device__ __forceinline__ void lagrangian_box(const MGeo<T>& g, const MLagIO<T>
                                         vav, cdx_q, cdy(i), dt_h, rcdx_q, rcdy(i));
       mput_cell(edge, io.e1, nx, ny, i, q, es);
       io.rho_old[c] = ri;
-      if (edge) {
-        const bool w = (q == kPad), ea = (q == nx - kPad - 1);
-        const bool s = (i == kPad), no = (i == ny - kPad - 1);
-        for (int d = 1; d <= kPad; ++d) {
-          if (w) io.rho_old[c - d] = io.rho[c - d];
-          if (ea) io.rho_old[c + d] = io.rho[c + d];
-          if (s) io.rho_old[c - d * nx] = io.rho[c - d * nx];
-          if (no) io.rho_old[c + d * nx] = io.rho[c + d * nx];
-          for (int d2 = 1; d2 <= kPad; ++d2) {
-            if (s && w) io.rho_old[c - d * nx - d2] = io.rho[c - d * nx - d2];
-            if (s && ea) io.rho_old[c - d * nx + d2] = io.rho[c - d * nx + d2];
-            if (no && w) io.rho_old[c + d * nx - d2] = io.rho[c + d * nx - d2];
-            if (no && ea) io.rho_old[c + d * nx + d2] = io.rho[c + d * nx + d2];
-          }
-        }
-      }
-      /* FP64 CFL candidate (squared in the FP32-state form), unless it
-       * certainly cannot lower the lane's minimum (and none is dumped) */
-      constexpr bool kSq = std::is_same<T, float>::value;
-      if (io.cfl || !cfl_above(double(es), double(qx), double(qy_prev), double(ri),
-                               double(cdx_q), double(cdy(i)),
-                               kSq ? local_min : local_min * local_min)) {
-        const double cand = kSq ? cell_timestep_sq(double(es), double(qx), double(qy_prev),
-                                                   double(ri), double(cdx_q), double(cdy(i)))
-                                : cell_timestep(double(es), double(qx), double(qy_prev),
-                                                double(ri), double(cdx_q), double(cdy(i)));
-        if (cand == cand)
-          local_min = lesser(local_min, cand);
-        else
-          ++nan_count;
-        if (io.cfl) io.cfl[c] = cand;
-      }
+      if (edge) copy_ghosts(io.rho_old, io.rho, nx, ny, i, q);
+      cfl_candidate<T>(io, c, es, qx, qy_prev, ri, cdx_q, cdy(i), local_min, nan_count);
     }
 
     /* advance the windows */

@@ -5,6 +5,7 @@
 #include <cmath>
 
 #include "march.h"
+#include "rows.h"
 
 namespace flowhip {
 
@@ -184,6 +185,78 @@ hipError_t launch_march_momxy_p(MGeo<T> g, MMom2IO<T> io, int tt, FkReduce r, in
   return hipGetLastError();
 }
 
+/* Blocks of a row-parallel kernel (rows.h): waves per block, 0 where the march
+ * is the faster form, and the items.
+ *
+ * The time of such a launch goes with the waves on the fullest CU: blocks of n
+ * waves own n - halo rows, so tall blocks compute fewer halo rows twice and low
+ * ones divide more evenly. n is the one of 8 to 16 that leaves that CU the
+ * fewest waves (6 and 7 were no faster at 64^2). Measured on MI355X (us a
+ * step, FP64; FP32), blocks of 16 and then this rule: 64^2 21.9 -> 17.9; 18.3
+ * -> 15.9, 300x200 26.5 -> 23.8; 20.2 -> 19.1, 512^2 42.7 -> 40.8; 31.6 -> 30.4.
+ *
+ * Above 48 waves on that CU the march takes over: its chunks then have rows
+ * enough to pay for their prologue, and it computes no halo row twice. Rows
+ * against march at 30 to 48 waves (512^2, 3000x150, and mass/energy and
+ * momentum at 700^2): 7 to 22% faster; at 56 (the Lagrangian at 700^2) 7%
+ * slower in FP64 and 3% faster in FP32; at 75 to 112 (1000^2) 2 to 18% slower.
+ * A given chunk height asks for the march. */
+constexpr int kRowsMostWaves = 48;
+
+struct RowsGrid {
+  int waves;
+  MarchList ml;
+};
+inline RowsGrid rows_grid(int nx, int ny, int chunk_rows, int W, int halo) {
+  RowsGrid best{0, {}};
+  if (chunk_rows > 0) return best;
+  long least = kRowsMostWaves + 1;
+  for (int nw = kRowsMinWaves; nw <= kRowsMaxWaves; ++nw) {
+    const MarchList ml = make_march(nx, ny, W, nw - halo);
+    const long waves = (long)nw * ((ml.nitems + march_cus() - 1) / march_cus());
+    if (ml.nitems < 1 || ml.nitems > kMaxReduceBlocks || waves >= least) continue;
+    best = RowsGrid{nw, ml};
+    least = waves;
+  }
+  return best;
+}
+
+template <typename T, bool P2, bool UNI>
+hipError_t launch_rows_lagrangian(const RowsGrid& rg, MGeo<T> g, MLagIO<T> io, FkReduce r,
+                                  double max_dt, int* parts, hipStream_t s) {
+  if (!r.queue) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((k_rows_lagrangian<T, P2, UNI>), dim3(rg.ml.nitems),
+                     dim3(rg.waves * kWave), 0, s, g, io, r, max_dt, rg.ml);
+  *parts = rg.ml.nitems;
+  return hipGetLastError();
+}
+
+template <typename T, bool P2, bool UNI>
+hipError_t launch_rows_mass(const RowsGrid& rg, MGeo<T> g, MMassIO<T> io, int tt, FkReduce r,
+                            MarchStep st, int* parts, hipStream_t s) {
+  if (!r.queue) return hipErrorInvalidValue;
+  const dim3 grid(rg.ml.nitems), block(rg.waves * kWave);
+  if (tt % 2 == 0)
+    hipLaunchKernelGGL((k_rows_mass_xy<T, P2, UNI>), grid, block, 0, s, g, io, r, st, rg.ml);
+  else
+    hipLaunchKernelGGL((k_rows_mass_yx<T, P2, UNI>), grid, block, 0, s, g, io, r, st, rg.ml);
+  *parts = rg.ml.nitems;
+  return hipGetLastError();
+}
+
+template <typename T, bool P2, bool UNI>
+hipError_t launch_rows_momxy(const RowsGrid& rg, MGeo<T> g, MMom2IO<T> io, int tt, FkReduce r,
+                             int parts, hipStream_t s) {
+  if (!r.queue) return hipErrorInvalidValue;
+  /* one block more, for the step's epilogue */
+  const dim3 grid(rg.ml.nitems + 1), block(rg.waves * kWave);
+  if (tt % 2)
+    hipLaunchKernelGGL((k_rows_momxy_xy<T, P2, UNI>), grid, block, 0, s, g, io, r, parts, rg.ml);
+  else
+    hipLaunchKernelGGL((k_rows_momxy_yx<T, P2, UNI>), grid, block, 0, s, g, io, r, parts, rg.ml);
+  return hipGetLastError();
+}
+
 /* Dispatch on whether every mesh spacing is a power of two (quotients by
  * spacings become products with exact reciprocals) and whether the mesh is
  * uniform (MUni): launch<P2, UNI>. */
@@ -201,6 +274,13 @@ hipError_t launch_march_mass(MGeo<T> g, MMassIO<T> io, int tt, FkReduce r, March
                              hipStream_t s) {
   if (pairs_wanted(pairs, g.nx, g.ny) && pow2 && uniform && pairs_fit(g, io))
     return launch_march_mass_p<T, true, true, true>(g, io, tt, r, st, parts, chunk_rows, s);
+  const RowsGrid rg = rows_grid(g.nx, g.ny, chunk_rows, kMassW,
+                                tt % 2 ? kRowsMassYXHalo : kRowsMassXYHalo);
+  if (rg.waves)
+    return by_geometry(pow2, uniform, [&](auto p2, auto uni) {
+      return launch_rows_mass<T, decltype(p2)::value, decltype(uni)::value>(
+          rg, g, io, tt, r, st, parts, s);
+    });
   return by_geometry(pow2, uniform, [&](auto p2, auto uni) {
     return launch_march_mass_p<T, decltype(p2)::value, decltype(uni)::value>(
         g, io, tt, r, st, parts, chunk_rows, s);
@@ -214,6 +294,12 @@ hipError_t launch_march_lagrangian(MGeo<T> g, MLagIO<T> io, FkReduce r, double m
   if (pairs_wanted(pairs, g.nx, g.ny) && pow2 && uniform && lag_pairs_fit(g, io))
     return launch_march_lagrangian_p<T, true, true, true>(g, io, r, max_dt, parts,
                                                           chunk_rows, s);
+  const RowsGrid rg = rows_grid(g.nx, g.ny, chunk_rows, kLagW, kRowsLagHalo);
+  if (rg.waves)
+    return by_geometry(pow2, uniform, [&](auto p2, auto uni) {
+      return launch_rows_lagrangian<T, decltype(p2)::value, decltype(uni)::value>(
+          rg, g, io, r, max_dt, parts, s);
+    });
   return by_geometry(pow2, uniform, [&](auto p2, auto uni) {
     return launch_march_lagrangian_p<T, decltype(p2)::value, decltype(uni)::value>(
         g, io, r, max_dt, parts, chunk_rows, s);
@@ -231,6 +317,13 @@ hipError_t launch_march_momentum(MGeo<T> g, MMomIO<T> io, int tt, int ydir,
 template <typename T>
 hipError_t launch_march_momxy(MGeo<T> g, MMom2IO<T> io, int tt, FkReduce r, int parts,
                               int chunk_rows, int pow2, int uniform, hipStream_t s) {
+  const RowsGrid rg = rows_grid(g.nx, g.ny, chunk_rows, kMomXYW,
+                                tt % 2 ? kRowsMomXYHalo : kRowsMomYXHalo);
+  if (rg.waves)
+    return by_geometry(pow2, uniform, [&](auto p2, auto uni) {
+      return launch_rows_momxy<T, decltype(p2)::value, decltype(uni)::value>(
+          rg, g, io, tt, r, parts, s);
+    });
   return by_geometry(pow2, uniform, [&](auto p2, auto uni) {
     return launch_march_momxy_p<T, decltype(p2)::value, decltype(uni)::value>(
         g, io, tt, r, parts, chunk_rows, s);

@@ -48,10 +48,11 @@ __global__ __launch_bounds__(kRedThreads) void k_timestep(
 }
 
 /* The (dt, dt_h) update from parts blocks' minima. */
-__global__ __launch_bounds__(kWave) void k_finish_timestep(FkReduce r, int parts,
+__global__ __launch_bounds__(kRedThreads) void k_finish_timestep(FkReduce r, int parts,
                                                            double max_dt, int first_step) {
-  const double g = fold_min<false>(r, parts, max_dt);
-  const int bad = fold_undefined(r, parts);
+  const MinFold m = fold_min<false>(r, parts, max_dt);
+  const double g = m.g;
+  const int bad = m.bad;
   if (threadIdx.x == 0) {
     const DtPair p = next_pair(g, r.dtp[1], first_step);
     r.dtp[0] = p.dt;
@@ -242,7 +243,7 @@ int fk_reduce_blocks(void) { return kPartialsDoubles; }
 
 hipError_t fk_finish_timestep(FkReduce r, int parts, double max_dt, int first_step,
                               hipStream_t s) {
-  hipLaunchKernelGGL(k_finish_timestep, dim3(1), dim3(kWave), 0, s, r, parts, max_dt,
+  hipLaunchKernelGGL(k_finish_timestep, dim3(1), dim3(kRedThreads), 0, s, r, parts, max_dt,
                      first_step);
   return hipGetLastError();
 }

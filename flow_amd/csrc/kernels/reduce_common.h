@@ -22,8 +22,9 @@ constexpr int kTotalsOffset = 2 * kMaxReduceBlocks;
 constexpr int kTotalsWords = 8;
 constexpr int kPartialsDoubles = kTotalsOffset + kTotalsWords * kMaxReduceBlocks;
 
+/* (of a block of at most NT threads) */
 template <int NT>
-__device__ __forceinline__ double block_min(double x) {
+__device__ __forceinline__ double block_min(double x, int waves = NT / kWave) {
   __shared__ double red[NT / kWave];
   x = wave_min(x);
   const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
@@ -31,7 +32,7 @@ __device__ __forceinline__ double block_min(double x) {
   if (lane == 0) red[w] = x;
   __syncthreads();
   if (w == 0) {
-    x = (lane < NT / kWave) ? red[lane] : red[0];
+    x = (lane < waves) ? red[lane] : red[0];
     x = wave_min(x);
   }
   return x; /* valid in wave 0 */
@@ -66,41 +67,60 @@ __device__ __forceinline__ CSum block_csum(CSum v) {
  * set_timestep of a 512^2 mesh (1024 blocks) took 70 us of which 64 were
  * that, the 752-block Lagrangian march of a 1000^2 mesh about 45 of 117. */
 
-/* A block's CFL minimum and its count of undefined candidates. */
+/* A block's CFL minimum and its count of undefined candidates (at most NT
+ * threads). */
 template <int NT>
-__device__ __forceinline__ void publish_min(double local_min, int nan_count, FkReduce r) {
+__device__ __forceinline__ void publish_min(double local_min, int nan_count, FkReduce r,
+                                            int waves = NT / kWave) {
   __shared__ int s_nan[NT / kWave];
   const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
   /* almost always none */
   if (__ballot(nan_count != 0)) nan_count = wave_sum(nan_count);
   if (lane == 0) s_nan[w] = nan_count;
-  const double bmin = block_min<NT>(local_min);
+  const double bmin = block_min<NT>(local_min, waves);
   if (threadIdx.x == 0) {
     int bad = 0;
-    for (int k = 0; k < NT / kWave; ++k) bad += s_nan[k];
+    for (int k = 0; k < waves; ++k) bad += s_nan[k];
     r.partials[2 * blockIdx.x] = bmin;
     r.partials[2 * blockIdx.x + 1] = (double)bad;
   }
 }
 
-/* The minimum over parts blocks' partials and max_dt; the same in every
- * thread. Each wave folds all of them for itself: no LDS, no barrier. kSquared:
- * the candidates are squared time steps (the FP32-state form); the minimum's
- * square root is taken once, here. */
+/* The minimum over parts blocks' partials and max_dt, the same in every thread
+ * of the block (at most 16 waves), and their undefined candidates, valid in
+ * thread 0. The block shares the loads out: one or two a thread in flight at
+ * once, then one barrier. (With each wave folding all of them for itself, the
+ * batches of loads took 7800 of the 16100 cycles that a block of the
+ * mass/energy kernel runs for on a 512^2 mesh.) kSquared: the candidates are
+ * squared time steps (the FP32-state form); the minimum's square root is
+ * taken once, here. */
+struct MinFold {
+  double g;
+  int bad;
+};
 template <bool kSquared>
-__device__ __forceinline__ double fold_min(const FkReduce& r, int parts, double max_dt) {
+__device__ __forceinline__ MinFold fold_min(const FkReduce& r, int parts, double max_dt) {
+  __shared__ double s_min[16];
+  __shared__ int s_bad[16];
+  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave, waves = blockDim.x / kWave;
   double g = kSquared ? max_dt * max_dt : max_dt;
-#pragma unroll 4
-  for (int b = threadIdx.x % kWave; b < parts; b += kWave) g = lesser(g, r.partials[2 * b]);
-  g = wave_min(g);
-  return kSquared ? __builtin_sqrt(g) : g;
-}
-
-/* The undefined candidates of parts blocks, by one wave. */
-__device__ __forceinline__ int fold_undefined(const FkReduce& r, int parts) {
   int bad = 0;
-  for (int b = threadIdx.x % kWave; b < parts; b += kWave) bad += (int)r.partials[2 * b + 1];
-  return wave_sum(bad);
+#pragma unroll 4
+  for (int b = threadIdx.x; b < parts; b += blockDim.x) {
+    g = lesser(g, r.partials[2 * b]);
+    bad += (int)r.partials[2 * b + 1];
+  }
+  g = wave_min(g);
+  if (__ballot(bad != 0)) bad = wave_sum(bad);
+  if (lane == 0) {
+    s_min[w] = g;
+    s_bad[w] = bad;
+  }
+  __syncthreads();
+  g = wave_min(s_min[lane < waves ? lane : 0]);
+  if (threadIdx.x == 0)
+    for (int k = 1; k < waves; ++k) bad += s_bad[k];
+  return MinFold{kSquared ? __builtin_sqrt(g) : g, bad};
 }
 
 /* The (dt, dt_h) update of omp3/flow.c:103-105 from the grid minimum g. */
@@ -281,8 +301,8 @@ __device__ __forceinline__ void post(const FkReduce& r, int k, double v) {
   if (r.mail) r.mail[k] = v;
 }
 
-/* The totals of parts blocks' words -> r.sums[0..1], by one block: its first
- * half the mass, its second the energy. */
+/* The totals of parts blocks' words -> r.sums[0..1], by the first NT threads of
+ * one block: the first half the mass, the second the energy. */
 template <int NT>
 __device__ void fold_totals(const FkReduce& r, int parts) {
   constexpr int kHalf = NT / 2;
@@ -294,19 +314,19 @@ __device__ void fold_totals(const FkReduce& r, int parts) {
   Words192 t{0, 0, 0};
   unsigned long long any = 0;
 #pragma unroll 2
-  for (int b = threadIdx.x % kHalf; b < parts; b += kHalf) {
+  for (int b = threadIdx.x % kHalf; q < 2 && b < parts; b += kHalf) {
     const unsigned long long* v = p + kTotalsWords * b;
     add192(t, Words192{v[0], v[1], v[2]});
     any |= v[3];
   }
   t = wave_sum192(t);
   const bool bad = __ballot(any != 0ull) != 0ull;
-  if (lane == kWave - 1) {
+  if (q < 2 && lane == kWave - 1) {
     s_sum[w] = t;
     s_bad[w] = bad;
   }
   __syncthreads();
-  if (threadIdx.x % kHalf == 0) {
+  if (q < 2 && threadIdx.x % kHalf == 0) {
     constexpr int kPer = kHalf / kWave;
     Words192 s = s_sum[q * kPer];
     unsigned int b = s_bad[q * kPer];
