@@ -35,7 +35,7 @@ struct FlowHipEnsemble {
   size_t pool_bytes;
   void* snap;          /* autotuner snapshot of pool + dt pairs */
   void* geo;           /* geometry of all instances */
-  double* d_dtp;       /* 2 per instance */
+  double* d_dtp;       /* 2 per instance, then 2 per instance for dtp_new */
   double* h_dtp;       /* pinned */
   double* set_dtp;     /* pinned: pairs set by the caller, on their way */
   char* is_set;        /* per instance: set_dtp holds a pair to upload */
@@ -144,11 +144,7 @@ static void ens_build_work(FlowHipEnsemble* E) {
   HIPCHECK(hipMemcpy(E->d_work, pairs, sizeof(int) * 2 * (size_t)total,
                      hipMemcpyHostToDevice));
   if (total > E->part_items) {
-    HIPCHECK(hipFree(E->part.min));
-    HIPCHECK(hipFree(E->part.nan));
     HIPCHECK(hipFree(E->part.sums));
-    HIPCHECK(hipMalloc((void**)&E->part.min, sizeof(double) * (size_t)total));
-    HIPCHECK(hipMalloc((void**)&E->part.nan, sizeof(int) * (size_t)total));
     HIPCHECK(hipMalloc((void**)&E->part.sums, sizeof(double) * 4 * (size_t)total));
     E->part_items = total;
   }
@@ -220,7 +216,7 @@ FlowHipEnsemble* flowhip_ensemble_new(int ninst, const int* global_nx,
   HIPCHECK(hipMalloc(&E->pool, off));
   HIPCHECK(hipMemset(E->pool, 0, off));
   HIPCHECK(hipMalloc(&E->geo, goff));
-  HIPCHECK(hipMalloc((void**)&E->d_dtp, sizeof(double) * 2 * (size_t)ninst));
+  HIPCHECK(hipMalloc((void**)&E->d_dtp, sizeof(double) * 4 * (size_t)ninst));
   HIPCHECK(hipHostMalloc((void**)&E->h_dtp, sizeof(double) * 2 * (size_t)ninst,
                          hipHostMallocDefault));
   HIPCHECK(hipHostMalloc((void**)&E->set_dtp, sizeof(double) * 2 * (size_t)ninst,
@@ -272,6 +268,7 @@ FlowHipEnsemble* flowhip_ensemble_new(int ninst, const int* global_nx,
     const double dx = width[i] / global_nx[i], dy = height[i] / global_ny[i];
     in->u = fp32 ? flowhip_uniform32(dx, dy, dx, dy) : flowhip_uniform(dx, dy, dx, dy);
     in->dtp = E->d_dtp + 2 * i;
+    in->dtp_new = E->d_dtp + 2 * (ninst + i);
     in->max_dt = max_dt[i];
     E->h_dtp[2 * i] = C_T * dt_param[i];
     E->h_dtp[2 * i + 1] = C_T * dt_param[i];
@@ -305,6 +302,10 @@ FlowHipEnsemble* flowhip_ensemble_new(int ninst, const int* global_nx,
   free(aoff);
   free(gof);
   HIPCHECK(hipMalloc((void**)&E->d_insts, sizeof(FkEnsInst) * (size_t)ninst));
+  HIPCHECK(hipMalloc((void**)&E->part.min, sizeof(unsigned long long) * (size_t)ninst));
+  HIPCHECK(hipMemset(E->part.min, 0xff, sizeof(unsigned long long) * (size_t)ninst));
+  HIPCHECK(hipMalloc((void**)&E->part.nan, sizeof(int) * (size_t)ninst));
+  HIPCHECK(hipMemset(E->part.nan, 0, sizeof(int) * (size_t)ninst));
   HIPCHECK(hipMalloc((void**)&E->hist.counter, sizeof(int)));
   HIPCHECK(hipMemset(E->hist.counter, 0, sizeof(int)));
   HIPCHECK(hipMalloc((void**)&E->d_queue, sizeof(unsigned int) * FK_MARCH_QUEUE_WORDS));
@@ -492,7 +493,7 @@ int flowhip_ensemble_run(FlowHipEnsemble* E, int niters, int tt0, int pre_timest
   if (pre_timestep) HIPCHECK(fk_ens_timestep(ens_launch(E), E->fp32, E->stream));
   HIPCHECK(hipMemcpyAsync(E->h_dtp, E->d_dtp, sizeof(double) * 2 * (size_t)n,
                           hipMemcpyDeviceToHost, E->stream));
-  HIPCHECK(fk_ens_set_counter(E->hist.counter, 0, E->stream));
+  HIPCHECK(fk_ens_set_counter(E->hist.counter, -1, E->stream));
   HIPCHECK(hipStreamSynchronize(E->stream));
   if (dt_pairs)
     for (int i = 0; i < n; ++i) {
@@ -570,7 +571,7 @@ int flowhip_ensemble_autotune(FlowHipEnsemble* E, int trial_steps, int tt0,
       E->order = o;
       E->fused_momentum = fm;
       ens_build_work(E);
-      HIPCHECK(fk_ens_set_counter(E->hist.counter, 0, E->stream));
+      HIPCHECK(fk_ens_set_counter(E->hist.counter, -1, E->stream));
       /* one untimed step, then the timed ones */
       HIPCHECK(fk_ens_step(ens_launch(E), tt0 + 1, E->fp32, E->stream));
       HIPCHECK(hipEventRecord(a, E->stream));

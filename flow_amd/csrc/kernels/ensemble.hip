@@ -10,12 +10,13 @@
  * and runs the same per-item body as the single-mesh march kernels, so a
  * batched instance computes bit for bit what it computes alone.
  *
- * Per-instance reductions go through per-item partials, indexed by the
- * item's position inside its instance, and small per-instance kernels that
- * combine them in item order: the CFL minimum and dt update of
- * omp3/flow.c:77-105 (one dt pair per instance) and the compensated mass
- * and energy totals of omp3/flow.c:973-995. Per-step dt pairs and totals
- * are appended to device history buffers at a device-side step counter,
+ * A step is the three march kernels and nothing between them. An instance's CFL
+ * minimum (omp3/flow.c:77-105) is one word that the Lagrangian march's items
+ * lower; the mass/energy march's items each take the new dt pair from it. The
+ * compensated mass and energy totals (omp3/flow.c:973-995) go through per-item
+ * partials, indexed by the item's position inside its instance, which blocks at
+ * the front of the momentum march combine in item order. Per-step dt pairs and
+ * totals are appended to device history buffers at a device-side step counter,
  * so a step can be captured once in a hipGraph and replayed.
  */
 #include <cmath>
@@ -65,14 +66,56 @@ __device__ __forceinline__ MarchList ens_list(const FkEnsInst& in, int H) {
   return ml;
 }
 
-/* ---- the four stages ---- */
+/* ---- CFL minima, one word per instance ----
+ * A double as an unsigned key of the same order (any sign), so that the minimum
+ * is an integer atomic whose result does not depend on the order of the items;
+ * all ones: no candidate yet. An item whose candidates all lie at or above its
+ * seed (cfl_seed: they cannot count) leaves the word alone, which on most steps
+ * is nearly every item. */
+constexpr unsigned long long kNoCandidate = ~0ull;
+
+__device__ __forceinline__ unsigned long long min_key(double x) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+  return b ^ ((unsigned long long)((long long)b >> 63) | 0x8000000000000000ull);
+}
+__device__ __forceinline__ double min_value(unsigned long long key) {
+  const unsigned long long b = (key >> 63) ? key ^ 0x8000000000000000ull : ~key;
+  return __longlong_as_double((long long)b);
+}
+
+/* An item's minimum and its undefined candidates, per lane. */
+__device__ __forceinline__ void publish_item(const FkEnsPartials& part, int inst, int lane,
+                                             double local_min, double seed, int nan_count) {
+  local_min = wave_min(local_min);
+  if (lane == 0 && local_min < seed) atomicMin(part.min + inst, min_key(local_min));
+  if (__ballot(nan_count != 0)) {
+    nan_count = wave_sum(nan_count);
+    if (lane == 0) atomicAdd(part.nan + inst, nan_count);
+  }
+}
+
+/* The instance's new pair (omp3/flow.c:103-105). */
+template <bool kSquared>
+__device__ __forceinline__ DtPair ens_pair(const FkEnsInst& in, unsigned long long key,
+                                           int first_step) {
+  double g = kSquared ? in.max_dt * in.max_dt : in.max_dt;
+  if (key != kNoCandidate) g = lesser(g, min_value(key));
+  if (kSquared) g = __builtin_sqrt(g);
+  return next_pair(g, in.dtp[1], first_step);
+}
+
+/* ---- the stages ---- */
 
 template <typename T, bool P2, bool UNI>
 __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_lagrangian(
     const FkEnsInst* __restrict__ insts, const int2* __restrict__ work, int nwork,
     unsigned int* __restrict__ queue,
-    int H, FkEnsPartials part) {
+    int H, FkEnsPartials part, int* __restrict__ counter) {
   const int lane = threadIdx.x % kWave;
+  if (blockIdx.x == 0) {
+    march_queue_reset(queue, kStageLag);
+    if (threadIdx.x == 0) *counter += 1; /* this step's history row */
+  }
   MarchQueue<true> mq(queue, kStageLag, nwork, blockIdx.x, gridDim.x);
   for (int w = mq.first(); w < mq.end; w = mq.next()) {
     const int2 wi = work[w];
@@ -82,7 +125,8 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_lagrangian(
                        arr<T>(in, kUFx),   arr<T>(in, kUFy), arr<T>(in, kP),
                        arr<T>(in, kRhoOld)};
     const T dt = T(in.dtp[0]), dt_h = T(in.dtp[1]);
-    double local_min = cfl_seed<T>(in.max_dt, in.dtp[1]);
+    const double seed = cfl_seed<T>(in.max_dt, in.dtp[1]);
+    double local_min = seed;
     int nan_count = 0;
     const MGeo<T> g = ens_geo<T>(in);
     const MarchList ml = ens_list(in, H);
@@ -95,12 +139,7 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_lagrangian(
       lagrangian_box<T, P2, 0, false, kUni>(g, io, dt, dt_h, b, lane, local_min, nan_count);
     else
       lagrangian_box<T, P2, -1, true, kUni>(g, io, dt, dt_h, b, lane, local_min, nan_count);
-    local_min = wave_min(local_min);
-    nan_count = wave_sum(nan_count);
-    if (lane == 0) {
-      part.min[in.item0 + wi.y] = local_min;
-      part.nan[in.item0 + wi.y] = nan_count;
-    }
+    publish_item(part, wi.x, lane, local_min, seed, nan_count);
   }
 }
 
@@ -108,8 +147,9 @@ template <typename T, bool P2, bool UNI>
 __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_mass(
     const FkEnsInst* __restrict__ insts, const int2* __restrict__ work, int nwork,
     unsigned int* __restrict__ queue,
-    int H, int tt, FkEnsPartials part) {
+    int H, int tt, int ninst, FkEnsPartials part, FkEnsHistory hist) {
   const int lane = threadIdx.x % kWave;
+  if (blockIdx.x == 0) march_queue_reset(queue, kStageMass);
   MarchQueue<true> mq(queue, kStageMass, nwork, blockIdx.x, gridDim.x);
   for (int w = mq.first(); w < mq.end; w = mq.next()) {
     const int2 wi = work[w];
@@ -117,7 +157,15 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_mass(
     const MMassIO<T> io{arr<T>(in, kUFx), arr<T>(in, kUFy), arr<T>(in, kRhoOld),
                         arr<T>(in, kP),   arr<T>(in, kRho), arr<T>(in, kE),
                         arr<T>(in, kFx),  arr<T>(in, kFy)};
-    const T dt = T(in.dtp[0]), dt_h = T(in.dtp[1]);
+    const DtPair pair =
+        ens_pair<std::is_same<T, float>::value>(in, part.min[wi.x], tt == 0 ? 1 : 0);
+    const T dt = T(pair.dt), dt_h = T(pair.dt_h);
+    if (wi.y == 0 && lane == 0) {
+      const long h = (long)*hist.counter * ninst + wi.x;
+      in.dtp_new[0] = hist.dt[2 * h] = pair.dt;
+      in.dtp_new[1] = hist.dt[2 * h + 1] = pair.dt_h;
+      hist.nan[h] = part.nan[wi.x];
+    }
     CSum ms{0.0, 0.0}, es{0.0, 0.0};
     const MGeo<T> g = ens_geo<T>(in);
     const MarchList ml = ens_list(in, H);
@@ -146,19 +194,64 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_mass(
   }
 }
 
+/* ---- the step's epilogue ----
+ * The first ens_epilogue_blocks blocks of the momentum march march nothing: a
+ * wave per instance folds the totals' partials in item order, moves the new dt
+ * pair to where the next step's Lagrangian march reads it, and clears the CFL
+ * words. As kernels of their own (dt pair, totals, counter) these took 15 us of
+ * a 150 us step of 24 instances of 64^2 to 464^2 on MI355X and 31 of 750 us for
+ * 96 FP32 instances up to 1013^2. */
+__host__ __device__ inline int ens_epilogue_blocks(int ninst) { return (ninst + kMWaves - 1) / kMWaves; }
+
+__device__ __forceinline__ void ens_epilogue(const FkEnsInst* __restrict__ insts, int ninst,
+                                             const FkEnsPartials& part,
+                                             const FkEnsHistory& hist) {
+  const int lane = threadIdx.x % kWave;
+  const int inst =
+      __builtin_amdgcn_readfirstlane(blockIdx.x * kMWaves + threadIdx.x / kWave);
+  if (inst >= ninst) return;
+  const FkEnsInst& in = insts[inst];
+  CSum gm{0.0, 0.0}, ge{0.0, 0.0};
+#pragma unroll 4
+  for (int k = lane; k < in.nitems; k += kWave) {
+    const double* p = part.sums + 4 * (in.item0 + k);
+    gm.merge(CSum{p[0], p[1]});
+    ge.merge(CSum{p[2], p[3]});
+  }
+  gm = wave_csum(gm);
+  ge = wave_csum(ge);
+  if (lane == 0) {
+    const long h = (long)*hist.counter * ninst + inst;
+    hist.sums[2 * h] = gm.s + gm.c;
+    hist.sums[2 * h + 1] = ge.s + ge.c;
+    in.dtp[0] = in.dtp_new[0];
+    in.dtp[1] = in.dtp_new[1];
+    part.min[inst] = kNoCandidate;
+    part.nan[inst] = 0;
+  }
+}
+
 /* ydir 0: x momentum (u0 = uF_x), 1: y momentum (io.u = the u just written) */
 template <typename T, bool P2>
 __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_momentum(
     const FkEnsInst* __restrict__ insts, const int2* __restrict__ work, int nwork,
     unsigned int* __restrict__ queue,
-    int H, int tt, int ydir) {
+    int H, int tt, int ydir, int ninst, FkEnsPartials part, FkEnsHistory hist) {
   const int lane = threadIdx.x % kWave;
-  /* no epilogue kernel between the two directions: a set each */
-  MarchQueue<true> mq(queue, ydir ? kStageLag : kStageMom, nwork, blockIdx.x, gridDim.x);
+  const int front = ydir ? 0 : ens_epilogue_blocks(ninst);
+  /* the y direction counts in the mass/energy march's set, which the x
+   * direction has zeroed */
+  const int stage = ydir ? kStageMass : kStageMom;
+  if (blockIdx.x == 0) march_queue_reset(queue, stage);
+  if ((int)blockIdx.x < front) {
+    ens_epilogue(insts, ninst, part, hist);
+    return;
+  }
+  MarchQueue<true> mq(queue, stage, nwork, blockIdx.x - front, gridDim.x - front);
   for (int w = mq.first(); w < mq.end; w = mq.next()) {
     const int2 wi = work[w];
     const FkEnsInst& in = insts[wi.x];
-    const T dt = T(in.dtp[0]), dt_h = T(in.dtp[1]);
+    const T dt = T(in.dtp_new[0]), dt_h = T(in.dtp_new[1]);
     const MGeo<T> g = ens_geo<T>(in);
     const MarchList ml = ens_list(in, H);
     if (!ydir) {
@@ -186,17 +279,23 @@ template <typename T, bool P2, bool UNI>
 __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_momentum_xy(
     const FkEnsInst* __restrict__ insts, const int2* __restrict__ work, int nwork,
     unsigned int* __restrict__ queue,
-    int H, int tt) {
+    int H, int tt, int ninst, FkEnsPartials part, FkEnsHistory hist) {
   const int lane = threadIdx.x % kWave;
+  const int front = ens_epilogue_blocks(ninst);
+  if (blockIdx.x == 0) march_queue_reset(queue, kStageMom);
+  if ((int)blockIdx.x < front) {
+    ens_epilogue(insts, ninst, part, hist);
+    return;
+  }
   /* claimed per block, as the single-mesh fused momentum march */
   const int wave = threadIdx.x / kWave;
-  MarchBlockQueue mq(queue, kStageMom, nwork, blockIdx.x, gridDim.x);
+  MarchBlockQueue mq(queue, kStageMom, nwork, blockIdx.x - front, gridDim.x - front);
   for (int base = mq.first(); base < mq.end; base = mq.next()) {
     const int w = __builtin_amdgcn_readfirstlane(base + wave);
     if (w >= mq.end) continue;
     const int2 wi = work[w];
     const FkEnsInst& in = insts[wi.x];
-    const T dt = T(in.dtp[0]), dt_h = T(in.dtp[1]);
+    const T dt = T(in.dtp_new[0]), dt_h = T(in.dtp_new[1]);
     const MMom2IO<T> io{arr<T>(in, kUFx), arr<T>(in, kUFy), arr<T>(in, kFx),
                         arr<T>(in, kFy),  arr<T>(in, kRho), arr<T>(in, kQxx),
                         arr<T>(in, kQyy), arr<T>(in, kMomX), arr<T>(in, kMomY),
@@ -242,94 +341,34 @@ __global__ __launch_bounds__(kMNT) void k_ens_timestep(
     if (j < x1) {
       for (int i = y0; i < y1; ++i) {
         const int c = i * nx + j;
-        const double cand =
-            cell_timestep(double(e[c]), double(qxx[c]), double(qyy[c]),
-                          double(rho[c]), double(g.cdx[j]), double(g.cdy[i]));
+        const double ec = double(e[c]), qx = double(qxx[c]), qy = double(qyy[c]),
+                     rc = double(rho[c]), dx = double(g.cdx[j]), dy = double(g.cdy[i]);
+        if (cfl_above(ec, qx, qy, rc, dx, dy, local_min * local_min)) continue;
+        const double cand = cell_timestep(ec, qx, qy, rc, dx, dy);
         if (cand == cand)
           local_min = lesser(local_min, cand);
         else
           ++nan_count;
       }
     }
-    local_min = wave_min(local_min);
-    nan_count = wave_sum(nan_count);
-    if (lane == 0) {
-      part.min[in.item0 + wi.y] = local_min;
-      part.nan[in.item0 + wi.y] = nan_count;
-    }
+    publish_item(part, wi.x, lane, local_min, in.max_dt, nan_count);
   }
 }
 
-/* ---- per-instance epilogues: one wave per instance ----
- * One of them follows each march stage of a step; its first block also
- * zeroes the work-queue counters, which no other kernel uses meanwhile. */
-
-/* dt pair of omp3/flow.c:103-105 from the instance's item minima; history
- * row *counter when hist != null. */
-__global__ __launch_bounds__(kWave) void k_ens_dt(const FkEnsInst* __restrict__ insts,
-                                                  int ninst, FkEnsPartials part,
-                                                  int first_step, int squared,
-                                                  FkEnsHistory hist,
-                                                  unsigned int* __restrict__ queue) {
-  const int inst = blockIdx.x;
-  if (inst == 0) march_queue_reset(queue, -1);
+/* The pre-loop pair of every instance; clears the CFL words and the work-queue
+ * counters. */
+__global__ __launch_bounds__(kMNT) void k_ens_dt(const FkEnsInst* __restrict__ insts, int ninst,
+                                                 FkEnsPartials part,
+                                                 unsigned int* __restrict__ queue) {
+  if (blockIdx.x == 0) march_queue_reset(queue, -1);
+  const int inst = blockIdx.x * kMNT + threadIdx.x;
   if (inst >= ninst) return;
   const FkEnsInst& in = insts[inst];
-  const int lane = threadIdx.x;
-  double g = squared ? in.max_dt * in.max_dt : in.max_dt;
-  int bad = 0;
-  for (int k = lane; k < in.nitems; k += kWave) {
-    g = lesser(g, part.min[in.item0 + k]);
-    bad += part.nan[in.item0 + k];
-  }
-  g = wave_min(g);
-  if (squared) g = __builtin_sqrt(g);
-  bad = wave_sum(bad);
-  if (lane == 0) {
-    const double dt_h = in.dtp[1];
-    const double final_min = lesser(g, kCM * dt_h);
-    const double dt = 0.5 * (kCT * final_min + dt_h);
-    in.dtp[0] = dt;
-    in.dtp[1] = first_step ? dt : kCT * final_min;
-    if (hist.dt) {
-      const int row = *hist.counter;
-      hist.dt[2 * ((long)row * ninst + inst)] = in.dtp[0];
-      hist.dt[2 * ((long)row * ninst + inst) + 1] = in.dtp[1];
-      hist.nan[(long)row * ninst + inst] = bad;
-    }
-  }
-}
-
-/* Mass and energy totals from the instance's item partials, merged in item
- * order; history row *counter. */
-__global__ __launch_bounds__(kWave) void k_ens_sums(const FkEnsInst* __restrict__ insts,
-                                                    int ninst, FkEnsPartials part,
-                                                    FkEnsHistory hist,
-                                                    unsigned int* __restrict__ queue) {
-  const int inst = blockIdx.x;
-  if (inst == 0) march_queue_reset(queue, -1);
-  if (inst >= ninst) return;
-  const FkEnsInst& in = insts[inst];
-  const int lane = threadIdx.x;
-  CSum gm{0.0, 0.0}, ge{0.0, 0.0};
-  for (int k = lane; k < in.nitems; k += kWave) {
-    const double* p = part.sums + 4 * (in.item0 + k);
-    gm.merge(CSum{p[0], p[1]});
-    ge.merge(CSum{p[2], p[3]});
-  }
-  gm = wave_csum(gm);
-  ge = wave_csum(ge);
-  if (lane == 0) {
-    const int row = *hist.counter;
-    hist.sums[2 * ((long)row * ninst + inst)] = gm.s + gm.c;
-    hist.sums[2 * ((long)row * ninst + inst) + 1] = ge.s + ge.c;
-  }
-}
-
-__global__ __launch_bounds__(kWave) void k_ens_advance(int* counter,
-                                                       unsigned int* __restrict__ queue) {
-  march_queue_reset(queue, -1);
-  if (threadIdx.x == 0) *counter += 1;
+  const DtPair p = ens_pair<false>(in, part.min[inst], 0);
+  in.dtp[0] = p.dt;
+  in.dtp[1] = p.dt_h;
+  part.min[inst] = kNoCandidate;
+  part.nan[inst] = 0;
 }
 
 __global__ void k_ens_set_counter(int* counter, int v) {
@@ -346,29 +385,27 @@ hipError_t ens_step_p(const FkEnsLaunch& L, int tt, hipStream_t s) {
   const int2* work = (const int2*)L.work;
   hipLaunchKernelGGL((k_ens_lagrangian<T, P2, UNI>),
                      dim3(march_grid(k_ens_lagrangian<T, P2, UNI>, pc_lag, nw, kMarchMaxWaves<T>)),
-                     dim3(kMNT), 0, s, L.insts, work, nw, L.queue, L.chunk_rows, L.part);
-  hipLaunchKernelGGL(k_ens_dt, dim3(L.ninst), dim3(kWave), 0, s, L.insts, L.ninst,
-                     L.part, tt == 0 ? 1 : 0, std::is_same<T, float>::value ? 1 : 0,
-                     L.hist, L.queue);
+                     dim3(kMNT), 0, s, L.insts, work, nw, L.queue, L.chunk_rows, L.part,
+                     L.hist.counter);
   hipLaunchKernelGGL((k_ens_mass<T, P2, UNI>),
                      dim3(march_grid(k_ens_mass<T, P2, UNI>, pc_mass, nw, kMarchMaxWaves<T>)),
-                     dim3(kMNT), 0, s, L.insts, work, nw, L.queue, L.chunk_rows, tt, L.part);
-  hipLaunchKernelGGL(k_ens_sums, dim3(L.ninst), dim3(kWave), 0, s, L.insts, L.ninst,
-                     L.part, L.hist, L.queue);
+                     dim3(kMNT), 0, s, L.insts, work, nw, L.queue, L.chunk_rows, tt, L.ninst,
+                     L.part, L.hist);
+  const int front = ens_epilogue_blocks(L.ninst);
   if (L.fused_momentum) {
     static int pc_momxy = 0;
     hipLaunchKernelGGL((k_ens_momentum_xy<T, P2, UNI>),
-                       dim3(march_grid(k_ens_momentum_xy<T, P2, UNI>, pc_momxy, nw,
-                                       kMarchMaxWaves<T>)),
-                       dim3(kMNT), 0, s, L.insts, work, nw, L.queue, L.chunk_rows, tt);
+                       dim3(front + march_grid(k_ens_momentum_xy<T, P2, UNI>, pc_momxy, nw,
+                                               kMarchMaxWaves<T>)),
+                       dim3(kMNT), 0, s, L.insts, work, nw, L.queue, L.chunk_rows, tt, L.ninst,
+                       L.part, L.hist);
   } else {
     const int gm = march_grid(k_ens_momentum<T, P2>, pc_mom, nw);
-    hipLaunchKernelGGL((k_ens_momentum<T, P2>), dim3(gm), dim3(kMNT), 0, s, L.insts,
-                       work, nw, L.queue, L.chunk_rows, tt, 0);
-    hipLaunchKernelGGL((k_ens_momentum<T, P2>), dim3(gm), dim3(kMNT), 0, s, L.insts,
-                       work, nw, L.queue, L.chunk_rows, tt, 1);
+    hipLaunchKernelGGL((k_ens_momentum<T, P2>), dim3(front + gm), dim3(kMNT), 0, s, L.insts,
+                       work, nw, L.queue, L.chunk_rows, tt, 0, L.ninst, L.part, L.hist);
+    hipLaunchKernelGGL((k_ens_momentum<T, P2>), dim3(gm), dim3(kMNT), 0, s, L.insts, work, nw,
+                       L.queue, L.chunk_rows, tt, 1, L.ninst, L.part, L.hist);
   }
-  hipLaunchKernelGGL(k_ens_advance, dim3(1), dim3(kWave), 0, s, L.hist.counter, L.queue);
   return hipGetLastError();
 }
 
@@ -387,13 +424,11 @@ hipError_t ens_timestep(const FkEnsLaunch& L, hipStream_t s) {
   static int pc = 0;
   const int nw = L.nwork;
   if (nw < 1 || L.ninst < 1 || !L.queue) return hipErrorInvalidValue;
-  FkEnsHistory none = L.hist;
-  none.dt = nullptr;
   hipLaunchKernelGGL(k_ens_timestep<T>, dim3(march_grid(k_ens_timestep<T>, pc, nw)),
                      dim3(kMNT), 0, s, L.insts, (const int2*)L.work, nw, L.queue,
                      L.chunk_rows, L.part);
-  hipLaunchKernelGGL(k_ens_dt, dim3(L.ninst), dim3(kWave), 0, s, L.insts, L.ninst,
-                     L.part, 0, 0, none, L.queue);
+  hipLaunchKernelGGL(k_ens_dt, dim3((L.ninst + kMNT - 1) / kMNT), dim3(kMNT), 0, s, L.insts,
+                     L.ninst, L.part, L.queue);
   return hipGetLastError();
 }
 

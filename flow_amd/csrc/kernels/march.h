@@ -193,8 +193,7 @@ __device__ __forceinline__ MarchWalk march_walk(int nitems) {
  *
  * The counters come in sets, one per stage of a step. A launch uses its
  * stage's set, which is zero when it starts, and zeroes the other sets
- * (march_queue_reset; the ensemble's epilogue kernels do it there), so no
- * wave counts itself out at the end of a kernel and no memset is needed
+ * (march_queue_reset), so no wave counts itself out at the end of a kernel and no memset is needed
  * (the launches stay capturable in a graph). Counting the waves out, with
  * the last one resetting the counters, was an atomic per wave on one
  * address, up to 30 us at the end of a launch whose 2800 waves end together.

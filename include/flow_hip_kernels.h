@@ -324,6 +324,7 @@ typedef struct FkEnsInst {
   FkUniform u;             /* the same, by value */
   void* a[16];             /* solve_hydro_2d's arrays, in its order */
   double* dtp;             /* {dt, dt_h} of this instance (device) */
+  double* dtp_new;         /* the pair the step under way computes */
   double max_dt;
   int nstrips, nchunks, nitems;
   unsigned long long strip_inv; /* fk_strip_inverse(nstrips) */
@@ -331,8 +332,9 @@ typedef struct FkEnsInst {
 } FkEnsInst;
 
 typedef struct FkEnsPartials {
-  double* min;   /* per item: CFL minimum */
-  int* nan;      /* per item: undefined CFL candidates */
+  unsigned long long* min; /* per instance: the CFL minimum as an ordered key,
+                              all ones between steps */
+  int* nan;      /* per instance: undefined CFL candidates, 0 between steps */
   double* sums;  /* per item: compensated mass and energy (4 doubles) */
 } FkEnsPartials;
 
@@ -340,7 +342,7 @@ typedef struct FkEnsHistory {
   double* dt;    /* [step][instance][2]: dt pair after the step */
   double* sums;  /* [step][instance][2]: mass and energy totals */
   int* nan;      /* [step][instance]: undefined CFL candidates */
-  int* counter;  /* device step counter (the history row) */
+  int* counter;  /* device step counter: the history row of the last step */
 } FkEnsHistory;
 
 typedef struct FkEnsLaunch {
@@ -351,8 +353,8 @@ typedef struct FkEnsLaunch {
   int uniform;             /* take each instance's spacings by value (its
                               arrays hold one value throughout) */
   int fused_momentum;      /* both momentum directions in one march */
-  unsigned int* queue;     /* FK_MARCH_QUEUE_WORDS work-queue words, zero
-                              between steps (the epilogue kernels zero them) */
+  unsigned int* queue;     /* FK_MARCH_QUEUE_WORDS work-queue words, zeroed
+                              once (each launch zeroes the sets it leaves) */
   FkEnsPartials part;
   FkEnsHistory hist;
 } FkEnsLaunch;
@@ -363,8 +365,9 @@ int fk_ens_strip_width(void);
 unsigned long long fk_strip_inverse(int nstrips);
 /* Chunk height of an ensemble of so many interior cells, all instances. */
 int fk_ens_default_rows(double cells, int fp32);
-/* One step (omp3/flow.c:10-52) of every instance: Lagrangian stage, dt,
- * mass/energy advection, totals, x and y momentum, counter advance. */
+/* One step (omp3/flow.c:10-52) of every instance: Lagrangian stage with the
+ * counter's advance, mass/energy advection with the dt pairs, x and y momentum
+ * with the totals. */
 hipError_t fk_ens_step(FkEnsLaunch L, int tt, int fp32, hipStream_t s);
 /* The pre-loop set_timestep (first_step = 0) of every instance. */
 hipError_t fk_ens_timestep(FkEnsLaunch L, int fp32, hipStream_t s);
