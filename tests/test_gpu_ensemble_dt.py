@@ -16,7 +16,7 @@ from flow_amd import problems
 pytestmark = pytest.mark.gpu
 
 SIZES = [33, 2, 64, 130, 17, 58, 59, 90, 121]
-STEPS = 3
+STEPS = 6
 
 
 def _init(kind, k, n):
