@@ -130,15 +130,12 @@ __global__ __launch_bounds__(kMNT, FLOWHIP_MARCH_WAVES) void k_ens_lagrangian(
     int nan_count = 0;
     const MGeo<T> g = ens_geo<T>(in);
     const MarchList ml = ens_list(in, H);
-    /* interior items take the straight-line form, as on a single mesh; the
-     * uniform-geometry form in FP64 only (0.3% faster there, 1% slower in
-     * FP32, where the per-row reciprocals are cheap) */
-    constexpr bool kUni = UNI && sizeof(T) == 8;
+    /* interior items take the straight-line form, as on a single mesh */
     const ItemBox b = item_box(ml, g.nx, g.ny, wi.y);
     if (!box_edge(b, g.nx, g.ny))
-      lagrangian_box<T, P2, 0, false, kUni>(g, io, dt, dt_h, b, lane, local_min, nan_count);
+      lagrangian_box<T, P2, 0, false, UNI>(g, io, dt, dt_h, b, lane, local_min, nan_count);
     else
-      lagrangian_box<T, P2, -1, true, kUni>(g, io, dt, dt_h, b, lane, local_min, nan_count);
+      lagrangian_box<T, P2, -1, true, UNI>(g, io, dt, dt_h, b, lane, local_min, nan_count);
     publish_item(part, wi.x, lane, local_min, seed, nan_count);
   }
 }
