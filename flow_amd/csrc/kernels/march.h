@@ -433,6 +433,35 @@ using RowS = typename std::conditional<UNI, RowConst<T>, RowScalar<T>>::type;
 template <typename T, bool P2, bool UNI>
 using RowR = typename std::conditional<UNI, RowConst<T>, RowRecip<T, P2>>::type;
 
+/* row(r) for the rows [r, end), U at a time. A row of a march ends by shifting
+ * its register windows on, some 40 moves of the mass/energy march's 390 vector
+ * operations a row; over several rows in one block the shifts become renamings.
+ * (The compiler does not unroll a loop around cross-lane moves by itself.) The
+ * interior mass/energy marches take two rows at a time in FP64 and four in
+ * FP32; measured on MI355X (us, one, two and four rows at a time, FP64; FP32):
+ * 1000^2 35.0, 34.2, 33.8; 23.5, 23.3, 23.4, 1536^2 59.6, 58.1, 58.2; 33.2, 32.5,
+ * 32.4, 2048^2 91.0, 86.7, 89.6; 46.3, 45.2, 45.0, 3001x2999 184, 173, 173; 96.0,
+ * 93.1, 91.6, 4096^2 285, 274, 276; 156, 156, 152. The Lagrangian march was
+ * slower at two and at four (FP64 3001x2999 205 -> 213 and 208), the momentum
+ * march the same; they keep one. */
+template <typename T>
+constexpr int kMassUnroll = sizeof(T) == 8 ? 2 : 4;
+
+template <int U, typename F>
+__device__ __forceinline__ void each_row(int r, int end, F&& row) {
+  if constexpr (U > 1) {
+    for (; r + U <= end; r += U) {
+      row(r);
+      row(r + 1);
+      if constexpr (U > 2) {
+        row(r + 2);
+        row(r + 3);
+      }
+    }
+  }
+  for (; r < end; ++r) row(r);
+}
+
 /* ---- boundary-strip writers (ghost writes only in edge items) ---- */
 template <typename T>
 __device__ __forceinline__ void mput_cell(bool edge, T* a, int nx, int ny, int i,
@@ -672,7 +701,7 @@ __device__ __forceinline__ void mass_xy_box(const MGeo<T>& g, const MMassIO<T>& 
   /* row rb's inputs; later rows are loaded one step ahead */
   T a_r = io.rho0[rb * nx + qc], a_e = io.e1[rb * nx + qc];
   T a_u = io.u0[rb * sx + qf], a_v = io.v0[rb * nx + qc];
-  for (int r = rb; r <= y1 + 1; ++r) {
+  each_row<EDGE ? 1 : kMassUnroll<T>>(rb, y1 + 2, [&](int r) __attribute__((always_inline)) {
     const bool ghost_row = EDGE && r >= ny - kPad;
     /* prefetch the next row (the last row, y1+1, has none) */
     T n_r = T(0), n_e = T(0), n_u = T(0), n_v = T(0);
@@ -756,7 +785,7 @@ __device__ __forceinline__ void mass_xy_box(const MGeo<T>& g, const MMassIO<T>& 
     a_e = n_e;
     a_u = n_u;
     a_v = n_v;
-  }
+  });
 }
 
 /* The x-first mass/energy march of an interior item, two columns per lane
@@ -1010,7 +1039,7 @@ __device__ __forceinline__ void mass_yx_box(const MGeo<T>& g, const MMassIO<T>& 
   T n_v = io.v0[(y0 + 2) * nx + qm];
   T a_u = io.u0[y0 * sx + qf];
   T a_r0 = io.rho0[y0 * nx + qc];
-  for (int r = y0; r < y1; ++r) {
+  each_row<EDGE ? 1 : kMassUnroll<T>>(y0, y1, [&](int r) __attribute__((always_inline)) {
     wr[3] = n_r;
     we[3] = n_e;
     wv[2] = n_v;
@@ -1065,7 +1094,7 @@ __device__ __forceinline__ void mass_yx_box(const MGeo<T>& g, const MMassIO<T>& 
     }
     wv[0] = wv[1];
     wv[1] = wv[2];
-  }
+  });
 }
 
 /* The y-first mass/energy march of an interior item, two columns per lane
