@@ -5,8 +5,8 @@ One step = one solve_hydro_2d + print_conservation pass (main.c:82-91) over an
 8192^2 FP64 mesh (4x4 seeded blasts, log-uniform pressures in [10, 1000] on a
 rho=1 p=0.1 background, +/-5% seeded density noise). Inputs are resident in
 HBM before the timed region; the driver loop runs on the host through the C
-ABI (flowhip_run), with one device-to-host transfer of the scalars per
-interface call, exactly as main.c would drive it.
+ABI (flowhip_run), which hands the scalars of every step back to the host,
+exactly as main.c would drive it.
 
 Prints ONE JSON line: whole-job cell-updates/s, the roofline of the dominant
 kernel (HIP-event durations on the kernel set's stream x its algorithmic

@@ -1,7 +1,7 @@
 /*
  * flowhip_ctx.h -- private per-Mesh state of the hip kernel set: its stream,
  * the device-resident timestep pair, reduction scratch, pinned staging for
- * the one device-to-host transfer per step, captured step graphs and the
+ * the scalars that cross to and from the host, captured step graphs and the
  * per-kernel event timers.
  */
 #ifndef FLOWHIP_CTX_H

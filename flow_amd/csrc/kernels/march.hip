@@ -1,6 +1,7 @@
 /*
  * march.hip -- launchers of the row-marching kernels on one mesh (FP64 and
- * the FP32-state form). The kernels are in march.h.
+ * the FP32-state form). The kernels are in march.h, their row-parallel form for
+ * small meshes in rows.h.
  */
 #include <cmath>
 
