@@ -22,27 +22,39 @@ namespace flowhip {
  * fixed heights of 24 / 20 / 16 rows (24 / 16 / 16) before and this rule
  * after: 64^2 168 -> 64; 138 -> 52, 512^2 180 -> 83; 144 -> 60, 1000^2 197
  * -> 130; 156 -> 90, 3000x150 195 -> 96; 156 -> 72, 2048^2 323 -> 323; 191 ->
- * 166, 3001x2999 and up within 2%. */
+ * 166, 3001x2999 and up within 2%.
+ *
+ * Where a mass/energy or momentum chunk up to 1.6 times as tall lets the items
+ * fit the waves in one round, it is taken: items a little over one round leave
+ * the last ones to march alone. Measured (us a kernel, the height above and this
+ * one): FP64 momentum 1150^2 35.7 -> 33.0, 1250^2 39.8 -> 36.3, 1400^2 45.3 -> 41.4,
+ * mass/energy 1100^2 39.0 -> 36.0, 1400^2 50.7 -> 49.3; FP32 momentum 1250^2 24.0
+ * -> 22.1, 1400^2 27.3 -> 24.7, 2500x600 23.6 -> 22.0. Past 1.6 times the longer
+ * items cost what the round saves (FP64 momentum 1536^2 with 14 rows for 9: the
+ * same). The Lagrangian, whose prologue is short, gained at 900^2 (5 rows for 4:
+ * 32 -> 30) and lost at 850^2 (5 for 3: 27.8 -> 29.5); it keeps the root.
+ */
 struct Rows {
-  double p;  /* prologue, in rows */
-  int most;  /* height on large meshes */
+  double p;      /* prologue, in rows */
+  int most;      /* height on large meshes */
+  double taller; /* how much taller a chunk may be to fit one round */
 };
 enum { kKLag = 0, kKMass = 1, kKMom = 2 };
 template <typename T>
 constexpr Rows rows_of(int kernel) {
-  return sizeof(T) == 8 ? (kernel == kKLag    ? Rows{2.9, 24}
-                           : kernel == kKMass ? Rows{5.7, 20}
-                                              : Rows{6.2, 16})
-                        : (kernel == kKLag    ? Rows{2.1, 24}
-                           : kernel == kKMass ? Rows{8.5, 16}
-                                              : Rows{5.2, 16});
+  return sizeof(T) == 8 ? (kernel == kKLag    ? Rows{2.9, 24, 1.0}
+                           : kernel == kKMass ? Rows{5.7, 20, 1.6}
+                                              : Rows{6.2, 16, 1.6})
+                        : (kernel == kKLag    ? Rows{2.1, 24, 1.0}
+                           : kernel == kKMass ? Rows{8.5, 16, 1.6}
+                                              : Rows{5.2, 16, 1.6});
 }
 
 /* the marches with two columns per lane (12 rows in FP64, measured 8 to 24; 10
  * in FP32, measured 4 to 24) run on large meshes, or where a caller asks */
 template <typename T>
 constexpr Rows pair_rows() {
-  return sizeof(T) == 8 ? Rows{2.9, 12} : Rows{2.1, 10};
+  return sizeof(T) == 8 ? Rows{2.9, 12, 1.0} : Rows{2.1, 10, 1.0};
 }
 
 inline MarchList march_items(int nx, int ny, int W, int chunk_rows, Rows r, int waves_per_simd,
@@ -50,9 +62,16 @@ inline MarchList march_items(int nx, int ny, int W, int chunk_rows, Rows r, int 
   if (chunk_rows > 0)
     return make_march(nx, ny, W, chunk_rows < kMaxChunkRows ? chunk_rows : kMaxChunkRows);
   const double cells = (double)(nx - 2 * kPad) * (ny - 2 * kPad);
-  const double slots = (double)march_cus() * kMWaves * waves_per_simd;
-  const int H = (int)(std::sqrt(r.p * cells / (W * slots)) + 0.5);
-  return make_march(nx, ny, W, H < least ? least : H > r.most ? r.most : H);
+  const int slots = march_cus() * kMWaves * waves_per_simd;
+  const double h = std::sqrt(r.p * cells / ((double)W * slots));
+  int H = (int)(h + 0.5);
+  H = H < least ? least : H > r.most ? r.most : H;
+  const int strips = make_march(nx, ny, W, H).nstrips;
+  if (strips >= 1 && strips <= slots) {
+    const int chunks = slots / strips, one_round = (ny - 2 * kPad + chunks - 1) / chunks;
+    if (one_round > H && one_round <= r.taller * h && one_round <= r.most) H = one_round;
+  }
+  return make_march(nx, ny, W, H);
 }
 
 template <typename T, bool P2, bool UNI, bool PAIR = false>
