@@ -66,11 +66,11 @@ void solve_hydro_2d(Mesh* mesh, int tt, double* P, double* rho,
                    Qxx, Qyy, F_x,     F_y, uF_x, uF_y, vF_x,  vF_y};
   const FlowHipStep st = flowhip_step_of(mesh, tt, a);
   flowhip_post_to(h, 0);
+  h->sums_valid = 0; /* until this step leaves totals of its own */
   flowhip_push_pair(h, mesh);
   flowhip_enqueue_step(h, &st);
   flowhip_wait(h);
   flowhip_take_pair(h, mesh, 0, kWho);
-  memcpy(h->totals, h->mail + 2, sizeof(h->totals));
 }
 
 /* omp3/flow.c:73-106 (reduce_all_min is the identity on one GPU) */
@@ -118,8 +118,9 @@ void print_conservation(const int nx, const int ny, double* rho, double* e,
     FK_LAUNCH(h, "conservation",
               fk_conservation(m, rho, e, h->red, h->stream));
     flowhip_wait(h);
-    memcpy(h->totals, h->mail + 2, sizeof(h->totals));
   }
+  /* posted by the launch above or, while sums_valid, by the last step */
+  memcpy(h->totals, h->mail + 2, sizeof(h->totals));
   h->sums_valid = 0; /* a step's totals are used at most once */
   if (mesh->rank == MASTER && mesh->verbose) {
     printf("Total mass:      %.12e\n", h->totals[0]);
@@ -127,7 +128,7 @@ void print_conservation(const int nx, const int ny, double* rho, double* e,
   }
 }
 
-/* Totals from the last print_conservation, for callers of flowhip_run. */
+/* Totals from the last print_conservation or step of flowhip_run. */
 void flowhip_last_sums(Mesh* mesh, double* mass, double* energy) {
   FlowHipCtx* h = flowhip_ctx(mesh);
   *mass = h->totals[0];

@@ -62,7 +62,8 @@ typedef struct FlowHipCtx {
   double* mail;         /* pinned: FK_MAIL_WORDS for each step in flight */
   double pair[2];       /* the device's dt pair, when pair_known */
   int pair_known;
-  double totals[2];     /* mass and energy of the last step or conservation call */
+  double totals[2];     /* mass and energy of the last print_conservation or
+                           flowhip_run step */
   int undefined;        /* of the last dt computation */
   int schedule;
   int march_rows;       /* chunk height of every march kernel; 0: each its own */
