@@ -85,15 +85,17 @@ typedef struct RunArgs32 {
   FkMesh32 m;
 } RunArgs32;
 
-static void enqueue_f32(void* arg, int tt) {
+static void enqueue_pre_f32(void* arg) {
   RunArgs32* r = (RunArgs32*)arg;
   FlowHipCtx* h = r->h;
-  if (tt < 0)
-    FK_LAUNCH(h, "timestep_f32",
-              fk_timestep_f32(r->m, r->a[8], r->a[9], r->a[1], r->a[3], h->red,
-                              r->mesh->max_dt, 0, h->stream));
-  else
-    step_f32(h, r->mesh, r->m, tt, r->a);
+  FK_LAUNCH(h, "timestep_f32",
+            fk_timestep_f32(r->m, r->a[8], r->a[9], r->a[1], r->a[3], h->red,
+                            r->mesh->max_dt, 0, h->stream));
+}
+
+static void enqueue_step_f32(void* arg, int tt) {
+  RunArgs32* r = (RunArgs32*)arg;
+  step_f32(r->h, r->mesh, r->m, tt, r->a);
 }
 
 /* main.c:64-115 on FP32 state; the arguments mean what flowhip_run's do. */
@@ -106,7 +108,7 @@ int flowhip_run_f32(Mesh* mesh, float** a, int niters, int tt0,
   RunArgs32 r = {flowhip_ctx(mesh), mesh, a, {0}};
   r.m = flowhip_fkmesh32(mesh);
   r.h->sums_valid = 0;
-  return flowhip_run_loop(r.h, mesh, enqueue_f32, &r, "hip kernel set (FP32 state)", niters,
-                          tt0, pre_timestep, dt_pairs, mass, energy, wall_seconds,
-                          undefined);
+  return flowhip_run_loop(r.h, mesh, enqueue_pre_f32, enqueue_step_f32, &r,
+                          "hip kernel set (FP32 state)", niters, tt0, pre_timestep, dt_pairs,
+                          mass, energy, wall_seconds, undefined);
 }

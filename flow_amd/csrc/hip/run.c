@@ -56,8 +56,8 @@ static int steps_ahead(const Mesh* mesh, double elapsed, int most) {
   return n;
 }
 
-int flowhip_run_loop(FlowHipCtx* h, Mesh* mesh, void (*enqueue)(void*, int), void* arg,
-                     const char* who, int niters, int tt0, int pre_timestep,
+int flowhip_run_loop(FlowHipCtx* h, Mesh* mesh, void (*pre)(void*), void (*step)(void*, int),
+                     void* arg, const char* who, int niters, int tt0, int pre_timestep,
                      double* dt_pairs, double* mass, double* energy, double* wall_seconds,
                      int* undefined) {
   /* replayed graphs post to the slot they were captured with; printed steps
@@ -68,7 +68,7 @@ int flowhip_run_loop(FlowHipCtx* h, Mesh* mesh, void (*enqueue)(void*, int), voi
   flowhip_push_pair(h, mesh);
   if (pre_timestep) {
     flowhip_post_to(h, 0);
-    enqueue(arg, -1);
+    pre(arg);
     flowhip_wait(h);
     flowhip_take_pair(h, mesh, 0, who);
   }
@@ -83,7 +83,7 @@ int flowhip_run_loop(FlowHipCtx* h, Mesh* mesh, void (*enqueue)(void*, int), voi
     const double w0 = now_seconds();
     for (int q = 0; q < n; ++q) {
       flowhip_post_to(h, q);
-      enqueue(arg, tt0 + k + q);
+      step(arg, tt0 + k + q);
     }
     flowhip_wait(h);
     wall += now_seconds() - w0;
@@ -121,14 +121,16 @@ typedef struct RunArgs {
   FlowHipStep st;
 } RunArgs;
 
-static void enqueue_f64(void* arg, int tt) {
+static void enqueue_pre_f64(void* arg) {
+  const RunArgs* r = (const RunArgs*)arg;
+  const FlowHipStep* st = &r->st;
+  flowhip_enqueue_timestep(r->h, st->m, st->Qxx, st->Qyy, st->rho, st->e, st->max_dt, 0);
+}
+
+static void enqueue_step_f64(void* arg, int tt) {
   RunArgs* r = (RunArgs*)arg;
   FlowHipCtx* h = r->h;
   FlowHipStep* st = &r->st;
-  if (tt < 0) {
-    flowhip_enqueue_timestep(h, st->m, st->Qxx, st->Qyy, st->rho, st->e, st->max_dt, 0);
-    return;
-  }
   st->tt = tt;
   h->sums_valid = 0;
   flowhip_enqueue_step(h, st);
@@ -147,8 +149,9 @@ int flowhip_run(Mesh* mesh, double** a, int niters, int tt0, int pre_timestep,
     r.h = flowhip_ctx(mesh);
     r.st = flowhip_step_of(mesh, tt0, a);
     if (niters > 0) flowhip_check_size(mesh);
-    return flowhip_run_loop(r.h, mesh, enqueue_f64, &r, "hip kernel set", niters, tt0,
-                            pre_timestep, dt_pairs, mass, energy, wall_seconds, undefined);
+    return flowhip_run_loop(r.h, mesh, enqueue_pre_f64, enqueue_step_f64, &r, "hip kernel set",
+                            niters, tt0, pre_timestep, dt_pairs, mass, energy, wall_seconds,
+                            undefined);
   }
   /* the calls main.c makes, with their prints */
   const int nx = mesh->local_nx, ny = mesh->local_ny;

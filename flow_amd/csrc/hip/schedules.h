@@ -24,11 +24,11 @@ void flowhip_enqueue_timestep(FlowHipCtx* h, FkMesh m, const double* Qxx, const 
                               const double* rho, const double* e, double max_dt,
                               int first_step);
 
-/* main.c:64-115's loop for flowhip_run and flowhip_run_f32: enqueue(arg, tt)
- * puts step tt and its totals on the stream, tt < 0 the pre-loop
- * set_timestep. The other arguments are flowhip_run's. */
-int flowhip_run_loop(FlowHipCtx* h, Mesh* mesh, void (*enqueue)(void*, int), void* arg,
-                     const char* who, int niters, int tt0, int pre_timestep,
+/* main.c:64-115's loop for flowhip_run and flowhip_run_f32: pre(arg) puts the
+ * pre-loop set_timestep on the stream, step(arg, tt) step tt (any number) and
+ * its totals. The other arguments are flowhip_run's. */
+int flowhip_run_loop(FlowHipCtx* h, Mesh* mesh, void (*pre)(void*), void (*step)(void*, int),
+                     void* arg, const char* who, int niters, int tt0, int pre_timestep,
                      double* dt_pairs, double* mass, double* energy, double* wall_seconds,
                      int* undefined);
 
