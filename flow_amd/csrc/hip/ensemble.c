@@ -460,10 +460,11 @@ static void ens_reserve_history(FlowHipEnsemble* E, int rows) {
 #define ENS_GRAPH_STEPS 4
 
 /* Steps from tt on, at most left of them: one, or a replay of the graph of tt's
- * sweep parity where a whole one fits (never the first step of a run, which
- * also has tt == 0's first_step dt). Returns how many. */
+ * sweep parity where a whole one fits. Never the first step of a run; and step
+ * 0, whose first_step dt no other step has, is in no graph. Returns how many. */
 static int ens_steps(FlowHipEnsemble* E, int tt, int left, int first) {
-  if (!E->use_graphs || first || tt == 0 || left < ENS_GRAPH_STEPS) {
+  const int has_step0 = tt <= 0 && tt > -ENS_GRAPH_STEPS;
+  if (!E->use_graphs || first || has_step0 || left < ENS_GRAPH_STEPS) {
     HIPCHECK(fk_ens_step(ens_launch(E), tt, E->fp32, E->stream));
     return 1;
   }

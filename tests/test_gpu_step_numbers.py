@@ -1,6 +1,6 @@
-"""flowhip_run and flowhip_run_f32 take any step number, as solve_hydro_2d
-does: tt counts (below zero too) only by its parity and by tt == 0's first-step
-update of dt_h (omp3/flow.c:103-105, 307, 565)."""
+"""flowhip_run, flowhip_run_f32 and the ensemble take any step number, as
+solve_hydro_2d does: tt counts (below zero too) only by its parity and by
+tt == 0's first-step update of dt_h (omp3/flow.c:103-105, 307, 565)."""
 import numpy as np
 import pytest
 
@@ -69,3 +69,26 @@ def test_run_through_step_zero():
         np.testing.assert_array_equal(fields[f], st.download(f), err_msg=f)
     st.close()
     m.close()
+
+
+@pytest.mark.parametrize("tt0", [-6, -5, -4, -3, -2, -1, 0])
+def test_ensemble_replays_around_step_zero(tt0):
+    """Replayed steps equal direct ones, where the first run passes step zero
+    and the second replays what the first captured."""
+    print(f"case ensemble tt0={tt0}", flush=True)
+    sizes = [33, 64]
+    out = []
+    for graphs in (False, True):
+        ens = flow_amd.Ensemble(sizes, dt=2.0e-4)
+        for k, n in enumerate(sizes):
+            ens.set_state(k, *problems.sod_x(n))
+        ens.set_graphs(graphs)
+        runs = [ens.run(12, tt0=tt0)[:3],
+                ens.run(13, tt0=tt0 + 12, pre_timestep=False)[:3]]
+        out.append((runs, [ens.get(k, f) for k in range(2) for f in FIELDS]))
+        ens.close()
+    for a, b in zip(out[0][0], out[1][0]):
+        for x, y in zip(a, b):
+            np.testing.assert_array_equal(x, y)
+    for x, y in zip(out[0][1], out[1][1]):
+        np.testing.assert_array_equal(x, y)
