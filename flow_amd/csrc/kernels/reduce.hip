@@ -25,15 +25,12 @@ __global__ __launch_bounds__(kRedThreads) void k_timestep(
     M m, const T* __restrict__ Qxx, const T* __restrict__ Qyy,
     const T* __restrict__ rho, const T* __restrict__ e, FkReduce r,
     double max_dt) {
-  /* (the interior of the largest mesh has fewer than 2^31 cells, so a cell
-   * index and the stride past it fit 32 bits: one 32-bit division a cell) */
-  const int pad = m.pad;
-  const unsigned int wx = m.nx - 2 * pad, n = wx * (unsigned int)(m.ny - 2 * pad);
+  const Interior in(m.nx, m.ny, m.pad);
   double local = max_dt;
   int bad = 0;
-  for (unsigned int k = blockIdx.x * blockDim.x + threadIdx.x; k < n;
+  for (unsigned int k = blockIdx.x * blockDim.x + threadIdx.x; k < in.n;
        k += gridDim.x * blockDim.x) {
-    const int i = pad + (int)(k / wx), j = pad + (int)(k % wx);
+    const int i = in.row(k), j = in.col(k);
     const int c = i * m.nx + j;
     const double ec = double(e[c]), qx = double(Qxx[c]), qy = double(Qyy[c]),
                  rc = double(rho[c]), dx = double(m.celldx[j]), dy = double(m.celldy[i]);
@@ -135,8 +132,8 @@ __global__ __launch_bounds__(kRedThreads) void k_timestep_serial(
   constexpr int kWaves = kRedThreads / kWave;
   __shared__ SerialFold s_fold[kWaves];
   __shared__ int s_bad[kWaves];
-  const int pad = m.pad, wx = m.nx - 2 * pad, wy = m.ny - 2 * pad;
-  const long n = (long)wx * wy;
+  const Interior in(m.nx, m.ny, m.pad);
+  const long n = in.n;
   const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
   const long b0 = n * blockIdx.x / gridDim.x, b1 = n * (blockIdx.x + 1) / gridDim.x;
   const long k0 = b0 + (b1 - b0) * w / kWaves, k1 = b0 + (b1 - b0) * (w + 1) / kWaves;
@@ -147,7 +144,7 @@ __global__ __launch_bounds__(kRedThreads) void k_timestep_serial(
     const bool valid = k < k1;
     double cand = 0.0;
     if (valid) {
-      const int i = pad + (int)(k / wx), j = pad + (int)(k % wx);
+      const int i = in.row((unsigned int)k), j = in.col((unsigned int)k);
       const int c = i * m.nx + j;
       cand = kFromArrays ? cell_timestep(e[c], Qxx[c], Qyy[c], rho[c], m.celldx[j],
                                          m.celldy[i])
@@ -213,12 +210,11 @@ __global__ __launch_bounds__(kRedThreads) void k_finish_serial(FkReduce r, int p
 template <typename M, typename T>
 __global__ __launch_bounds__(kRedThreads) void k_conservation(
     M m, const T* __restrict__ rho, const T* __restrict__ e, FkReduce r) {
-  const int pad = m.pad;
-  const unsigned int wx = m.nx - 2 * pad, n = wx * (unsigned int)(m.ny - 2 * pad);
+  const Interior in(m.nx, m.ny, m.pad);
   CSum ms{0.0, 0.0}, es{0.0, 0.0};
-  for (unsigned int k = blockIdx.x * blockDim.x + threadIdx.x; k < n;
+  for (unsigned int k = blockIdx.x * blockDim.x + threadIdx.x; k < in.n;
        k += gridDim.x * blockDim.x) {
-    const int i = pad + (int)(k / wx), j = pad + (int)(k % wx);
+    const int i = in.row(k), j = in.col(k);
     const int c = i * m.nx + j;
     ms.add(double(rho[c]));
     es.add(double(rho[c]) * double(e[c]));
@@ -226,7 +222,9 @@ __global__ __launch_bounds__(kRedThreads) void k_conservation(
   publish_sums<kRedThreads>(ms, es, r);
 }
 
-int red_blocks(long n) {
+template <typename M>
+int red_blocks(const M& m) {
+  const long n = Interior(m.nx, m.ny, m.pad).n;
   long b = (n + kRedThreads - 1) / kRedThreads;
   if (b > kRedBlocks) b = kRedBlocks;
   return b < 1 ? 1 : (int)b;
@@ -256,7 +254,7 @@ hipError_t fk_finish_sums(FkReduce r, int parts, hipStream_t s) {
 hipError_t fk_timestep(FkMesh m, const double* Qxx, const double* Qyy,
                        const double* rho, const double* e, FkReduce r,
                        double max_dt, int first_step, hipStream_t s) {
-  const int grid = red_blocks((long)(m.nx - 2 * m.pad) * (m.ny - 2 * m.pad));
+  const int grid = red_blocks(m);
   hipLaunchKernelGGL((k_timestep<FkMesh, double>), dim3(grid), dim3(kRedThreads), 0, s, m,
                      Qxx, Qyy, rho, e, r, max_dt);
   return fk_finish_timestep(r, grid, max_dt, first_step, s);
@@ -266,7 +264,7 @@ hipError_t fk_timestep_serial(FkMesh m, const double* cfl, const double* Qxx,
                               const double* Qyy, const double* rho,
                               const double* e, FkReduce r, double max_dt,
                               int first_step, hipStream_t s) {
-  const int grid = red_blocks((long)(m.nx - 2 * m.pad) * (m.ny - 2 * m.pad));
+  const int grid = red_blocks(m);
   if (cfl)
     hipLaunchKernelGGL(k_timestep_serial<false>, dim3(grid), dim3(kRedThreads), 0, s, m,
                        cfl, Qxx, Qyy, rho, e, r);
@@ -280,7 +278,7 @@ hipError_t fk_timestep_serial(FkMesh m, const double* cfl, const double* Qxx,
 
 hipError_t fk_conservation(FkMesh m, const double* rho, const double* e,
                            FkReduce r, hipStream_t s) {
-  const int grid = red_blocks((long)(m.nx - 2 * m.pad) * (m.ny - 2 * m.pad));
+  const int grid = red_blocks(m);
   hipLaunchKernelGGL((k_conservation<FkMesh, double>), dim3(grid), dim3(kRedThreads), 0, s,
                      m, rho, e, r);
   return fk_finish_sums(r, grid, s);
@@ -289,7 +287,7 @@ hipError_t fk_conservation(FkMesh m, const double* rho, const double* e,
 hipError_t fk_timestep_f32(FkMesh32 m, const float* Qxx, const float* Qyy,
                            const float* rho, const float* e, FkReduce r,
                            double max_dt, int first_step, hipStream_t s) {
-  const int grid = red_blocks((long)(m.nx - 2 * m.pad) * (m.ny - 2 * m.pad));
+  const int grid = red_blocks(m);
   hipLaunchKernelGGL((k_timestep<FkMesh32, float>), dim3(grid), dim3(kRedThreads), 0, s, m,
                      Qxx, Qyy, rho, e, r, max_dt);
   return fk_finish_timestep(r, grid, max_dt, first_step, s);
@@ -297,7 +295,7 @@ hipError_t fk_timestep_f32(FkMesh32 m, const float* Qxx, const float* Qyy,
 
 hipError_t fk_conservation_f32(FkMesh32 m, const float* rho, const float* e,
                                FkReduce r, hipStream_t s) {
-  const int grid = red_blocks((long)(m.nx - 2 * m.pad) * (m.ny - 2 * m.pad));
+  const int grid = red_blocks(m);
   hipLaunchKernelGGL((k_conservation<FkMesh32, float>), dim3(grid), dim3(kRedThreads), 0, s,
                      m, rho, e, r);
   return fk_finish_sums(r, grid, s);

@@ -22,6 +22,23 @@ constexpr int kTotalsOffset = 2 * kMaxReduceBlocks;
 constexpr int kTotalsWords = 8;
 constexpr int kPartialsDoubles = kTotalsOffset + kTotalsWords * kMaxReduceBlocks;
 
+/* The cells of a local nx x ny array inside its pad, numbered in row-major
+ * order; none where the pad leaves none (set_timestep and print_conservation
+ * take the sizes from their caller). Unsigned 32-bit numbers: the largest
+ * mesh's interior has fewer than 2^31 cells, so a number and a grid's stride
+ * past it fit, and a cell costs one 32-bit division. */
+struct Interior {
+  int pad;
+  unsigned int wx, n;
+  __host__ __device__ Interior(int nx, int ny, int pad_) : pad(pad_), wx(1), n(0) {
+    if (nx <= 2 * pad || ny <= 2 * pad) return;
+    wx = (unsigned int)(nx - 2 * pad);
+    n = wx * (unsigned int)(ny - 2 * pad);
+  }
+  __host__ __device__ int row(unsigned int k) const { return pad + (int)(k / wx); }
+  __host__ __device__ int col(unsigned int k) const { return pad + (int)(k % wx); }
+};
+
 /* (of a block of at most NT threads) */
 template <int NT>
 __device__ __forceinline__ double block_min(double x, int waves = NT / kWave) {

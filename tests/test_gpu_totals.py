@@ -98,3 +98,24 @@ def test_last_totals_stay_until_the_next_ones():
     st.solve(5)
     assert _last_sums(m) == (mass[-1], energy[-1])
     _close(m, st)
+
+
+@pytest.mark.parametrize("rule", [flow_amd.CFL_DEFINED, flow_amd.CFL_OMP3_SERIAL])
+@pytest.mark.parametrize("nx,ny", [(3, 40), (40, 3), (4, 40), (2, 2)])
+def test_no_interior(nx, ny, rule):
+    """Sizes without interior cells: totals of nothing, and the dt pair that
+    max_dt and dt_h give (C_T 0.3, C_M 5: omp3/flow.c:103-105)."""
+    print(f"case no interior {nx}x{ny} rule={rule}", flush=True)
+    m, st = _state()
+    m.set_cfl_rule(rule)
+    m.s.max_dt = 1.0e-3
+    m.set_dt(3.0e-4, 4.0e-4)
+    arg = {k: ctypes.c_void_p(st.ptrs[k]) for k in ("Qxx", "Qyy", "rho", "e")}
+    native.lib().set_timestep(nx, ny, arg["Qxx"], arg["Qyy"], arg["rho"], arg["e"], m.ptr, None,
+                              0, ctypes.cast(m.s.celldx, ctypes.c_void_p),
+                              ctypes.cast(m.s.celldy, ctypes.c_void_p))
+    least = min(1.0e-3, (1.5 / 0.3) * 4.0e-4)
+    assert (m.dt, m.dt_h) == (0.5 * (0.3 * least + 4.0e-4), 0.3 * least)
+    native.lib().print_conservation(nx, ny, arg["rho"], arg["e"], None, m.ptr)
+    assert _last_sums(m) == (0.0, 0.0)
+    _close(m, st)
