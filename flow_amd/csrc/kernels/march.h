@@ -125,7 +125,7 @@ struct MarchList {
  * is exact while item * n < 2^40 (a mesh of 46335 columns has 800 strips and
  * fewer than 2^25 items). */
 inline __host__ __device__ unsigned long long strip_inverse(int nstrips) {
-  return (1ull << 40) / (unsigned int)nstrips + 1ull;
+  return nstrips < 1 ? 0ull : (1ull << 40) / (unsigned int)nstrips + 1ull;
 }
 
 /* Columns and rows of one item. */
@@ -275,11 +275,10 @@ struct MarchBlockQueue : MarchQueue<true> {
   }
 };
 
-/* Items of a mesh. */
+/* Items of a mesh; none where it has no interior cells. */
 inline MarchList make_march(int nx, int ny, int W, int H) {
-  MarchList m;
-  m.W = W;
-  m.H = H;
+  MarchList m{W, H, 0, 0, 0, 0};
+  if (nx <= 2 * kPad || ny <= 2 * kPad) return m;
   m.nstrips = (nx - 2 * kPad + W - 1) / W;
   m.nchunks = (ny - 2 * kPad + H - 1) / H;
   m.nitems = m.nstrips * m.nchunks;

@@ -61,6 +61,7 @@ inline MarchList march_items(int nx, int ny, int W, int chunk_rows, Rows r, int 
                              int least = kMinChunkRows) {
   if (chunk_rows > 0)
     return make_march(nx, ny, W, chunk_rows < kMaxChunkRows ? chunk_rows : kMaxChunkRows);
+  if (make_march(nx, ny, W, least).nitems < 1) return make_march(nx, ny, W, least);
   const double cells = (double)(nx - 2 * kPad) * (ny - 2 * kPad);
   const int slots = march_cus() * kMWaves * waves_per_simd;
   const double h = std::sqrt(r.p * cells / ((double)W * slots));
