@@ -122,8 +122,10 @@ struct MarchList {
 
 /* item / nstrips as (item * inv) >> 40, two scalar multiplies for a division
  * of some thirty vector operations: with inv = floor(2^40 / n) + 1 the quotient
- * is exact while item * n < 2^40 (a mesh of 46335 columns has 800 strips and
- * fewer than 2^25 items). */
+ * is exact while item * n < 2^40, and item * inv fits 64 bits while the
+ * quotient, a chunk, is below 2^24. A mesh of 46335 cells a side has 800 strips,
+ * fewer than 2^15 chunks and fewer than 2^25 items; make_march makes no items of
+ * a list past either bound. */
 inline __host__ __device__ unsigned long long strip_inverse(int nstrips) {
   return nstrips < 1 ? 0ull : (1ull << 40) / (unsigned int)nstrips + 1ull;
 }
@@ -275,13 +277,16 @@ struct MarchBlockQueue : MarchQueue<true> {
   }
 };
 
-/* Items of a mesh; none where it has no interior cells. */
+/* Items of a mesh; none where it has no interior cells, or past what the strip
+ * quotient holds for. */
 inline MarchList make_march(int nx, int ny, int W, int H) {
   MarchList m{W, H, 0, 0, 0, 0};
   if (nx <= 2 * kPad || ny <= 2 * kPad) return m;
   m.nstrips = (nx - 2 * kPad + W - 1) / W;
   m.nchunks = (ny - 2 * kPad + H - 1) / H;
-  m.nitems = m.nstrips * m.nchunks;
+  const long n = (long)m.nstrips * m.nchunks;
+  if (m.nchunks >= (1 << 24) || n >= (1l << 31) || n * m.nstrips >= (1l << 40)) return m;
+  m.nitems = (int)n;
   m.inv = strip_inverse(m.nstrips);
   return m;
 }
