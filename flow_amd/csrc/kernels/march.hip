@@ -151,14 +151,20 @@ inline bool lag_pairs_fit(const MGeo<T>& g, const MLagIO<T>& io) {
 constexpr int kMomXW = kWave - 5;
 constexpr int kMomW = kWave - 4;
 
+/* The end of a step whose momentum directions march apart. */
+static __global__ __launch_bounds__(kMNT) void k_march_settle(FkReduce red, int parts) {
+  step_epilogue(red, parts);
+}
+
 template <typename T, bool P2>
-hipError_t launch_march_momentum_p(MGeo<T> g, MMomIO<T> io, int tt, int ydir,
-                                   const double* dtp, int chunk_rows, hipStream_t s) {
+hipError_t launch_march_momentum_p(MGeo<T> g, MMomIO<T> io, int tt, int ydir, FkReduce r,
+                                   int parts, int chunk_rows, hipStream_t s) {
   const bool odd = (tt % 2) != 0;
   const MarchList ml =
       march_items(g.nx, g.ny, (!ydir && !odd) ? kMomXW : kMomW, chunk_rows,
                   rows_of<T>(kKMom), kMarchMaxWaves<T>, 4);
-  if (ml.nitems < 1) return hipErrorInvalidValue;
+  if (ml.nitems < 1 || !r.queue) return hipErrorInvalidValue;
+  const double* dtp = r.dtp + 2; /* the pair the mass/energy march left */
   if (!ydir && odd) {
     static int per_cu = 0;
     const int grid = march_grid(k_march_momx_xy<T, P2>, per_cu, ml.nitems);
@@ -176,6 +182,7 @@ hipError_t launch_march_momentum_p(MGeo<T> g, MMomIO<T> io, int tt, int ydir,
     const int grid = march_grid(k_march_momy_yx<T, P2>, per_cu, ml.nitems);
     hipLaunchKernelGGL((k_march_momy_yx<T, P2>), dim3(grid), dim3(kMNT), 0, s, g, io, dtp, ml);
   }
+  if (ydir) hipLaunchKernelGGL(k_march_settle, dim3(1), dim3(kMNT), 0, s, r, parts);
   return hipGetLastError();
 }
 
@@ -328,11 +335,10 @@ hipError_t launch_march_lagrangian(MGeo<T> g, MLagIO<T> io, FkReduce r, double m
 }
 
 template <typename T>
-hipError_t launch_march_momentum(MGeo<T> g, MMomIO<T> io, int tt, int ydir,
-                                 const double* dtp, int chunk_rows, int pow2,
-                                 hipStream_t s) {
-  return pow2 ? launch_march_momentum_p<T, true>(g, io, tt, ydir, dtp, chunk_rows, s)
-              : launch_march_momentum_p<T, false>(g, io, tt, ydir, dtp, chunk_rows, s);
+hipError_t launch_march_momentum(MGeo<T> g, MMomIO<T> io, int tt, int ydir, FkReduce r,
+                                 int parts, int chunk_rows, int pow2, hipStream_t s) {
+  return pow2 ? launch_march_momentum_p<T, true>(g, io, tt, ydir, r, parts, chunk_rows, s)
+              : launch_march_momentum_p<T, false>(g, io, tt, ydir, r, parts, chunk_rows, s);
 }
 
 template <typename T>
@@ -387,18 +393,18 @@ hipError_t fk_march_momentum_x(FkMesh m, int tt, const double* u0,
                                const double* v0, const double* F_x,
                                const double* F_y, const double* rho,
                                const double* mx1, double* mom_x, double* u,
-                               const double* dtp, int chunk_rows, hipStream_t s) {
+                               FkReduce r, int chunk_rows, hipStream_t s) {
   MMomIO<double> io{u0, v0, F_x, F_y, rho, mx1, mom_x, u};
-  return launch_march_momentum<double>(mgeo64(m), io, tt, 0, dtp, chunk_rows, m.pow2, s);
+  return launch_march_momentum<double>(mgeo64(m), io, tt, 0, r, 0, chunk_rows, m.pow2, s);
 }
 
 hipError_t fk_march_momentum_y(FkMesh m, int tt, const double* u1,
                                const double* v0, const double* F_x,
                                const double* F_y, const double* rho,
                                const double* my1, double* mom_y, double* v,
-                               const double* dtp, int chunk_rows, hipStream_t s) {
+                               FkReduce r, int parts, int chunk_rows, hipStream_t s) {
   MMomIO<double> io{u1, v0, F_x, F_y, rho, my1, mom_y, v};
-  return launch_march_momentum<double>(mgeo64(m), io, tt, 1, dtp, chunk_rows, m.pow2, s);
+  return launch_march_momentum<double>(mgeo64(m), io, tt, 1, r, parts, chunk_rows, m.pow2, s);
 }
 
 hipError_t fk_march_mass_energy(FkMesh m, int tt, const double* u0,
@@ -456,20 +462,18 @@ hipError_t fk_march_momentum_x_f32(FkMesh32 m, int tt, const float* u0,
                                    const float* v0, const float* F_x,
                                    const float* F_y, const float* rho,
                                    const float* mx1, float* mom_x, float* u,
-                                   const double* dtp, int chunk_rows,
-                                   hipStream_t s) {
+                                   FkReduce r, int chunk_rows, hipStream_t s) {
   MMomIO<float> io{u0, v0, F_x, F_y, rho, mx1, mom_x, u};
-  return launch_march_momentum<float>(mgeo32(m), io, tt, 0, dtp, chunk_rows, m.pow2, s);
+  return launch_march_momentum<float>(mgeo32(m), io, tt, 0, r, 0, chunk_rows, m.pow2, s);
 }
 
 hipError_t fk_march_momentum_y_f32(FkMesh32 m, int tt, const float* u1,
                                    const float* v0, const float* F_x,
                                    const float* F_y, const float* rho,
                                    const float* my1, float* mom_y, float* v,
-                                   const double* dtp, int chunk_rows,
-                                   hipStream_t s) {
+                                   FkReduce r, int parts, int chunk_rows, hipStream_t s) {
   MMomIO<float> io{u1, v0, F_x, F_y, rho, my1, mom_y, v};
-  return launch_march_momentum<float>(mgeo32(m), io, tt, 1, dtp, chunk_rows, m.pow2, s);
+  return launch_march_momentum<float>(mgeo32(m), io, tt, 1, r, parts, chunk_rows, m.pow2, s);
 }
 
 }  // extern "C"

@@ -244,8 +244,8 @@ hipError_t fk_advect_momentum_y(FkMesh m, int tt, const double* u1,
  *   fk_march_mass_energy folds the lag_parts blocks' minima into the new
  *     pair (lag_parts 0: r.dtp holds it already) and leaves its blocks'
  *     totals (*parts blocks);
- *   fk_march_momentum folds the parts blocks' totals into r.sums and leaves
- *     the new pair in r.dtp. */
+ *   fk_march_momentum (or fk_march_momentum_x, then _y) folds the parts
+ *     blocks' totals into r.sums and leaves the new pair in r.dtp. */
 hipError_t fk_march_mass_energy(FkMesh m, int tt, const double* u0,
                                 const double* v0, const double* rho0,
                                 const double* e1, double* rho, double* e,
@@ -259,22 +259,25 @@ hipError_t fk_march_lagrangian(FkMesh m, const double* rho, const double* e,
                                int chunk_rows, hipStream_t s);
 /* omp3/flow.c:557-775: both momentum directions in one row march (the y
  * direction reads the u the x direction has just computed in the same
- * wave); the result equals fk_march_momentum_x then _y. */
+ * wave). */
 hipError_t fk_march_momentum(FkMesh m, int tt, const double* u0, const double* v0,
                              const double* F_x, const double* F_y, const double* rho,
                              const double* mx1, const double* my1, double* mom_x,
                              double* mom_y, double* u, double* v, FkReduce r,
                              int parts, int chunk_rows, hipStream_t s);
+/* The same in two marches, x then y, in place of fk_march_momentum: the same
+ * bits. u1 is the u that the x direction wrote; the y direction settles the pair
+ * and the totals. */
 hipError_t fk_march_momentum_x(FkMesh m, int tt, const double* u0,
                                const double* v0, const double* F_x,
                                const double* F_y, const double* rho,
                                const double* mx1, double* mom_x, double* u,
-                               const double* dtp, int chunk_rows, hipStream_t s);
+                               FkReduce r, int chunk_rows, hipStream_t s);
 hipError_t fk_march_momentum_y(FkMesh m, int tt, const double* u1,
                                const double* v0, const double* F_x,
                                const double* F_y, const double* rho,
                                const double* my1, double* mom_y, double* v,
-                               const double* dtp, int chunk_rows, hipStream_t s);
+                               FkReduce r, int parts, int chunk_rows, hipStream_t s);
 
 /* ---- FP32-state precision form (march kernels over float arrays) ----
  * Same contracts as the FP64 launchers. The CFL candidates, the dt
@@ -306,13 +309,12 @@ hipError_t fk_march_momentum_x_f32(FkMesh32 m, int tt, const float* u0,
                                    const float* v0, const float* F_x,
                                    const float* F_y, const float* rho,
                                    const float* mx1, float* mom_x, float* u,
-                                   const double* dtp, int chunk_rows,
-                                   hipStream_t s);
+                                   FkReduce r, int chunk_rows, hipStream_t s);
 hipError_t fk_march_momentum_y_f32(FkMesh32 m, int tt, const float* u1,
                                    const float* v0, const float* F_x,
                                    const float* F_y, const float* rho,
                                    const float* my1, float* mom_y, float* v,
-                                   const double* dtp, int chunk_rows,
+                                   FkReduce r, int parts, int chunk_rows,
                                    hipStream_t s);
 /* ---- ensemble (batching) form ----
  * One descriptor per instance; arrays and geometry are FP64 or FP32 (one

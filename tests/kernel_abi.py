@@ -32,7 +32,9 @@ def lib():
                 ("fk_march_mass_energy",
                  [FkMesh, _i] + [_vp] * 8 + [FkReduce, _d, _i, _i, _vp, _i, _vp]),
                 ("fk_march_momentum",
-                 [FkMesh, _i] + [_vp] * 11 + [FkReduce, _i, _i, _vp])):
+                 [FkMesh, _i] + [_vp] * 11 + [FkReduce, _i, _i, _vp]),
+                ("fk_march_momentum_x", [FkMesh, _i] + [_vp] * 8 + [FkReduce, _i, _vp]),
+                ("fk_march_momentum_y", [FkMesh, _i] + [_vp] * 8 + [FkReduce, _i, _i, _vp])):
             fn = getattr(L, name + suffix)
             fn.restype, fn.argtypes = _i, args
     return L
@@ -45,7 +47,7 @@ def mesh(fp32, nx, ny, pairs=0):
 
 
 def march_calls(L, m, fp32, tt, rows):
-    """The results of the three march launchers of a step with no arrays."""
+    """The results of the march launchers of a step with no arrays."""
     suffix = "_f32" if fp32 else ""
     r = FkReduce(queue=256)
     parts = ctypes.c_int()
@@ -53,5 +55,7 @@ def march_calls(L, m, fp32, tt, rows):
                                                       ctypes.byref(parts), rows, None),
            getattr(L, "fk_march_mass_energy" + suffix)(m, tt, *[None] * 8, r, 1.0, 0, 1,
                                                        ctypes.byref(parts), rows, None),
-           getattr(L, "fk_march_momentum" + suffix)(m, tt, *[None] * 11, r, 1, rows, None)]
+           getattr(L, "fk_march_momentum" + suffix)(m, tt, *[None] * 11, r, 1, rows, None),
+           getattr(L, "fk_march_momentum_x" + suffix)(m, tt, *[None] * 8, r, rows, None),
+           getattr(L, "fk_march_momentum_y" + suffix)(m, tt, *[None] * 8, r, 1, rows, None)]
     return out
