@@ -3,6 +3,8 @@
  * omp3's loop order (omp3/flow.c:10-52), with an on-device boundary kernel
  * at each of omp3's 19 handle_boundary_2d sites.
  */
+#include <string.h>
+
 #include "schedules.h"
 
 #define BND(h, nxp, nyp, arr, inv)                                        \
@@ -152,7 +154,10 @@ static int same_step(const FlowHipStep* a, const FlowHipStep* b) {
          a->m.edgedx == b->m.edgedx && a->m.edgedy == b->m.edgedy &&
          a->m.celldx == b->m.celldx && a->m.celldy == b->m.celldy &&
          a->m.inv_edgedx == b->m.inv_edgedx && a->m.inv_edgedy == b->m.inv_edgedy &&
-         a->m.pow2 == b->m.pow2 && a->m.uniform == b->m.uniform;
+         a->m.pow2 == b->m.pow2 && a->m.uniform == b->m.uniform &&
+         a->m.pairs == b->m.pairs &&
+         /* a captured launch holds a uniform mesh's spacings themselves */
+         memcmp(&a->m.u, &b->m.u, sizeof(a->m.u)) == 0;
 }
 
 void flowhip_enqueue_step(FlowHipCtx* h, const FlowHipStep* st) {
