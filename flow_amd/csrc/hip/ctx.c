@@ -239,6 +239,12 @@ static void ensure_reciprocals(FlowHipCtx* h, const Mesh* mesh) {
   h->inv_src_y = mesh->edgedy;
   h->inv_nx = lx;
   h->inv_ny = ly;
+  h->geo32_src[0] = NULL; /* the FP32 copies are of the arrays as they were */
+}
+
+int flowhip_geometry_changed(Mesh* mesh) {
+  flowhip_ctx(mesh)->inv_src_x = NULL;
+  return 0;
 }
 
 FkMesh flowhip_fkmesh(const Mesh* mesh) {

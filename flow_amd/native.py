@@ -63,6 +63,7 @@ def lib():
         "flowhip_set_schedule": (i, [mp, i]),
         "flowhip_get_schedule": (i, [mp]),
         "flowhip_set_graphs": (i, [mp, i]),
+        "flowhip_geometry_changed": (i, [mp]),
         "flowhip_set_march_rows": (i, [mp, i]),
         "flowhip_set_timing": (i, [mp, i]),
         "flowhip_timing_count": (i, [mp]),
@@ -170,6 +171,10 @@ class Mesh:
 
     def set_graphs(self, on):
         lib().flowhip_set_graphs(self.ptr, 1 if on else 0)
+
+    def geometry_changed(self):
+        """The spacing arrays hold other values than at the last call."""
+        lib().flowhip_geometry_changed(self.ptr)
 
     def set_cfl_rule(self, rule):
         """CFL_DEFINED or CFL_OMP3_SERIAL (flow_hip.h)."""

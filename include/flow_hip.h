@@ -46,6 +46,12 @@ int flowhip_set_march_rows(Mesh* mesh, int rows);
  * arrays, geometry, schedule or chunk height change. Per-kernel timing
  * (flowhip_set_timing) launches directly. */
 int flowhip_set_graphs(Mesh* mesh, int on);
+/* The spacing arrays (edgedx, edgedy, celldx, celldy) are looked at when the
+ * mesh's first call finds them, or others in their place: the march schedule
+ * passes a uniform mesh's spacings by value from then on, and their reciprocals
+ * are kept. A caller that writes other spacings into the same arrays says so
+ * with this call; the next one looks at them again. */
+int flowhip_geometry_changed(Mesh* mesh);
 
 /* Rules for set_timestep's undefined CFL candidates (cells with negative
  * energy or zero density, whose candidate omp3/flow.c:87-94 makes NaN).
