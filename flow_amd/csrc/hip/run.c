@@ -65,7 +65,8 @@ int flowhip_run_loop(FlowHipCtx* h, Mesh* mesh, void (*pre)(void*), void (*step)
   const int alone = h->use_graphs || (mesh->rank == MASTER && mesh->verbose);
   double wall = 0.0, elapsed = 0.0;
   int k = 0;
-  flowhip_push_pair(h, mesh);
+  /* with nothing to run the pair stays where it is: no wait would follow */
+  if (pre_timestep || niters > 0) flowhip_push_pair(h, mesh);
   if (pre_timestep) {
     flowhip_post_to(h, 0);
     pre(arg);
