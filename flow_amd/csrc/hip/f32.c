@@ -55,7 +55,7 @@ int flowhip_f32_boundary(Mesh* mesh, float* arr, int nxp, int nyp, int invert) {
   return 0;
 }
 
-/* One step of omp3/flow.c:10-52 on FP32 state, in the march schedule's four
+/* One step of omp3/flow.c:10-52 on FP32 state, in the march schedule's three
  * kernels (the same ping-pong use of P, Qxx, Qyy, uF_x, uF_y as the FP64
  * fused schedule). */
 static void step_f32(FlowHipCtx* h, Mesh* mesh, FkMesh32 m, int tt, float** a) {

@@ -100,10 +100,6 @@ hipError_t launch_march_mass_p(MGeo<T> g, MMassIO<T> io, int tt, FkReduce r, Mar
   return hipGetLastError();
 }
 
-/* Whether an FP32 mass/energy march can hold two columns per lane: rows of
- * the cell and y-face arrays it reads or writes as column pairs start on
- * 8-byte boundaries (nx even, arrays 8-byte aligned; strips start at even
- * columns). */
 /* Whether the two-column form runs: FkMesh.pairs 2 always, 1 on meshes of
  * at least FK_PAIR_MIN_CELLS interior cells. */
 inline bool pairs_wanted(int pairs, int nx, int ny) {
@@ -111,6 +107,9 @@ inline bool pairs_wanted(int pairs, int nx, int ny) {
          (pairs == 1 && (long)(nx - 2 * kPad) * (ny - 2 * kPad) >= FK_PAIR_MIN_CELLS);
 }
 
+/* Whether a mass/energy march can hold two columns per lane: rows of the cell
+ * and y-face arrays it reads or writes as column pairs start on boundaries of
+ * two values (nx even, arrays so aligned; strips start at even columns). */
 template <typename T>
 inline bool pairs_fit(const MGeo<T>& g, const MMassIO<T>& io) {
   const unsigned long long bits =

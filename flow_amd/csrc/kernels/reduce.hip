@@ -3,9 +3,10 @@
  * minimum (omp3/flow.c:77-105) and the conservation totals
  * (omp3/flow.c:973-995).
  *
- * Each block reduces its share through wave64 shuffles and LDS and writes
- * one partial; a one-block launch folds the partials (reduce_common.h says
- * why that beats folding in the last block to finish).
+ * Each block reduces its share across its waves (the minimum by DPP moves, the
+ * compensated sums by shuffles) and through LDS, and writes one partial; a
+ * one-block launch folds the partials (reduce_common.h says why that beats
+ * folding in the last block to finish).
  */
 #include "reduce_common.h"
 
@@ -15,8 +16,8 @@ namespace {
 constexpr int kRedThreads = 256;
 constexpr int kRedBlocks = 1024;
 
-/* CFL minimum over the interior, then the dt pair update in the last block.
- * min is exact, so the visiting order does not change the result. NaN
+/* Each block's CFL minimum over its share of the interior (k_finish_timestep
+ * folds them). min is exact, so the visiting order does not change the result. NaN
  * candidates (cells with negative energy: sqrt of a negative) are left out,
  * as the reference's min(a, b) = a < b ? a : b leaves them out in effect,
  * and counted. */
